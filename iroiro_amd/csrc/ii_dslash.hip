@@ -97,19 +97,17 @@ __device__ __forceinline__ void hop_epilogue(C o[12], const C* xs, int hs, const
   outr.st(hs, o);
 }
 
-// BS threads per block (kBlock for the variants with partial sums, which are
-// indexed by kBlock-site ranges; the autotuner picks it for the others).
+// One thread per site; the single-rhs hop of the 16-bit fields.
 template <bool G5IN, bool G5OUT, bool XPAY, int EPI, typename SpIn, typename Gauge,
-          typename StOut, typename SpX, int BS = kBlock>
-__global__ void __launch_bounds__(BS)
+          typename StOut, typename SpX>
+__global__ void __launch_bounds__(kBlock)
 k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
       typename SpIn::R a, bool tbc_flip, double* __restrict__ partials,
       const int* __restrict__ skip, int skip_stride, HopOrder order,
       const double* __restrict__ coef, int coef_stride) {
-  static_assert(EPI == kEpiStore || BS == kBlock, "partial sums are per kBlock sites");
   using C = typename SpIn::C;
   const int nblk = gridDim.x;
-  const int base = hop_block_base(g, order, blockIdx.x, nblk, BS);
+  const int base = hop_block_base(g, order, blockIdx.x, nblk, kBlock);
   const int hs = base + threadIdx.x;
   const int rhs = blockIdx.y;
   if (skip && skip[rhs * skip_stride]) return;  // uniform per block
@@ -148,6 +146,121 @@ k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
     double s = block_sum(dsum[j]);
     // indexed by the site range, so sums do not depend on the traversal
     if (threadIdx.x == 0) partials[j * plane + (size_t)rhs * nblk + base / kBlock] = s;
+  }
+}
+
+// hop_epilogue for the three colours of one output spin (the accumulation
+// type is the field's; the sums over sites are FP64).
+template <int EPI, typename R, typename C, typename SpX>
+__device__ __forceinline__ void hop_epilogue_spin(C o[3], const C xs[3], int hs, int spin,
+                                                  const SpX& dr, double alpha, double ds[3]) {
+  if constexpr (EPI == kEpiStore) return;
+  R u = R(0), v = R(0), w = R(0);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    C d = o[c];
+    if constexpr (EPI == kEpiDot || EPI == kEpiRUpd || EPI == kEpiCDot) d = dr.ld(hs, 3 * spin + c);
+    if constexpr (EPI == kEpiDot) u = fma(d.x, o[c].x, fma(d.y, o[c].y, u));
+    if constexpr (EPI == kEpiRUpd) {
+      o[c].x = fma(-(R)alpha, o[c].x, d.x);
+      o[c].y = fma(-(R)alpha, o[c].y, d.y);
+    }
+    if constexpr (EPI == kEpiNorm || EPI == kEpiRUpd)
+      u = fma(o[c].x, o[c].x, fma(o[c].y, o[c].y, u));
+    if constexpr (EPI == kEpiCDot) {
+      u = fma(d.x, o[c].x, fma(d.y, o[c].y, u));
+      v = fma(d.x, o[c].y, fma(-d.y, o[c].x, v));
+    }
+    if constexpr (EPI == kEpiTS) {
+      u = fma(o[c].x, xs[c].x, fma(o[c].y, xs[c].y, u));
+      v = fma(o[c].x, xs[c].y, fma(-o[c].y, xs[c].x, v));
+      w = fma(o[c].x, o[c].x, fma(o[c].y, o[c].y, w));
+    }
+  }
+  ds[0] = (double)u;
+  ds[1] = (double)v;
+  ds[2] = (double)w;
+}
+
+// Single-rhs hop of the FP64 and FP32 fields, bound by latency on lattices
+// whose fields stay in the Infinity Cache and by HBM beyond.  The four
+// dimensions of a site are split over the four waves of a block: a block is
+// 64 sites, wave mu adds the two directions of dimension mu and leaves the
+// sum in LDS; wave s then adds spin s over the dimensions and runs that
+// spin's share of the epilogue.  Against one thread per site over all eight
+// directions (256 registers in FP64, one wave per SIMD) a site has four
+// times the waves, each with a quarter of the load chain: FP64 6.4 -> 3.9 us
+// at 8^3x16, 10.0 -> 5.0 us at 12x10x14x18, 18.6 -> 16.8 us at 16^3x32,
+// 274.6 -> 262.3 us at 32^3x64 (6.14 TB/s of algorithmic bytes); FP32 9.8 ->
+// 4.0, 11.6 -> 8.5 and 123.8 -> 123.0 us on the last three (with links_cached).
+// 48 KB of LDS (FP64) and 140 registers leave three blocks per CU; launch
+// bounds of 1, 2 and 3 waves per SIMD compile alike.
+template <bool G5IN, bool G5OUT, bool XPAY, int EPI, typename SpIn, typename Gauge,
+          typename StOut, typename SpX>
+__global__ void __launch_bounds__(256)
+k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
+            typename SpIn::R a, bool tbc_flip, double* __restrict__ partials,
+            const int* __restrict__ skip, HopOrder order, const double* __restrict__ coef) {
+  using C = typename SpIn::C;
+  using R = typename SpIn::R;
+  __shared__ C part[4][12][64];  // [dimension][3 spin + colour][site]
+  if (skip && skip[0]) return;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int base = hop_block_base(g, order, blockIdx.x, gridDim.x, 64);
+  const int hs = base + lane;
+  const bool valid = hs < g.Vh;
+  const SiteCoord sc = decode_site(g, valid ? hs : 0, out_par);
+  auto dimension = [&](auto W) {
+    constexpr int MU = decltype(W)::value;
+    C acc[4][3];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) acc[s][c] = cmk<C>(R(0), R(0));
+    if (valid) {
+      const int nf = neighbour(g, sc, hs, MU, true), nb = neighbour(g, sc, hs, MU, false);
+      hop_dir<MU, true, G5IN>(acc, in, gauge, nf, out_par, hs,
+                              MU == 3 && tbc_flip && sc.t == g.L[3] - 1);
+      hop_dir<MU, false, G5IN>(acc, in, gauge, nb, 1 - out_par, nb,
+                               MU == 3 && tbc_flip && sc.t == 0);
+    }
+#pragma unroll
+    for (int k = 0; k < 12; ++k) part[MU][k][lane] = acc[k / 3][k % 3];
+  };
+  if (w == 0) dimension(std::integral_constant<int, 0>());
+  else if (w == 1) dimension(std::integral_constant<int, 1>());
+  else if (w == 2) dimension(std::integral_constant<int, 2>());
+  else dimension(std::integral_constant<int, 3>());
+  __syncthreads();
+  double dsum[3] = {0.0, 0.0, 0.0};
+  if (valid) {
+    C o[3], xsv[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      C sum = cmk<C>(R(0), R(0));
+#pragma unroll
+      for (int m = 0; m < 4; ++m)  // x, y, z, t: the same order in every wave
+        sum = cadd(sum, part[m][3 * w + c][lane]);
+      o[c] = cscale(sum, a);
+    }
+    const int so = G5OUT ? (w ^ 2) : w;  // output spin of this wave
+    if (XPAY) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        xsv[c] = x.ld(hs, 3 * so + c);
+        o[c] = cadd(o[c], xsv[c]);
+      }
+    }
+    hop_epilogue_spin<EPI, R>(o, xsv, hs, so, dv, EPI == kEpiRUpd ? coef[0] : 0.0, dsum);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) out.st1(hs, 3 * so + c, o[c]);
+  }
+  constexpr int NS = epi_sums(EPI);
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    double s = block_sum(dsum[j]);
+    if (threadIdx.x == 0) partials[(size_t)j * gridDim.x + base / 64] = s;
   }
 }
 
@@ -323,7 +436,7 @@ namespace {
 template <typename Gauge> struct MrhsShape { static constexpr int TS = 64, MAXT = 768; };
 template <> struct MrhsShape<GaugeF64> { static constexpr int TS = 64, MAXT = 768; };
 // storage precision (II_PREC_*) of a gauge accessor
-template <typename Gauge> struct GaugePrec;
+template <typename Gauge> struct GaugePrec { static constexpr int value = -1; };  // single rhs only
 template <> struct GaugePrec<GaugeF64> { static constexpr int value = II_PREC_DOUBLE; };
 template <> struct GaugePrec<GaugeF32r12> { static constexpr int value = II_PREC_SINGLE; };
 template <> struct GaugePrec<GaugeLoR12<__half2>> { static constexpr int value = II_PREC_HALF; };
@@ -338,27 +451,19 @@ ii_status launch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, const 
   const Geom& g = ctx->g;
   bool flip = ctx->tbc_sign < 0;
   if (h.nrhs == 1) {
-    const HopOrder& o = ctx->hop_order;
-    if constexpr (EPI == kEpiStore && (std::is_same<Gauge, GaugeF64>::value ||
-                                       std::is_same<Gauge, GaugeF64Flat>::value)) {
-      if (o.bs == 128) {
-        dim3 grid(blocks_for(g.Vh, 128), 1);
-        hipLaunchKernelGGL((k_hop<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX, 128>), grid,
-                           dim3(128), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a,
-                           flip, h.partials, h.skip, h.skip_stride, o, h.coef, h.coef_stride);
-        II_HIP(ctx, hipGetLastError());
-        return II_OK;
-      }
-    }
-    HopOrder ok = o;
-    ok.bs = kBlock;
-    if (ok.mode == 1 && o.bs != kBlock) ok = HopOrder();  // strip orders are built for kBlock
-    dim3 grid(blocks_for(g.Vh), 1);
-    hipLaunchKernelGGL((k_hop<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX>), grid,
-                       dim3(kBlock), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a, flip,
-                       h.partials, h.skip, h.skip_stride, ok, h.coef, h.coef_stride);
-  } else if constexpr (std::is_same<Gauge, GaugeF64Flat>::value) {
-    return set_error(ctx, II_ERR_STATE, "the flat FP64 gauge form serves single-rhs hops only");
+    constexpr int bs = SpIn::kScaled ? kBlock : 64;  // sites per block
+    const HopOrder o = ctx->hop_order.mode == 1 ? strip_order(g, ctx->hop_order.W, bs) : HopOrder();
+    const dim3 grid(blocks_for(g.Vh, bs));
+    if constexpr (SpIn::kScaled)
+      hipLaunchKernelGGL((k_hop<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX>), grid,
+                         dim3(kBlock), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a,
+                         flip, h.partials, h.skip, h.skip_stride, o, h.coef, h.coef_stride);
+    else
+      hipLaunchKernelGGL((k_hop_split<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX>), grid,
+                         dim3(kBlock), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a,
+                         flip, h.partials, h.skip, o, h.coef);
+  } else if constexpr (GaugePrec<Gauge>::value < 0) {
+    return set_error(ctx, II_ERR_STATE, "this gauge form serves single-rhs hops only");
   } else {
     constexpr int TS = MrhsShape<Gauge>::TS, MAXT = MrhsShape<Gauge>::MAXT;
     constexpr int P = GaugePrec<Gauge>::value;
@@ -417,7 +522,7 @@ ii_status dispatch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, cons
 }  // namespace
 
 int hop_dot_parts(const Geom& g, int nrhs, int precision) {
-  if (nrhs == 1) return blocks_for(g.Vh);
+  if (nrhs == 1) return blocks_for(g.Vh, precision >= II_PREC_HALF ? kBlock : 64);
   const int ts = precision == II_PREC_DOUBLE ? MrhsShape<GaugeF64>::TS
                                              : MrhsShape<GaugeF32r12>::TS;
   return (g.Vh + ts - 1) / ts;
@@ -430,27 +535,14 @@ int hop_dot_parts(const Geom& g, int nrhs, int precision) {
 ii_status tune_hop(ii_context* ctx) {
   ctx->hop_tuned = true;
   const Geom& g = ctx->g;
-  const int P = g.Lxh * g.L[1];
   std::vector<HopOrder> cands(1);
-  // contiguous order with 128 threads per block (FP64 hops without partial sums; 512
-  // would cap the FP64 stencil's 256 registers and spill)
-  if (g.Vh >= 8 * 128) {
-    HopOrder o;
-    o.bs = 128;
-    cands.push_back(o);
-  }
-  const bool tiled = P % kBlock == 0 && g.L[3] % 8 == 0 && g.Vh >= 8 * kBlock;
+  const bool tiled = strip_order(g, 1, 64).mode == 1 && g.Vh >= 8 * kBlock;
   if (tiled)
     for (int W : {1, 2, 4, 8, 16})
-      if ((g.L[3] / 8) % W == 0) cands.push_back(HopOrder{1, W, P / kBlock});
+      if (strip_order(g, W, 64).mode == 1) cands.push_back(strip_order(g, W, 64));
   if (const char* env = std::getenv("II_HOP_ORDER")) {
     HopOrder o;
-    if (env[0] == '1' && tiled) {
-      o.mode = 1;
-      o.W = env[1] == ':' ? std::atoi(env + 2) : 4;
-      o.bpp = P / kBlock;
-      if (o.W < 1 || (g.L[3] / 8) % o.W) o = HopOrder();
-    }
+    if (env[0] == '1' && tiled) o = strip_order(g, env[1] == ':' ? std::atoi(env + 2) : 4, 64);
     ctx->hop_order = o;
     ctx->tune_report = "hop order forced by II_HOP_ORDER";
     return II_OK;
@@ -496,7 +588,7 @@ ii_status tune_hop(ii_context* ctx) {
     if (cands[i].mode)
       std::snprintf(buf, sizeof buf, " strip%d=%.4f", cands[i].W, ms);
     else
-      std::snprintf(buf, sizeof buf, " contig/bs%d=%.4f", cands[i].bs, ms);
+      std::snprintf(buf, sizeof buf, " contig=%.4f", ms);
     rep += buf;
     if (ms < best) {
       best = ms;
@@ -600,6 +692,15 @@ ii_status tune_mrhs(ii_context* ctx, int P, int nrhs) {
   return II_OK;
 }
 
+// Link loads of the single-rhs hop: a solver's hops read the whole gauge field
+// one after the other, so while it stays in the 256 MB Infinity Cache beside
+// the vectors the links are loaded with the default policy; a larger field is
+// streamed (kNT), which keeps the neighbour spinors in L2.  Default against
+// kNT: FP64 5.0 / 6.0 us at 12x10x14x18, 16.8 / 18.7 us at 16^3x32 (75 MB of
+// links), 52.3 / 51.1 us at 20^3x40 (184 MB), 329 / 262 us at 32^3x64; FP32
+// 31.1 / 42.0 us at 24^3x48 (127 MB), 134.6 / 123.0 us at 32^3x64 (403 MB).
+static bool links_cached(unsigned long long gauge_bytes) { return gauge_bytes <= (128ull << 20); }
+
 ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* out,
                 const double2* x, const double2* dv, int rs) {
   const Geom& g = ctx->g;
@@ -608,10 +709,11 @@ ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* o
   StF64 so{out, g.stride};
   SpF64 sx{x ? x : in, g.stride, rs};
   SpF64 sd{dv ? dv : in, g.stride, rs};
-  if (h.nrhs == 1 && (unsigned long long)72 * g.stride * sizeof(double2) < (1ull << 32)) {
-    GaugeF64Flat gf{ctx->gauge64, g.stride};
-    return dispatch_hop(ctx, sin, gf, so, sx, sd, h);
-  }
+  const unsigned long long gb = (unsigned long long)72 * g.stride * sizeof(double2);
+  if (h.nrhs == 1 && links_cached(gb))
+    return dispatch_hop(ctx, sin, GaugeF64Flat<0>{ctx->gauge64, g.stride}, so, sx, sd, h);
+  if (h.nrhs == 1 && gb < (1ull << 32))
+    return dispatch_hop(ctx, sin, GaugeF64Flat<kNT>{ctx->gauge64, g.stride}, so, sx, sd, h);
   GaugeF64 gf{ctx->gauge64, g.stride};
   return dispatch_hop(ctx, sin, gf, so, sx, sd, h);
 }
@@ -620,10 +722,13 @@ ii_status hop32(ii_context* ctx, const HopSpec& h, const float2* in, float2* out
                 const float2* x, const float2* dv) {
   const Geom& g = ctx->g;
   SpF32 sin{in, g.stride};
-  GaugeF32r12 gf{(const float2*)ctx->gauge_lp[II_PREC_SINGLE], g.stride};
+  const float2* links = (const float2*)ctx->gauge_lp[II_PREC_SINGLE];
+  GaugeF32r12 gf{links, g.stride};
   StF32 so{out, g.stride};
   SpF32 sx{x ? x : in, g.stride};
   SpF32 sd{dv ? dv : in, g.stride};
+  if (h.nrhs == 1 && links_cached((unsigned long long)48 * g.stride * sizeof(float2)))
+    return dispatch_hop(ctx, sin, GaugeF32r12T<0>{links, g.stride}, so, sx, sd, h);
   return dispatch_hop(ctx, sin, gf, so, sx, sd, h);
 }
 

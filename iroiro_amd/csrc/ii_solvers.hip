@@ -691,8 +691,8 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
   const Geom& g = ctx->g;
   II_CHECK(ensure_ru_scalars(ctx, 1));
   RUScal* sc = dev_scal(ctx);
-  int nb = hop_blocks(g);
-  II_CHECK(ensure_partials(ctx, (size_t)nb + 8));
+  const int nb = hop_blocks(g), nh = hop_dot_parts(g, 1, II_PREC_DOUBLE);
+  II_CHECK(ensure_partials(ctx, (size_t)std::max(nb, nh) + 8));
   double* part = ctx->partials;
   double* tmp2 = nullptr;
   {
@@ -727,7 +727,7 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
     int n = std::min(chunk, maxiter - queued);
     for (int i = 0; i < n; ++i) {
       II_CHECK(ddagdP(ctx, 0, kappa, fp, fs, fq, ft, &fp, part, 1, skip, ss));
-      hipLaunchKernelGGL(k_fin_pap, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, sc, nullptr,
+      hipLaunchKernelGGL(k_fin_pap, dim3(1), dim3(kBlock), 0, ctx->stream, part, nh, sc, nullptr,
                          0, 0);
       II_CHECK(cg_blas_P(ctx, 0, fp, fs, fr, fx, 0, sc, 1, part, nb));
       hipLaunchKernelGGL(k_fin_rr, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, sc, 0);
@@ -2696,8 +2696,8 @@ ii_status ii_autotune(ii_context* ctx, char* report, size_t len) {
 // Tuning file: one line per choice, for one lattice.
 //   iroiro-hip tuning 1
 //   lattice Lx Ly Lz Lt
-//   hop mode W bpp bs                      (the single-rhs FP64 hop's order)
-//   mrhs P nrhs rb mode W bpp bs           (each tuned multi-rhs precision P)
+//   hop mode W bpp 256                     (the single-rhs FP64 hop's order)
+//   mrhs P nrhs rb mode W bpp 256          (each tuned multi-rhs precision P)
 //   net nrhs rg0..rg3 by0..by3 bz0..bz3    (the network stages)
 ii_status ii_tune_save(ii_context* ctx, const char* path) {
   if (!ctx || !path) return II_ERR_BAD_ARG;
@@ -2707,13 +2707,13 @@ ii_status ii_tune_save(ii_context* ctx, const char* path) {
   std::fprintf(f, "iroiro-hip tuning 1\nlattice %d %d %d %d\n", g.L[0], g.L[1], g.L[2], g.L[3]);
   if (ctx->hop_tuned) {
     const HopOrder& o = ctx->hop_order;
-    std::fprintf(f, "hop %d %d %d %d\n", o.mode, o.W, o.bpp, o.bs);
+    std::fprintf(f, "hop %d %d %d %d\n", o.mode, o.W, o.bpp, kBlock);
   }
   for (int P = 0; P < 4; ++P)
     if (ctx->mrhs_nrhs[P] > 0) {
       const HopOrder& o = ctx->mrhs_ord[P];
       std::fprintf(f, "mrhs %d %d %d %d %d %d %d\n", P, ctx->mrhs_nrhs[P], ctx->mrhs_rb[P], o.mode,
-                   o.W, o.bpp, o.bs);
+                   o.W, o.bpp, kBlock);
     }
   int nn = 0, rg[4], by[4], bz[4];
   bnet_shapes_get(ctx, &nn, rg, by, bz);
@@ -2747,14 +2747,14 @@ ii_status ii_tune_load(ii_context* ctx, const char* path) {
   ii_status st = II_OK;
   while (st == II_OK && std::fgets(line, sizeof line, f)) {
     HopOrder o;
-    int P = 0, n = 0, rb = 0;
+    int P = 0, n = 0, rb = 0, last = 0;
     int v[13];
-    if (std::sscanf(line, "hop %d %d %d %d", &o.mode, &o.W, &o.bpp, &o.bs) == 4) {
+    if (std::sscanf(line, "hop %d %d %d %d", &o.mode, &o.W, &o.bpp, &last) == 4) {
       ctx->hop_order = o;
       ctx->hop_tuned = true;
       ctx->tune_report = "hop order loaded from a tuning file";
     } else if (std::sscanf(line, "mrhs %d %d %d %d %d %d %d", &P, &n, &rb, &o.mode, &o.W, &o.bpp,
-                           &o.bs) == 7) {
+                           &last) == 7) {
       if (P < 0 || P > 3 || n < 1 || rb < 1) {
         st = set_error(ctx, II_ERR_BAD_ARG, "bad mrhs line in tuning file");
         break;

@@ -112,6 +112,9 @@ struct StF64 {
 #pragma unroll
     for (int k = 0; k < 12; ++k) st_at<double2, kNT>(p, (uint32_t)(k * stride), (uint32_t)site, v[k]);
   }
+  __device__ __forceinline__ void st1(int site, int comp, C v) const {
+    st_at<double2, kNT>(p, (uint32_t)(comp * stride), (uint32_t)site, v);
+  }
   __device__ __forceinline__ StF64 rhs(int r) const { return StF64{p + (size_t)r * 12 * stride, stride}; }
 };
 
@@ -136,6 +139,9 @@ struct StF32 {
   __device__ __forceinline__ void st(int site, const C v[12]) const {
 #pragma unroll
     for (int k = 0; k < 12; ++k) st_at<float2, kNT>(p, (uint32_t)(k * stride), (uint32_t)site, v[k]);
+  }
+  __device__ __forceinline__ void st1(int site, int comp, C v) const {
+    st_at<float2, kNT>(p, (uint32_t)(comp * stride), (uint32_t)site, v);
   }
   __device__ __forceinline__ StF32 rhs(int r) const { return StF32{p + (size_t)r * 12 * stride, stride}; }
 };
@@ -268,7 +274,9 @@ struct GaugeF64 {
 // The whole FP64 gauge field in one descriptor (72 components in the scalar
 // offset): the single-rhs FP64 hop runs 3-4% faster this way than with one
 // descriptor per block (0.282 against 0.293 ms at 32^3x64), so it is used
-// wherever the field fits 4 GiB (V/2 up to about 3.7M sites).
+// wherever the field fits 4 GiB (V/2 up to about 3.7M sites).  CP: cache
+// policy of the link loads (links_cached in ii_dslash.hip).
+template <int CP>
 struct GaugeF64Flat {
   using R = double;
   using C = double2;
@@ -278,11 +286,12 @@ struct GaugeF64Flat {
 #pragma unroll
     for (int k = 0; k < 9; ++k)
       U[k / 3][k % 3] =
-          ld_at<double2, kNT>(p, (uint32_t)(((par * 4 + mu) * 9 + k) * stride), (uint32_t)site);
+          ld_at<double2, CP>(p, (uint32_t)(((par * 4 + mu) * 9 + k) * stride), (uint32_t)site);
   }
 };
 
-struct GaugeF32r12 {
+template <int CP>
+struct GaugeF32r12T {
   using R = float;
   using C = float2;
   const float2* __restrict__ p;  // [2][4][6][stride]
@@ -291,10 +300,11 @@ struct GaugeF32r12 {
     const float2* b = p + (size_t)((par * 4 + mu) * 6) * (size_t)stride;
 #pragma unroll
     for (int k = 0; k < 6; ++k)
-      U[k / 3][k % 3] = ld_at<float2, kNT>(b, (uint32_t)(k * stride), (uint32_t)site);
+      U[k / 3][k % 3] = ld_at<float2, CP>(b, (uint32_t)(k * stride), (uint32_t)site);
     r12_third_row(U, tflip);
   }
 };
+using GaugeF32r12 = GaugeF32r12T<kNT>;
 
 template <typename TT>
 struct GaugeLoR12 {
@@ -719,12 +729,12 @@ __device__ __forceinline__ void wilson_hop_site(typename SpIn::C acc[4][3], cons
 }
 
 // XCD-aware block order: hardware dispatches block b to XCD b % 8; the
-// remap gives each XCD a contiguous range of logical blocks so that
-// neighbouring sites (and the rhs of one site tile) share an L2.
+// remap gives each XCD a contiguous range of logical blocks (the first
+// nblocks % 8 XCDs one more) so that neighbouring sites (and the rhs of one
+// site tile) share an L2.
 __host__ __device__ __forceinline__ int xcd_remap(int b, int nblocks) {
-  const int nx = 8;
-  if (nblocks % nx) return b;
-  return (b % nx) * (nblocks / nx) + b / nx;
+  const int nx = 8, x = b % nx, q = nblocks / nx, r = nblocks % nx;
+  return x * q + (x < r ? x : r) + b / nx;
 }
 
 // First half site of the logical block that physical block b handles.
