@@ -49,6 +49,7 @@ struct HopOrder {
   int mode = 0;
   int W = 4;
   int bpp = 1;
+  int bs = 256;  // block size, the fourth number of a tuning file's order
 };
 
 // Solver scalars kept on the device so that iterations need no host sync.

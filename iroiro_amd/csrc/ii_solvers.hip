@@ -2696,8 +2696,8 @@ ii_status ii_autotune(ii_context* ctx, char* report, size_t len) {
 // Tuning file: one line per choice, for one lattice.
 //   iroiro-hip tuning 1
 //   lattice Lx Ly Lz Lt
-//   hop mode W bpp 256                     (the single-rhs FP64 hop's order)
-//   mrhs P nrhs rb mode W bpp 256          (each tuned multi-rhs precision P)
+//   hop mode W bpp bs                      (the single-rhs FP64 hop's order)
+//   mrhs P nrhs rb mode W bpp bs           (each tuned multi-rhs precision P)
 //   net nrhs rg0..rg3 by0..by3 bz0..bz3    (the network stages)
 ii_status ii_tune_save(ii_context* ctx, const char* path) {
   if (!ctx || !path) return II_ERR_BAD_ARG;
@@ -2707,13 +2707,13 @@ ii_status ii_tune_save(ii_context* ctx, const char* path) {
   std::fprintf(f, "iroiro-hip tuning 1\nlattice %d %d %d %d\n", g.L[0], g.L[1], g.L[2], g.L[3]);
   if (ctx->hop_tuned) {
     const HopOrder& o = ctx->hop_order;
-    std::fprintf(f, "hop %d %d %d %d\n", o.mode, o.W, o.bpp, kBlock);
+    std::fprintf(f, "hop %d %d %d %d\n", o.mode, o.W, o.bpp, o.bs);
   }
   for (int P = 0; P < 4; ++P)
     if (ctx->mrhs_nrhs[P] > 0) {
       const HopOrder& o = ctx->mrhs_ord[P];
       std::fprintf(f, "mrhs %d %d %d %d %d %d %d\n", P, ctx->mrhs_nrhs[P], ctx->mrhs_rb[P], o.mode,
-                   o.W, o.bpp, kBlock);
+                   o.W, o.bpp, o.bs);
     }
   int nn = 0, rg[4], by[4], bz[4];
   bnet_shapes_get(ctx, &nn, rg, by, bz);
@@ -2747,14 +2747,14 @@ ii_status ii_tune_load(ii_context* ctx, const char* path) {
   ii_status st = II_OK;
   while (st == II_OK && std::fgets(line, sizeof line, f)) {
     HopOrder o;
-    int P = 0, n = 0, rb = 0, last = 0;
+    int P = 0, n = 0, rb = 0;
     int v[13];
-    if (std::sscanf(line, "hop %d %d %d %d", &o.mode, &o.W, &o.bpp, &last) == 4) {
+    if (std::sscanf(line, "hop %d %d %d %d", &o.mode, &o.W, &o.bpp, &o.bs) == 4) {
       ctx->hop_order = o;
       ctx->hop_tuned = true;
       ctx->tune_report = "hop order loaded from a tuning file";
     } else if (std::sscanf(line, "mrhs %d %d %d %d %d %d %d", &P, &n, &rb, &o.mode, &o.W, &o.bpp,
-                           &last) == 7) {
+                           &o.bs) == 7) {
       if (P < 0 || P > 3 || n < 1 || rb < 1) {
         st = set_error(ctx, II_ERR_BAD_ARG, "bad mrhs line in tuning file");
         break;
