@@ -480,8 +480,8 @@ ii_status ii_qprop_multishift(ii_context* ctx, double kappa, const int site[4],
  * warm-up; nrhs > 1 times the fused multi-rhs hop.  avg_ms per launch. */
 ii_status ii_bench_hop(ii_context* ctx, int precision, int nrhs, int nrep, double* avg_ms);
 /* Launch-shape autotuner: times the admissible site traversals of the
- * single-rhs hop on this lattice (run automatically before the first FP64
- * single-rhs hop) and, for 12 rhs in each storage precision, the fused
+ * single-rhs hop on this lattice (a context starts with the contiguous
+ * order) and, for 12 rhs in each storage precision, the fused
  * multi-rhs hop's rhs per block and tile order (run automatically before a
  * batch's first multi-rhs hop of that precision); reports the timings and
  * the choices as text. */

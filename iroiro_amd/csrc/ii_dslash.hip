@@ -149,37 +149,43 @@ k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
   }
 }
 
-// hop_epilogue for the three colours of one output spin (the accumulation
-// type is the field's; the sums over sites are FP64).
-template <int EPI, typename R, typename C, typename SpX>
+// hop_epilogue for the three colours of one output spin, in FP64 arithmetic
+// (18 to 30 operations a thread beside the hop's 330).  shift, p: the term of
+// RUpdFold (shift = 0: none).
+template <int EPI, typename C, typename SpX>
 __device__ __forceinline__ void hop_epilogue_spin(C o[3], const C xs[3], int hs, int spin,
-                                                  const SpX& dr, double alpha, double ds[3]) {
+                                                  const SpX& dr, double alpha, double shift,
+                                                  const SpX& p, double ds[3]) {
   if constexpr (EPI == kEpiStore) return;
-  R u = R(0), v = R(0), w = R(0);
+  using R = decltype(C::x);
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     C d = o[c];
     if constexpr (EPI == kEpiDot || EPI == kEpiRUpd || EPI == kEpiCDot) d = dr.ld(hs, 3 * spin + c);
-    if constexpr (EPI == kEpiDot) u = fma(d.x, o[c].x, fma(d.y, o[c].y, u));
     if constexpr (EPI == kEpiRUpd) {
-      o[c].x = fma(-(R)alpha, o[c].x, d.x);
-      o[c].y = fma(-(R)alpha, o[c].y, d.y);
+      double ox = o[c].x, oy = o[c].y;
+      if (shift != 0.0) {
+        const C pv = p.ld(hs, 3 * spin + c);
+        ox = fma(shift, (double)pv.x, ox);
+        oy = fma(shift, (double)pv.y, oy);
+      }
+      o[c].x = (R)fma(-alpha, ox, (double)d.x);
+      o[c].y = (R)fma(-alpha, oy, (double)d.y);
     }
-    if constexpr (EPI == kEpiNorm || EPI == kEpiRUpd)
-      u = fma(o[c].x, o[c].x, fma(o[c].y, o[c].y, u));
+    const double ox = o[c].x, oy = o[c].y, dx = d.x, dy = d.y;
+    if constexpr (EPI == kEpiDot) ds[0] = fma(dx, ox, fma(dy, oy, ds[0]));
+    if constexpr (EPI == kEpiNorm || EPI == kEpiRUpd) ds[0] = fma(ox, ox, fma(oy, oy, ds[0]));
     if constexpr (EPI == kEpiCDot) {
-      u = fma(d.x, o[c].x, fma(d.y, o[c].y, u));
-      v = fma(d.x, o[c].y, fma(-d.y, o[c].x, v));
+      ds[0] = fma(dx, ox, fma(dy, oy, ds[0]));
+      ds[1] = fma(dx, oy, fma(-dy, ox, ds[1]));
     }
     if constexpr (EPI == kEpiTS) {
-      u = fma(o[c].x, xs[c].x, fma(o[c].y, xs[c].y, u));
-      v = fma(o[c].x, xs[c].y, fma(-o[c].y, xs[c].x, v));
-      w = fma(o[c].x, o[c].x, fma(o[c].y, o[c].y, w));
+      const double xx = xs[c].x, xy = xs[c].y;
+      ds[0] = fma(ox, xx, fma(oy, xy, ds[0]));
+      ds[1] = fma(ox, xy, fma(-oy, xx, ds[1]));
+      ds[2] = fma(ox, ox, fma(oy, oy, ds[2]));
     }
   }
-  ds[0] = (double)u;
-  ds[1] = (double)v;
-  ds[2] = (double)w;
 }
 
 // Single-rhs hop of the FP64 and FP32 fields, bound by latency on lattices
@@ -200,11 +206,22 @@ template <bool G5IN, bool G5OUT, bool XPAY, int EPI, typename SpIn, typename Gau
 __global__ void __launch_bounds__(256)
 k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
             typename SpIn::R a, bool tbc_flip, double* __restrict__ partials,
-            const int* __restrict__ skip, HopOrder order, const double* __restrict__ coef) {
+            const int* __restrict__ skip, HopOrder order, const double* __restrict__ coef,
+            RUpdFold ru) {
   using C = typename SpIn::C;
   using R = typename SpIn::R;
   __shared__ C part[4][12][64];  // [dimension][3 spin + colour][site]
+  __shared__ double dsh[4];
   if (skip && skip[0]) return;
+  double den[kMaxFold / 256] = {};
+  if constexpr (EPI == kEpiRUpd) {  // requested before the hop, summed after it
+    if (ru.den)
+#pragma unroll
+      for (int j = 0; j < kMaxFold / 256; ++j) {
+        const int i = j * 256 + threadIdx.x;
+        if (i < ru.nden) den[j] = ru.den[i];
+      }
+  }
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int base = hop_block_base(g, order, blockIdx.x, gridDim.x, 64);
@@ -232,7 +249,30 @@ k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
   else if (w == 1) dimension(std::integral_constant<int, 1>());
   else if (w == 2) dimension(std::integral_constant<int, 2>());
   else dimension(std::integral_constant<int, 3>());
+  if constexpr (EPI == kEpiRUpd) {
+    double d = 0.0;
+#pragma unroll
+    for (int j = 0; j < kMaxFold / 256; ++j) d += den[j];
+    d = wave_sum(d);
+    if (lane == 0) dsh[w] = d;
+  }
   __syncthreads();
+  double alpha = 0.0, shift = 0.0;
+  SpX sp = dv;
+  if constexpr (EPI == kEpiRUpd) {
+    if (ru.den) {
+      double d = dsh[0] + dsh[1] + dsh[2] + dsh[3];
+      shift = ru.shift;
+      if (shift != 0.0) {
+        d = fma(shift, *ru.den2, d);
+        sp.p = (decltype(sp.p))ru.p;
+      }
+      alpha = *ru.num / d;
+      if (blockIdx.x == 0 && threadIdx.x == 0) *ru.alpha = alpha;
+    } else {
+      alpha = coef[0];
+    }
+  }
   double dsum[3] = {0.0, 0.0, 0.0};
   if (valid) {
     C o[3], xsv[3];
@@ -252,7 +292,7 @@ k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
         o[c] = cadd(o[c], xsv[c]);
       }
     }
-    hop_epilogue_spin<EPI, R>(o, xsv, hs, so, dv, EPI == kEpiRUpd ? coef[0] : 0.0, dsum);
+    hop_epilogue_spin<EPI>(o, xsv, hs, so, dv, alpha, shift, sp, dsum);
 #pragma unroll
     for (int c = 0; c < 3; ++c) out.st1(hs, 3 * so + c, o[c]);
   }
@@ -461,7 +501,7 @@ ii_status launch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, const 
     else
       hipLaunchKernelGGL((k_hop_split<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX>), grid,
                          dim3(kBlock), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a,
-                         flip, h.partials, h.skip, o, h.coef);
+                         flip, h.partials, h.skip, o, h.coef, h.ru);
   } else if constexpr (GaugePrec<Gauge>::value < 0) {
     return set_error(ctx, II_ERR_STATE, "this gauge form serves single-rhs hops only");
   } else {
@@ -491,7 +531,11 @@ ii_status dispatch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, cons
     return set_error(ctx, II_ERR_BAD_ARG, "unknown hop epilogue");
   if (h.epi == kEpiTS && !h.xpay)
     return set_error(ctx, II_ERR_BAD_ARG, "kEpiTS needs the XPAY term");
-  if (h.epi == kEpiRUpd && !h.coef)
+  if (h.epi == kEpiRUpd && h.ru.den &&
+      (h.nrhs != 1 || SpIn::kScaled || h.ru.nden > kMaxFold || !h.ru.num || !h.ru.alpha ||
+       (h.ru.shift != 0.0 && (!h.ru.p || !h.ru.den2))))
+    return set_error(ctx, II_ERR_BAD_ARG, "bad folded residual update");
+  if (h.epi == kEpiRUpd && !h.coef && !h.ru.den)
     return set_error(ctx, II_ERR_BAD_ARG, "residual-update hop without its scalars");
   const int sel = (h.g5in ? 32 : 0) | (h.g5out ? 16 : 0) | (h.xpay ? 8 : 0) | h.epi;
 #define II_CASE(A, B, CC, E)                                                                 \
@@ -530,8 +574,10 @@ int hop_dot_parts(const Geom& g, int nrhs, int precision) {
 
 // Autotuner of the single-rhs hop traversal (HopOrder): times every
 // admissible order on this lattice with the FP64 hop and keeps the fastest.
-// Runs once per context on the first single-rhs FP64 hop, never inside a
-// stream capture.  II_HOP_ORDER=0 or II_HOP_ORDER=1:W forces an order.
+// Runs when ii_autotune asks for it, never inside a stream capture: the
+// contiguous order that a context starts with is within 2% of the best strip
+// everywhere (us, contiguous / best strip: 17.8 / 17.5 at 16^3x32, 139.0 /
+// 139.3 at 32^4, 262.8 / 262.0 at 32^3x64).  II_HOP_ORDER=0 or II_HOP_ORDER=1:W forces an order.
 ii_status tune_hop(ii_context* ctx) {
   ctx->hop_tuned = true;
   const Geom& g = ctx->g;
@@ -607,7 +653,10 @@ ii_status tune_hop(ii_context* ctx) {
 // give more, smaller blocks) and the tile order (contiguous per XCD, or
 // strips of W time slices, as for the single-rhs hop).  Timed with the
 // plain hop (no epilogue) of this precision on scratch fields of nrhs rhs,
-// one warm-up and 3 timed launches per candidate.
+// one warm-up and 3 timed launches per candidate.  Candidates are 12 and 6
+// rhs per block: 4, 3 and 2 lost on every lattice and precision (12 / 6 / 4 /
+// 3 / 2 at 32^3x64: FP64 1.86 / 1.79 / 1.84 / 2.03 / 2.53 ms, FP32 0.98 / 1.01
+// / 1.07 / 1.12 / 1.27, FP16 0.48 / 0.56 / 0.58 / 0.74 / 1.07).
 ii_status tune_mrhs(ii_context* ctx, int P, int nrhs) {
   if (P < 0 || P > 3 || nrhs < 2) return II_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -617,7 +666,7 @@ ii_status tune_mrhs(ii_context* ctx, int P, int nrhs) {
   const Geom& g = ctx->g;
   constexpr int TS = 64, RBMAX = 768 / 64;
   std::vector<int> rbs;
-  for (int rb : {RBMAX, 6, 4, 3, 2})
+  for (int rb : {RBMAX, 6})
     if (rb <= std::min(nrhs, RBMAX) && std::find(rbs.begin(), rbs.end(), rb) == rbs.end())
       rbs.push_back(rb);
   if (rbs.empty() || rbs.front() != std::min(nrhs, RBMAX)) rbs.insert(rbs.begin(), std::min(nrhs, RBMAX));
@@ -704,7 +753,8 @@ static bool links_cached(unsigned long long gauge_bytes) { return gauge_bytes <=
 ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* out,
                 const double2* x, const double2* dv, int rs) {
   const Geom& g = ctx->g;
-  if (h.nrhs == 1 && !ctx->hop_tuned && !h.no_tune) II_CHECK(tune_hop(ctx));
+  static const bool forced = std::getenv("II_HOP_ORDER") != nullptr;
+  if (forced && h.nrhs == 1 && !ctx->hop_tuned && !h.no_tune) II_CHECK(tune_hop(ctx));
   SpF64 sin{in, g.stride, rs};
   StF64 so{out, g.stride};
   SpF64 sx{x ? x : in, g.stride, rs};

@@ -26,6 +26,22 @@ namespace ii {
 enum HopEpilogue {
   kEpiStore = 0, kEpiDot = 1, kEpiNorm = 2, kEpiRUpd = 3, kEpiCDot = 4, kEpiTS = 5
 };
+// Single-rhs FP64 / FP32 hops also take kEpiRUpd with the scalar and a shift
+// folded in (HopSpec::ru):
+//   alpha = *num / (sum of den[0 .. nden) + shift * *den2),   stored to *alpha
+//   r = dv - alpha (o + shift p)
+// every block sums the few partial sums itself, in the same order, so a CG
+// step needs no launch of its own for alpha.
+constexpr int kMaxFold = 1024;  // partial sums a consumer sums itself; more go through psum
+struct RUpdFold {
+  const double* den = nullptr;
+  int nden = 0;                  // at most kMaxFold
+  const double* den2 = nullptr;  // |p|^2, read when shift != 0
+  double shift = 0.0;
+  const double* num = nullptr;
+  double* alpha = nullptr;
+  const void* p = nullptr;       // the field of the shift term, in the hop's precision
+};
 constexpr int epi_sums(int epi) { return epi == kEpiStore ? 0 : epi == kEpiCDot ? 2 : epi == kEpiTS ? 3 : 1; }
 
 struct HopSpec {
@@ -37,6 +53,7 @@ struct HopSpec {
   int epi = kEpiStore;
   const double* coef = nullptr;  // kEpiRUpd: alpha of rhs r at coef[r * coef_stride]
   int coef_stride = 0;
+  RUpdFold ru;                   // kEpiRUpd, single rhs: used when ru.den is set
   int nrhs = 1;
   double* partials = nullptr;
   // optional per-rhs skip flags: rhs r is skipped when skip[r * skip_stride] != 0

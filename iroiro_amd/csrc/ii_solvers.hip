@@ -684,16 +684,122 @@ __global__ void k_scal_init(RUScal* sc, const double* __restrict__ rr, const dou
   S = z;
 }
 
+// ============================================================ FP64 / FP32 single-rhs steps
+// Sum of n values by every thread of a 256-thread block, the same order in
+// every block (s: 5 doubles of shared memory; a barrier before reuse is the
+// caller's).
+__device__ __forceinline__ double fold_sum(const double* __restrict__ v, int n, double* s) {
+  double d = 0.0;
+  for (int i = threadIdx.x; i < n; i += kBlock) d += v[i];
+  d = wave_sum(d);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = d;
+  __syncthreads();
+  return s[0] + s[1] + s[2] + s[3];
+}
+
+// dst = sum of n partial sums (where they are too many for every consumer
+// block to add up itself)
+__global__ void __launch_bounds__(kFinThreads)
+k_psum(const double* __restrict__ v, int n, double* __restrict__ dst) {
+  double d = 0.0;
+  for (int i = threadIdx.x; i < n; i += kFinThreads) d += v[i];
+  d = block_sum(d);
+  if (threadIdx.x == 0) *dst = d;
+}
+
+// The partial sums of a single-rhs hop as its consumers take them: as they
+// are up to kMaxFold, else reduced to one value at dst.  A consumer block
+// reads them from L2 (8 KB at 16^3x32) while its own loads are in flight; at
+// 24^3x48 (5184 sums) every block would read 41 KB, more than its share of
+// the fields, so one block sums them first (3 us of a 300 us step).
+ii_status fold_parts(ii_context* ctx, const double* parts, int n, double* dst,
+                     const double** out, int* nout) {
+  *out = parts;
+  *nout = n;
+  if (n <= kMaxFold) return II_OK;
+  hipLaunchKernelGGL(k_psum, dim3(1), dim3(kFinThreads), 0, ctx->stream, parts, n, dst);
+  II_HIP(ctx, hipGetLastError());
+  *out = dst;
+  *nout = 1;
+  return II_OK;
+}
+
+// Iterations to queue before the host looks at the solver's state again:
+// about as many as the mean convergence rate so far still asks for.  Too few
+// cost a synchronisation (about 20 us), too many run as empty launches
+// (about 2 us each, 5 or 6 an iteration).  left, made: log of the reduction
+// still to make and made so far, in `count` iterations.
+int next_chunk(int chunk, int count, double left, double made) {
+  const int twice = std::min(2 * chunk, 64);
+  if (!(made > 0.0) || !(left > 0.0) || count < 4) return twice;
+  const double need = left / made * count;
+  if (!(need < 64.0)) return twice;
+  return std::max(1, std::min(twice, (int)std::ceil(need * (need > 12.0 ? 0.8 : 1.0))));
+}
+
+// One queued step of the reference CG ends here: x += alpha p and p = r +
+// beta p in one pass over the flat arrays of n double2, with beta from the
+// partial sums of |r|^2.  The state is double-buffered: every block reads
+// `cur`, one writes `nxt` (copied on when the solve is done), so the launch
+// needs no scalar kernel before it.  (solver_CG.cpp:131-160)
+__global__ void __launch_bounds__(kBlock)
+k_cg_xp(size_t n, double2* __restrict__ x, double2* __restrict__ p, const double2* __restrict__ r,
+        const RUScal* __restrict__ cur, RUScal* __restrict__ nxt,
+        const double* __restrict__ parts, int nparts) {
+  __shared__ double sh[4];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (cur->done) {
+    if (first) *nxt = *cur;
+    return;
+  }
+  const double rr = fold_sum(parts, nparts, sh);
+  const double a = cur->alpha, b = rr / cur->rr;
+  const bool ok = finite(a) && finite(rr) && finite(b);
+  if (ok) {
+    const size_t step = (size_t)gridDim.x * kBlock;
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += step) {
+      double2 xv = x[i], pv = p[i];
+      const double2 rv = r[i];
+      xv.x = fma(a, pv.x, xv.x);
+      xv.y = fma(a, pv.y, xv.y);
+      pv.x = fma(pv.x, b, rv.x);
+      pv.y = fma(pv.y, b, rv.y);
+      x[i] = xv;
+      p[i] = pv;
+    }
+  }
+  if (first) {
+    RUScal s = *cur;
+    s.rr = rr;
+    s.beta = b;
+    s.count += 1;
+    if (!ok) {
+      s.nan = 1;
+      s.done = 1;
+    } else if (rr * s.snorm < s.prec) {
+      s.done = 1;
+      s.iter = s.count - 1;
+    }
+    *nxt = s;
+  }
+}
+
 // ============================================================ reference CG
-// Solver_CG::solve semantics on Fopr_DdagD: x0 = b (solver_CG.cpp:40).
+// Solver_CG::solve semantics on Fopr_DdagD: x0 = b (solver_CG.cpp:40).  One
+// iteration is five launches: t = H p; q = Dhat p with |q|^2 = <p, A p>;
+// t = H g5 q; r -= alpha Dhat^dag q with |r|^2 (A p is never stored); x and p
+// together.  That is 7 passes over vectors beside the hops' neighbours, where
+// <p, A p>, the x and r update and the p update in kernels of their own took
+// 11, and three launches more.  Solver_CG on host arrays: 2.39 -> 1.90 ms at
+// 8^3x16 (launches), 53.2 -> 48.7 ms at 24^3x48 (HBM, and the host copies).
 ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2* b, double prec,
                        int maxiter, ii_solver_output* out) {
   const Geom& g = ctx->g;
-  II_CHECK(ensure_ru_scalars(ctx, 1));
+  II_CHECK(ensure_ru_scalars(ctx, 2));
   RUScal* sc = dev_scal(ctx);
-  const int nb = hop_blocks(g), nh = hop_dot_parts(g, 1, II_PREC_DOUBLE);
-  II_CHECK(ensure_partials(ctx, (size_t)std::max(nb, nh) + 8));
-  double* part = ctx->partials;
+  const int nh = hop_dot_parts(g, 1, II_PREC_DOUBLE);
+  II_CHECK(ensure_partials(ctx, (size_t)2 * nh + 8));
+  double *part = ctx->partials, *part2 = part + nh, *one = part2 + nh;
   double* tmp2 = nullptr;
   {
     void* p;
@@ -706,8 +812,6 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
   II_CHECK(fieldP(ctx, 12, 0, 1, &fs));
   II_CHECK(fieldP(ctx, 13, 0, 1, &fq));
   II_CHECK(fieldP(ctx, 14, 0, 1, &ft));
-  const int ss = kScalInts;
-  const int* skip = &sc[0].done;
   II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   II_CHECK(copy64(ctx, x, b));
   // r = b - A x
@@ -720,25 +824,55 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
   hipLaunchKernelGGL(k_scal_init, dim3(1), dim3(64), 0, ctx->stream, sc, tmp2, tmp2 + 1, prec,
                      0.0, 0.0, 0);
   II_HIP(ctx, hipGetLastError());
-  int queued = 0;
-  int chunk = 1;
+  const size_t n = half_elems(g);
+  const int xpblk = std::min(blocks_for((long)n, 2 * kBlock), 2048);
+  int queued = 0, chunk = 4;
   bool conv = false;
+  double rr0 = -1.0;
   while (queued < maxiter) {
-    int n = std::min(chunk, maxiter - queued);
-    for (int i = 0; i < n; ++i) {
-      II_CHECK(ddagdP(ctx, 0, kappa, fp, fs, fq, ft, &fp, part, 1, skip, ss));
-      hipLaunchKernelGGL(k_fin_pap, dim3(1), dim3(kBlock), 0, ctx->stream, part, nh, sc, nullptr,
-                         0, 0);
-      II_CHECK(cg_blas_P(ctx, 0, fp, fs, fr, fx, 0, sc, 1, part, nb));
-      hipLaunchKernelGGL(k_fin_rr, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, sc, 0);
-      II_CHECK(cg_p_P(ctx, 0, fr, fp, fp, sc, 1));
+    const int m = std::min(chunk, maxiter - queued);
+    for (int i = 0; i < m; ++i, ++queued) {
+      RUScal *cur = sc + (queued & 1), *nxt = sc + ((queued + 1) & 1);
+      const double* pp = nullptr;
+      HopSpec h;
+      h.skip = &cur->done;
+      h.out_par = 1;
+      II_CHECK(hopP(ctx, 0, h, fp, ft, nullptr, nullptr));
+      h.out_par = 0;
+      h.a = -kappa * kappa;
+      h.xpay = true;
+      h.epi = kEpiNorm;
+      h.partials = part;
+      II_CHECK(hopP(ctx, 0, h, ft, fq, &fp, nullptr));  // q = Dhat p, |q|^2
+      II_CHECK(fold_parts(ctx, part, nh, one, &h.ru.den, &h.ru.nden));
+      h.out_par = 1;
+      h.a = 1.0;
+      h.xpay = false;
+      h.g5in = true;
+      h.epi = kEpiStore;
+      II_CHECK(hopP(ctx, 0, h, fq, ft, nullptr, nullptr));
+      h.out_par = 0;
+      h.a = -kappa * kappa;
+      h.xpay = true;
+      h.g5in = false;
+      h.g5out = true;
+      h.epi = kEpiRUpd;
+      h.partials = part2;
+      h.ru.num = &cur->rr;
+      h.ru.alpha = &cur->alpha;
+      II_CHECK(hopP(ctx, 0, h, ft, fr, &fq, &fr));  // r -= alpha Dhat^dag q, |r|^2
+      int np = 0;
+      II_CHECK(fold_parts(ctx, part2, nh, one + 1, &pp, &np));
+      hipLaunchKernelGGL(k_cg_xp, dim3(xpblk), dim3(kBlock), 0, ctx->stream, n, x, (double2*)fp.v,
+                         (const double2*)fr.v, cur, nxt, pp, np);
+      II_HIP(ctx, hipGetLastError());
     }
-    queued += n;
-    II_CHECK(read_scalars(ctx, 1));
-    const RUScal& H = host_scal(ctx)[0];
+    II_CHECK(read_scalars(ctx, 2));
+    const RUScal& H = host_scal(ctx)[queued & 1];
     if (H.nan) return set_error(ctx, II_ERR_NAN, "non-finite CG scalar");
     if (H.done) { conv = true; break; }
-    chunk = std::min(chunk * 2, 64);
+    if (rr0 < 0.0) rr0 = H.rmax2;
+    chunk = next_chunk(chunk, H.count, std::log(H.rr * H.snorm / H.prec), std::log(rr0 / H.rr));
   }
   // diff = |A x - b| / |b|  (solver_CG.cpp:69-71)
   II_CHECK(ddagdP(ctx, 0, kappa, fx, fs, fq, ft, nullptr, nullptr, 1, nullptr, 0));
@@ -747,8 +881,8 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
   II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
   double h[3];
   II_HIP(ctx, hipMemcpyAsync(h, tmp2, 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  II_CHECK(read_scalars(ctx, 1));
-  const RUScal& H = host_scal(ctx)[0];
+  II_CHECK(read_scalars(ctx, 2));
+  const RUScal& H = host_scal(ctx)[queued & 1];
   float ms = 0.f;
   II_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   if (out) {
@@ -2705,10 +2839,8 @@ ii_status ii_tune_save(ii_context* ctx, const char* path) {
   std::FILE* f = std::fopen(path, "w");
   if (!f) return set_error(ctx, II_ERR_BAD_ARG, std::string("cannot create tuning file ") + path);
   std::fprintf(f, "iroiro-hip tuning 1\nlattice %d %d %d %d\n", g.L[0], g.L[1], g.L[2], g.L[3]);
-  if (ctx->hop_tuned) {
-    const HopOrder& o = ctx->hop_order;
-    std::fprintf(f, "hop %d %d %d %d\n", o.mode, o.W, o.bpp, o.bs);
-  }
+  const HopOrder& h = ctx->hop_order;
+  std::fprintf(f, "hop %d %d %d %d\n", h.mode, h.W, h.bpp, h.bs);
   for (int P = 0; P < 4; ++P)
     if (ctx->mrhs_nrhs[P] > 0) {
       const HopOrder& o = ctx->mrhs_ord[P];
