@@ -21,8 +21,8 @@
 // the 9 paths.  The adjoint layer is the same kernel with the paths
 // mirrored and W -> W^dag (channel-transposed): T_{+mu}^dag = T_{-mu}.
 //
-// Weight gradient: VALU, gw[d][o][i] = sum_{x,c} g[o](x) conj(T_d in[i](x)),
-// per-block partials in FP32 then a fixed-order FP64 sum.
+// Weight gradient: FP32 matrix cores, gw[d][o][i] = sum_{x,c} g[o](x)
+// conj(T_d in[i](x)), per-block partials in FP32 then a fixed-order FP64 sum.
 #include "ii_ops.h"
 #include "ii_stencil.h"
 
@@ -207,16 +207,6 @@ __device__ __forceinline__ void net_transport(const float2* __restrict__ base, u
     }
 }
 
-// r12 FP32 link with every offset in the lane offset (for kernels whose
-// threads may hold sites of different parities)
-__device__ __forceinline__ void ld_link_lane(const float2* __restrict__ gp, int stride, int par,
-                                             int mu, int site, bool flip, float2 U[3][3]) {
-  const uint32_t loff = (uint32_t)((par * 4 + mu) * 6 * stride + site);
-#pragma unroll
-  for (int k = 0; k < 6; ++k) U[k / 3][k % 3] = ld_at(gp, (uint32_t)(k * stride), loff);
-  r12_third_row(U, flip);
-}
-
 // Path d of half site s (parity par): neighbour half index (in parity
 // par ^ (d > 0)) and link.
 __device__ __forceinline__ int net_path(const Geom& g, const GaugeF32r12& gauge, int flip, int d,
@@ -329,123 +319,243 @@ __global__ void __launch_bounds__(kLayerThreads) k_net_layer(LayerArgs a) {
   }
 }
 
-// Weight gradient partials.  Block b covers global sites q in
-// [b*spb, (b+1)*spb) of the 2*Vh sites (q = par*Vh + hs), in stages of 16
-// sites; thread groups split the sites of a stage, each thread of a group
-// owns a 2x2 tile of the (4*COUT) x (4*CIN) complex matrix of every path.
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(kWgThreads)
-k_net_wgrad(Geom g, const float2* __restrict__ in, const float2* __restrict__ gout,
-            const float2* __restrict__ gaugep, int flip, int spb, float2* __restrict__ partial) {
-  constexpr int ROWS = 4 * COUT, COLS = 4 * CIN;
-  constexpr int OWN = ROWS * COLS / 4;
-  constexpr int G = kWgThreads / OWN;
-  constexpr int ST = 16;
-  static_assert(OWN * G == kWgThreads, "tile owners must divide the block");
-  __shared__ float2 sg[ST][3][ROWS];
-  __shared__ float2 sta[ST][3][COLS];
-  const int tid = threadIdx.x;
-  const int owner = tid % OWN, grp = tid / OWN;
-  const int r0 = 2 * (owner / (COLS / 2)), c0 = 2 * (owner % (COLS / 2));
+// Weight gradient partials on the matrix cores, in FP32 throughout
+// (v_mfma_f32_16x16x4_f32):
+//   gw[d][o][i] = sum_{x,c} g[o](x) conj((T_d in[i])(x))
+// is, per path, a product of the local field's 32 complex rows (8 channels x
+// 4 spins at the site itself) with the transported field's columns over
+// k = (site, colour, re/im).  The side with one channel is the transported one
+// where a layer has one (CT = 1): for the last layer that is the gradient,
+//   sum_x g (T_d in)^dag = sum_y (T_d^dag g)(y) in(y)^dag, T_d^dag = T_mirror(d),
+// and then the columns of all nine paths make one product of 36.
+// Re and Im of the result are rows of their own: waves 0, 1 form
+// Re = gr tr + gi ti, waves 2, 3 Im = gi tr - gr ti, 16 rows each.
+// A block covers kWgSites sites at a time: both fields are staged in LDS as
+// [re/im][row][3 site + colour] (rows padded to 100 floats: the 16 rows of a
+// b128 read fall on different banks), the local operands then stay in
+// registers for all paths, and the next path's spinors and links are requested
+// before a path's products.  Two blocks per CU (registers).  One pair's
+// gradients at 16^3x32 (two 8x8 layers, one 1x8, one 8x1): 0.89 ms, where FP32
+// products on the VALU took 2.0 ms; with the reduction below, net_loss_grad of
+// 4 pairs 44.7 -> 18.9 ms on host arrays.  8x8 is bound by the FP32 matrix rate
+// (221 kFLOP per site), the others by the transports' loads.  Error against 64
+// bits on Gaussian fields, 1x8 / 8x8 / 8x1: 1.4 / 3.6 / 1.4e-7 on the VALU,
+// 1.2 / 2.5 / 1.2e-7 here (one-channel sums go over 8 accumulators for that).
+constexpr int kWgSites = 32;
+constexpr int kWgK = 3 * kWgSites;   // k of one re/im half
+constexpr int kWgRow = kWgK + 4;     // padded LDS row
+
+struct WgRaw {
+  float2 v[12];  // neighbour spinor, [3 spin + colour]
+  float2 u[6];   // r12 link
+  bool dag, flip;
+};
+
+// Requests path d's spinor (channel i of `f`) and link at site q (parity par,
+// half site hs).
+__device__ __forceinline__ void wg_request(const Geom& g, const float2* __restrict__ f, int i,
+                                           const float2* __restrict__ gaugep, int flip, int d,
+                                           int par, int hs, const SiteCoord& sc, WgRaw& r) {
   const size_t cs = (size_t)24 * g.stride;
-  const GaugeF32r12 gauge{gaugep, g.stride};
-  float2 acc[kPaths][2][2];
+  int nb = hs;
+  r.dag = false;
+  r.flip = false;
+  if (d > 0) {
+    const int mu = (d - 1) >> 1;
+    const bool fw = ((d - 1) & 1) == 0;
+    nb = neighbour(g, sc, hs, mu, fw);
+    r.dag = !fw;
+    r.flip = flip && mu == 3 && sc.t == (fw ? g.L[3] - 1 : 0);
+    const uint32_t lo = (uint32_t)(((fw ? par : 1 - par) * 4 + mu) * 6 * g.stride + (fw ? hs : nb));
 #pragma unroll
-  for (int d = 0; d < kPaths; ++d)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[d][i][j] = make_float2(0.f, 0.f);
-  const int nq = 2 * g.Vh;
-  const int q0 = blockIdx.x * spb;
-  const int q1 = min(q0 + spb, nq);
-  for (int qb = q0; qb < q1; qb += ST) {
-    for (int e = tid; e < ST * COUT * 12; e += kWgThreads) {
-      const int x = e % ST, rest = e / ST, comp = rest % 12, o = rest / 12;
-      const int q = qb + x;
-      float2 v = make_float2(0.f, 0.f);
-      if (q < q1) {
-        const int par = q >= g.Vh, hs = q - par * g.Vh;
-        v = ld_at(gout, 0u, (uint32_t)(o * cs + (par * 12 + comp) * g.stride + hs));
-      }
-      sg[x][comp % 3][4 * o + comp / 3] = v;
-    }
-#pragma unroll
-    for (int d = 0; d < kPaths; ++d) {
-      __syncthreads();
-      for (int e = tid; e < ST * CIN; e += kWgThreads) {
-        const int x = e % ST, i = e / ST;
-        const int q = qb + x;
-        float2 w[4][3];
-        if (q < q1) {
-          const int par = q >= g.Vh, hs = q - par * g.Vh;
-          const SiteCoord sc = decode_site(g, hs, par);
-          float2 U[3][3];
-          bool dag = false;
-          int nb = hs;
-          if (d > 0) {
-            const int mu = (d - 1) >> 1;
-            const bool fw = ((d - 1) & 1) == 0;
-            nb = neighbour(g, sc, hs, mu, fw);
-            if (fw) {
-              ld_link_lane(gaugep, g.stride, par, mu, hs, flip && mu == 3 && sc.t == g.L[3] - 1, U);
-            } else {
-              ld_link_lane(gaugep, g.stride, 1 - par, mu, nb, flip && mu == 3 && sc.t == 0, U);
-              dag = true;
-            }
-          }
-          const int npar = d == 0 ? par : 1 - par;
-          net_transport(in, 0u, g.stride, (uint32_t)(i * cs + npar * 12 * g.stride + nb), d != 0,
-                        dag, U, w);
-        } else {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) w[t][c] = make_float2(0.f, 0.f);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) sta[x][c][4 * i + t] = w[t][c];
-      }
-      __syncthreads();
-      for (int x = grp; x < ST; x += G)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const float2 ga = sg[x][c][r0], gb = sg[x][c][r0 + 1];
-          const float2 ta = sta[x][c][c0], tb = sta[x][c][c0 + 1];
-          cmacc(acc[d][0][0], ta, ga);
-          cmacc(acc[d][0][1], tb, ga);
-          cmacc(acc[d][1][0], ta, gb);
-          cmacc(acc[d][1][1], tb, gb);
-        }
-    }
-    __syncthreads();
+    for (int k = 0; k < 6; ++k) r.u[k] = ld_at(gaugep, (uint32_t)(k * g.stride), lo);
   }
-  constexpr int NE = COUT * CIN * 16;
-  float2* dst = partial + (size_t)(blockIdx.x * G + grp) * kPaths * NE;
+  const int npar = d == 0 ? par : 1 - par;
+  const uint32_t lo = (uint32_t)(i * cs + npar * 12 * g.stride + nb);
 #pragma unroll
-  for (int d = 0; d < kPaths; ++d)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int row = r0 + i, col = c0 + j;
-        const int o = row >> 2, s = row & 3, ci = col >> 2, t = col & 3;
-        dst[(size_t)d * NE + (o * CIN + ci) * 16 + 4 * s + t] = acc[d][i][j];
-      }
+  for (int k = 0; k < 12; ++k) r.v[k] = ld_at(f, (uint32_t)(k * g.stride), lo);
 }
 
-// gacc[e] += scale * sum_p partial[p][e], fixed order, FP64 sum.
-__global__ void k_net_wreduce(const float2* __restrict__ partial, int np, int ne, float scale,
-                              float2* __restrict__ gacc) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
+// w = M v of a requested path (M = 1, U or U^dag)
+__device__ __forceinline__ void wg_transport(const WgRaw& r, bool link, float2 w[12]) {
+  if (!link) {
+#pragma unroll
+    for (int k = 0; k < 12; ++k) w[k] = r.v[k];
+    return;
+  }
+  float2 U[3][3];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) U[k / 3][k % 3] = r.u[k];
+  r12_third_row(U, r.flip);
+  if (r.dag) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = a; b < 3; ++b) {
+        const float2 x = U[a][b], y = U[b][a];
+        U[a][b] = make_float2(y.x, -y.y);
+        U[b][a] = make_float2(x.x, -x.y);
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      float2 acc = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int b = 0; b < 3; ++b) cmac(acc, U[a][b], r.v[3 * t + b]);
+      w[3 * t + a] = acc;
+    }
+}
+
+// one channel's spinor at site x of the stage into rows row0 .. row0 + 3
+__device__ __forceinline__ void wg_store(float* __restrict__ s, int plane, int row0, int x,
+                                         const float2 w[12]) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int i = (row0 + t) * kWgRow + 3 * x + c;
+      s[i] = w[3 * t + c].x;
+      s[plane + i] = w[3 * t + c].y;
+    }
+}
+
+// T: transported field, CT channels; Lf: local field, 8 channels.  swap: the
+// roles of the last layer (local = in, transported = g, mirrored paths).
+// Block b covers global sites q in [b*spb, (b+1)*spb) of the 2*Vh sites
+// (q = par*Vh + hs).
+template <int CT>
+__global__ void __launch_bounds__(kWgThreads, 2)
+k_net_wgrad(Geom g, const float2* __restrict__ T, const float2* __restrict__ Lf,
+            const float2* __restrict__ gaugep, int flip, int swap, int spb,
+            float* __restrict__ partial) {
+  constexpr int NT = CT == 8 ? 2 : 3;          // 16-column tiles of one product
+  constexpr int NP = CT == 8 ? kPaths : 1;     // products per stage
+  constexpr int NA = CT == 8 ? 1 : 8;          // accumulators, for shorter FP32 sums
+  constexpr int LP = 32 * kWgRow, TP = 16 * NT * kWgRow;  // one re/im plane
+  __shared__ __attribute__((aligned(16))) float sL[2 * LP];
+  __shared__ __attribute__((aligned(16))) float sT[2 * TP];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kq = lane >> 4, l16 = lane & 15;
+  const int reim = kq & 1, k0 = (kq >> 1) * (kWgK / 2);
+  const int im = wv >> 1, rb = wv & 1;         // Re or Im rows, block of 16 rows
+  f32x4 acc[NP][NT][NA];
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int h = 0; h < NA; ++h) acc[p][n][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (CT == 1) {  // the columns past 9 paths x 4 spins stay zero
+    for (int e = tid; e < 2 * TP; e += kWgThreads) sT[e] = 0.f;
+  }
+  const int nq = 2 * g.Vh;
+  const int q0 = blockIdx.x * spb, q1 = min(q0 + spb, nq);
+  const int x = tid & (kWgSites - 1), ch = tid / kWgSites;  // site of the stage, channel
+  for (int qb = q0; qb < q1; qb += kWgSites) {
+    const bool live = qb + x < q1;
+    const int q = live ? qb + x : q1 - 1;
+    const int par = q >= g.Vh, hs = q - par * g.Vh;
+    const SiteCoord sc = decode_site(g, hs, par);
+    const float z = live ? 1.0f : 0.0f;  // sites past the end add nothing
+    WgRaw loc, raw;
+    wg_request(g, Lf, ch, gaugep, flip, 0, par, hs, sc, loc);
+    if (CT == 8) wg_request(g, T, ch, gaugep, flip, 0, par, hs, sc, raw);
+    __syncthreads();  // the last stage's products have read sL and sT
+    {
+      float2 w[12];
+#pragma unroll
+      for (int k = 0; k < 12; ++k) w[k] = make_float2(z * loc.v[k].x, z * loc.v[k].y);
+      wg_store(sL, LP, 4 * ch, x, w);
+    }
+    f32x4 A[kWgK / 8];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if (CT == 8) {
+        float2 w[12];
+        wg_transport(raw, p > 0, w);
+        if (p > 0) __syncthreads();
+        wg_store(sT, TP, 4 * ch, x, w);
+        __syncthreads();
+        if (p + 1 < NP) wg_request(g, T, ch, gaugep, flip, p + 1, par, hs, sc, raw);
+      } else {
+        for (int d = ch; d < kPaths; d += kWgThreads / kWgSites) {
+          float2 w[12];
+          wg_request(g, T, 0, gaugep, flip, swap ? mirror_path(d) : d, par, hs, sc, raw);
+          wg_transport(raw, d > 0, w);
+          wg_store(sT, TP, 4 * d, x, w);
+        }
+        __syncthreads();
+      }
+      if (p == 0) {
+        const float* a = sL + (im ? 1 - reim : reim) * LP + (16 * rb + l16) * kWgRow + k0;
+        const float sg = im && reim ? -1.0f : 1.0f;
+#pragma unroll
+        for (int j = 0; j < kWgK / 8; ++j) A[j] = *(const f32x4*)(a + 4 * j) * sg;
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const float* bp = sT + reim * TP + (16 * n + l16) * kWgRow + k0;
+#pragma unroll
+        for (int j = 0; j < kWgK / 8; ++j) {
+          const f32x4 B = *(const f32x4*)(bp + 4 * j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            f32x4& s = acc[p][n][(4 * j + e) % NA];
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(A[j][e], B[e], s, 0, 0, 0);
+          }
+        }
+      }
+    }
+  }
+  // D row 4 kq + r of the wave's 16, column l16; partials as the weights,
+  // [d][o][i][4 s + t] (re, im)
+  constexpr int NE = CT * 8 * 16;
+  float* dst = partial + (size_t)blockIdx.x * kPaths * NE * 2 + im;
+  const float sg = swap && im ? -1.0f : 1.0f;  // swapped: the conjugate
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+      for (int h = NA / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int k = 0; k < h; ++k) acc[p][n][k] += acc[p][n][k + h];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * rb + 4 * kq + r, col = 16 * n + l16;
+        const int lc = row >> 2, ls = row & 3, ts = col & 3;
+        const int d = CT == 8 ? p : col >> 2, tc = CT == 8 ? col >> 2 : 0;
+        if (d >= kPaths) continue;
+        const int e = swap ? 4 * ts + ls : 4 * ls + ts;
+        dst[2 * ((size_t)d * NE + (lc * CT + tc) * 16 + e)] = sg * acc[p][n][0][r];
+      }
+    }
+}
+
+// gacc[e] += scale * sum_p partial[p][e], fixed order, FP64 sum: 64 entries a
+// block, 16 threads an entry (one thread an entry left 5 blocks summing 8192
+// partials each: 2.4 ms for a one-channel layer, now 22 us).
+__global__ void __launch_bounds__(1024)
+k_net_wreduce(const float2* __restrict__ partial, int np, int ne, float scale,
+              float2* __restrict__ gacc) {
+  __shared__ double2 part[16][64];
+  const int e = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
   double sr = 0.0, si = 0.0;
-  for (int p = 0; p < np; ++p) {
-    const float2 v = partial[(size_t)p * ne + e];
-    sr += v.x;
-    si += v.y;
+  if (e < ne)
+    for (int p = sl; p < np; p += 16) {
+      const float2 v = partial[(size_t)p * ne + e];
+      sr += v.x;
+      si += v.y;
+    }
+  part[sl][threadIdx.x & 63] = make_double2(sr, si);
+  __syncthreads();
+  if (sl > 0 || e >= ne) return;
+  for (int k = 1; k < 16; ++k) {
+    sr += part[k][threadIdx.x].x;
+    si += part[k][threadIdx.x].y;
   }
   float2 a = gacc[e];
   a.x += (float)(scale * sr);
@@ -689,30 +799,30 @@ ii_status run_layer(ii_context* ctx, Net* N, int l, bool adj, const float2* in, 
   return set_error(ctx, II_ERR_STATE, "unsupported layer shape");
 }
 
-template <int CIN, int COUT>
-ii_status launch_wgrad(ii_context* ctx, Net* N, const float2* in, const float2* gout,
+// Weight gradient of one layer added to gacc: at most kWgBlocks blocks, so
+// that a block's FP32 sums stay as short as 2048 sites at 32^3x64.
+constexpr int kWgBlocks = 1024;
+template <int CT>
+ii_status launch_wgrad(ii_context* ctx, Net* N, const float2* T, const float2* Lf, bool swap,
                        float2* gacc, float scale) {
   const Geom& g = ctx->g;
-  constexpr int G = kWgThreads / (4 * COUT * CIN);
-  constexpr int NE = COUT * CIN * 16;
-  const int nq = 2 * g.Vh;
-  int nblk = std::min(1024, std::max(1, nq / 64));
-  const int spb = ((nq + nblk - 1) / nblk + 15) / 16 * 16;
-  nblk = (nq + spb - 1) / spb;
-  const size_t need = (size_t)nblk * G * kPaths * NE;
+  constexpr int ne = kPaths * CT * 8 * 16;
+  const int nq = 2 * g.Vh, stages = (nq + kWgSites - 1) / kWgSites;
+  const int spb = (stages + kWgBlocks - 1) / kWgBlocks * kWgSites;
+  const int nblk = (nq + spb - 1) / spb;
+  const size_t need = (size_t)nblk * ne;
   if (need > N->partial_len) {
     if (N->partial) dfree(N->partial);
     N->partial = nullptr;
     II_CHECK(dev_alloc(ctx, &N->partial, need));
     N->partial_len = need;
   }
-  hipLaunchKernelGGL((k_net_wgrad<CIN, COUT>), dim3(nblk), dim3(kWgThreads), 0, ctx->stream, g,
-                     in, gout, (const float2*)ctx->gauge_lp[II_PREC_SINGLE], ctx->tbc_sign < 0,
-                     spb, N->partial);
+  hipLaunchKernelGGL(k_net_wgrad<CT>, dim3(nblk), dim3(kWgThreads), 0, ctx->stream, g, T, Lf,
+                     (const float2*)ctx->gauge_lp[II_PREC_SINGLE], ctx->tbc_sign < 0, swap ? 1 : 0,
+                     spb, (float*)N->partial);
   II_HIP(ctx, hipGetLastError());
-  const int ne = kPaths * NE;
-  hipLaunchKernelGGL(k_net_wreduce, dim3((ne + 255) / 256), dim3(256), 0, ctx->stream, N->partial,
-                     nblk * G, ne, scale, gacc);
+  hipLaunchKernelGGL(k_net_wreduce, dim3((ne + 63) / 64), dim3(1024), 0, ctx->stream, N->partial,
+                     nblk, ne, scale, gacc);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
 }
@@ -721,9 +831,9 @@ ii_status run_wgrad(ii_context* ctx, Net* N, int l, const float2* in, const floa
                     float2* gacc, float scale) {
   II_CHECK(layer_fits(ctx));
   const LayerParams& P = N->L[l];
-  if (P.cin == 1 && P.cout == 8) return launch_wgrad<1, 8>(ctx, N, in, gout, gacc, scale);
-  if (P.cin == 8 && P.cout == 8) return launch_wgrad<8, 8>(ctx, N, in, gout, gacc, scale);
-  if (P.cin == 8 && P.cout == 1) return launch_wgrad<8, 1>(ctx, N, in, gout, gacc, scale);
+  if (P.cin == 1 && P.cout == 8) return launch_wgrad<1>(ctx, N, in, gout, false, gacc, scale);
+  if (P.cin == 8 && P.cout == 8) return launch_wgrad<8>(ctx, N, in, gout, false, gacc, scale);
+  if (P.cin == 8 && P.cout == 1) return launch_wgrad<1>(ctx, N, gout, in, true, gacc, scale);
   return set_error(ctx, II_ERR_STATE, "unsupported layer shape");
 }
 

@@ -86,6 +86,25 @@ def test_layer_weight_gradient_vs_oracle(env, layer):
     assert rel(got, ref) < 1e-5
 
 
+@pytest.mark.parametrize("dims", [(2, 2, 2, 2), (4, 2, 2, 6), (6, 4, 2, 10)])
+@pytest.mark.parametrize("layer", [0, 1, 3])
+def test_layer_weight_gradient_partial_stages(dims, layer):
+    """Lattices of 16, 96 and 480 sites against the kernel's stages of 32: a
+    stage with sites missing, a parity boundary inside a stage, blocks of one
+    stage.  Bar 1e-6: FP32 sums of 192 terms a stage (2^-24 sqrt(192) = 8e-7)."""
+    lat = orc.Lattice(dims)
+    u = lat.apbc(lat.gauge_expH(0.4, 31))
+    rng = np.random.default_rng(50 + layer)
+    cin, cout = WIDTHS[layer], WIDTHS[layer + 1]
+    x = rng.normal(size=cin * lat.full_size).astype(np.float32).astype(np.float64)
+    g = rng.normal(size=cout * lat.full_size).astype(np.float32).astype(np.float64)
+    ctx = ii.Context(dims)
+    ctx.upload_gauge(u)
+    got = ii.LearnedPreconditioner(ctx).layer_wgrad(layer, x, g)
+    ctx.close()
+    assert rel(got, lat.net_layer_wgrad(u, cin, cout, x, g)) < 1e-6
+
+
 def test_network_gradient_vs_oracle_finite_differences(env):
     lat, u, ctx, net = env
     rng = np.random.default_rng(40)
