@@ -552,6 +552,7 @@ ii_status dispatch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, cons
     II_CASE(true, true, false, kEpiStore)
     II_CASE(true, true, true, kEpiStore)
     II_CASE(true, true, true, kEpiDot)
+    II_CASE(true, true, true, kEpiRUpd)
     II_CASE(true, false, false, kEpiStore)
     II_CASE(false, true, false, kEpiStore)
     II_CASE(false, true, true, kEpiStore)

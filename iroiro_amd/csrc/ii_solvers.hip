@@ -901,241 +901,336 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
 }
 
 // ============================================================ multishift CG
-constexpr int kMaxShift = 64;
+constexpr int kMaxShift = 64;  // one lane of a wavefront per shift
 struct MSScal {
-  double rr, pap, alpha, beta, alphap, betap, snorm, prec;
-  double sigma[kMaxShift], csh2[kMaxShift], zeta1[kMaxShift], zeta2[kMaxShift];
-  double zeta[kMaxShift], alphas[kMaxShift], betas[kMaxShift], pp[kMaxShift];
-  int nshift, nshift2, done, count, nconv, nan;
+  double rr, alpha, alphap, betap, snorm, prec;  // alpha: rr / <p0, (A + sigma0) p0>
+  double csh2[kMaxShift], zeta1[kMaxShift], zeta2[kMaxShift];
+  int nshift2, done, count, nconv, nan, pad;
 };
 
-__global__ void k_ms_init(MSScal* S, const double* __restrict__ rrbb, const double* sigma, int n,
-                          double prec) {
-  if (threadIdx.x != 0) return;
-  S->rr = rrbb[0];
-  double bn = sqrt(rrbb[1]);
-  S->snorm = 1.0 / (bn * bn);
-  S->prec = prec;
-  S->alphap = 0.0;
-  S->betap = 1.0;
-  S->nshift = n;
-  S->nshift2 = n;
-  S->done = 0;
-  S->count = 0;
-  S->nconv = -1;
-  S->nan = 0;
-  for (int i = 0; i < n; ++i) {
-    S->sigma[i] = sigma[i];
-    S->csh2[i] = sigma[i] - sigma[0];
-    S->zeta1[i] = 1.0;
-    S->zeta2[i] = 1.0;
-    S->pp[i] = 0.0;
-  }
-}
-
-// The multishift kernels run on even half fields (NC = 12 complex
-// components per site) or on full fields of the full-index operator
-// (NC = 24: both parity blocks, [2][12][stride] = [24][stride]).
-// s += sigma0 p0 ; partial <s, p0>      (multiShiftSolver_CG.cpp:50-55)
-template <int NC, typename T = double2>
-__global__ void __launch_bounds__(kBlock)
-k_ms_sp(Geom g, T* __restrict__ s, const T* __restrict__ p0, const MSScal* S,
-        double* __restrict__ partials) {
-  if (S->done) return;
-  const double sig = S->sigma[0];
-  const int hs = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0.0;
-  if (hs < g.Vh) {
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      size_t i = (size_t)k * g.stride + hs;
-      const T s0 = s[i], p0v = p0[i];
-      double2 sv = make_double2(s0.x, s0.y), pv = make_double2(p0v.x, p0v.y);
-      sv.x = fma(sig, pv.x, sv.x);
-      sv.y = fma(sig, pv.y, sv.y);
-      s[i].x = sv.x;
-      s[i].y = sv.y;
-      acc = fma(sv.x, pv.x, fma(sv.y, pv.y, acc));
+// Both copies of the state, for rr = |b|^2 (start from x = 0); pps[i] =
+// |p_i|^2; consts: 1 and 0.
+__global__ void k_ms_init(MSScal* S, const double* __restrict__ bb, const double* sigma, int n,
+                          double prec, double* __restrict__ pps, double* __restrict__ consts) {
+  const int i = threadIdx.x;
+  for (int k = 0; k < 2; ++k) {
+    MSScal& Z = S[k];
+    Z.csh2[i] = i < n ? sigma[i] - sigma[0] : 0.0;
+    Z.zeta1[i] = Z.zeta2[i] = 1.0;
+    if (i == 0) {
+      Z.rr = bb[0];
+      const double bn = sqrt(bb[0]);
+      Z.snorm = 1.0 / (bn * bn);
+      Z.prec = prec;
+      Z.alpha = Z.alphap = 0.0;
+      Z.betap = 1.0;
+      Z.nshift2 = n;
+      Z.done = Z.count = Z.nan = Z.pad = 0;
+      Z.nconv = -1;
     }
   }
-  acc = block_sum(acc);
-  if (threadIdx.x == 0) partials[blockIdx.x] = acc;
+  pps[i] = bb[0];
+  if (i < 2) consts[i] = i == 0 ? 1.0 : 0.0;
 }
 
-__global__ void k_ms_fin_pap(const double* __restrict__ partials, int nb, MSScal* S) {
-  if (S->done) return;
-  double s = 0.0;
-  for (int i = threadIdx.x; i < nb; i += blockDim.x) s += partials[i];
-  s = block_sum(s);
-  if (threadIdx.x == 0) {
-    S->pap = s;
-    S->beta = -S->rr / s;
-    if (!isfinite(S->beta)) { S->nan = 1; S->done = 1; }
-  }
-}
-
-// x0 -= beta p0 ; r += beta s ; partial |r|^2   (:57-59)
-template <int NC, typename T = double2>
+// p_i = b, x_i = 0 for every shift, r = b (flat arrays of n elements)
+template <typename T>
 __global__ void __launch_bounds__(kBlock)
-k_ms_xr(Geom g, T* __restrict__ x0, const T* __restrict__ p0, T* __restrict__ r,
-        const T* __restrict__ s, const MSScal* S, double* __restrict__ partials) {
-  if (S->done) return;
-  const double b = S->beta;
-  const int hs = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0.0;
-  if (hs < g.Vh) {
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      size_t i = (size_t)k * g.stride + hs;
-      const T x_ = x0[i], p_ = p0[i], r_ = r[i], s_ = s[i];
-      double2 xv = make_double2(x_.x, x_.y), pv = make_double2(p_.x, p_.y);
-      double2 rv = make_double2(r_.x, r_.y), sv = make_double2(s_.x, s_.y);
-      xv.x = fma(-b, pv.x, xv.x);
-      xv.y = fma(-b, pv.y, xv.y);
-      rv.x = fma(b, sv.x, rv.x);
-      rv.y = fma(b, sv.y, rv.y);
-      x0[i].x = xv.x;
-      x0[i].y = xv.y;
-      r[i].x = rv.x;
-      r[i].y = rv.y;
-      acc = fma(rv.x, rv.x, fma(rv.y, rv.y, acc));
-    }
-  }
-  acc = block_sum(acc);
-  if (threadIdx.x == 0) partials[blockIdx.x] = acc;
-}
-
-// rr, alpha and the shift recurrences (:61-83)
-__global__ void k_ms_fin_rr(const double* __restrict__ partials, int nb, MSScal* S) {
-  if (S->done) return;
-  double s = 0.0;
-  for (int i = threadIdx.x; i < nb; i += blockDim.x) s += partials[i];
-  s = block_sum(s);
-  if (threadIdx.x == 0) {
-    double rrp = S->rr;
-    S->rr = s;
-    double alpha = s / rrp;
-    S->alpha = alpha;
-    S->pp[0] = s;
-    double beta = S->beta;
-    double alphah = 1.0 + S->alphap * beta / S->betap;
-    for (int ish = 1; ish < S->nshift2; ++ish) {
-      double zeta = (alphah - S->csh2[ish] * beta) / S->zeta1[ish] + (1.0 - alphah) / S->zeta2[ish];
-      zeta = 1.0 / zeta;
-      double zr = zeta / S->zeta1[ish];
-      S->betas[ish] = beta * zr;
-      S->alphas[ish] = alpha * zr * zr;
-      S->zeta[ish] = zeta;
-    }
-    if (!isfinite(alpha)) { S->nan = 1; S->done = 1; }
+k_ms_start(size_t n, const double2* __restrict__ b, T* __restrict__ x, T* __restrict__ p,
+           T* __restrict__ r, int nshift) {
+  const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const double2 v = b[i];
+  T t, z;
+  t.x = v.x;
+  t.y = v.y;
+  z.x = z.y = 0;
+  r[i] = t;
+  for (int k = 0; k < nshift; ++k) {
+    p[k * n + i] = t;
+    x[k * n + i] = z;
   }
 }
 
-// p0 = alpha p0 + r (:63-64) and, for ish in [1, nshift2):
-// x_i -= betas p_i ; p_i = alphas p_i + zeta r ; partial |p_i|^2 (:73-79)
-template <int NC, typename T = double2>
+// non-temporal access to a complex element
+template <typename T>
+__device__ __forceinline__ T ld_stream(const T* q) {
+  T v;
+  v.x = __builtin_nontemporal_load(&q->x);
+  v.y = __builtin_nontemporal_load(&q->y);
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ void st_stream(T* q, T v) {
+  __builtin_nontemporal_store(v.x, &q->x);
+  __builtin_nontemporal_store(v.y, &q->y);
+}
+
+// One iteration's shift recurrences and vectors (multiShiftSolver_CG.cpp:
+// 57-92, 148-152), after r += beta s has left the partial sums of |r|^2:
+//   beta = -rr_old / <p0, s>, alpha = rr / rr_old
+//   x_i -= betas_i p_i ; p_i = alphas_i p_i + zeta_i r ; partials of |p_i|^2
+// with betas_0 = beta, alphas_0 = alpha, zeta_0 = 1.  Lane i of every
+// wavefront forms the scalars of shift i; the state is double-buffered (every
+// block reads `cur`, one writes `nxt`).  A block takes kMsGroup shifts, so r is
+// read once for them.  The shifts still active follow from the |p_i|^2 of the
+// iteration before (pps; pp_0 is rr itself, as in the reference).  Bound by the
+// four passes over each shift's x and p.
+constexpr int kMsGroup = 2;
+template <typename T>
 __global__ void __launch_bounds__(kBlock)
-k_ms_vec(Geom g, T* __restrict__ x, T* __restrict__ p, const T* __restrict__ r,
-         const MSScal* S, double* __restrict__ partials) {
-  if (S->done) return;
-  const int ish = blockIdx.y;
-  const int hs = blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t he = (size_t)NC * g.stride;
-  if (ish == 0) {
-    if (hs < g.Vh) {
-      const double a = S->alpha;
-#pragma unroll
-      for (int k = 0; k < NC; ++k) {
-        size_t i = (size_t)k * g.stride + hs;
-        const T pv = p[i], rv = r[i];
-        p[i].x = fma((double)pv.x, a, (double)rv.x);
-        p[i].y = fma((double)pv.y, a, (double)rv.y);
+k_ms_vec(size_t n, T* __restrict__ x, T* __restrict__ p, const T* __restrict__ r,
+         const MSScal* __restrict__ cur, MSScal* __restrict__ nxt,
+         const double* __restrict__ parts, int nparts, const double* __restrict__ pps,
+         double* __restrict__ out) {
+  __shared__ double sh[4];
+  const int lane = threadIdx.x & 63;
+  const bool first = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64;
+  if (cur->done) {
+    if (first) {
+      nxt->csh2[lane] = cur->csh2[lane];
+      nxt->zeta1[lane] = cur->zeta1[lane];
+      nxt->zeta2[lane] = cur->zeta2[lane];
+      if (lane == 0) {
+        nxt->rr = cur->rr;
+        nxt->alpha = cur->alpha;
+        nxt->nshift2 = cur->nshift2;
+        nxt->done = 1;
+        nxt->count = cur->count;
+        nxt->nconv = cur->nconv;
+        nxt->nan = cur->nan;
       }
     }
     return;
   }
-  if (ish >= S->nshift2) return;
-  const double bs = S->betas[ish], as = S->alphas[ish], z = S->zeta[ish];
-  double acc = 0.0;
-  if (hs < g.Vh) {
-    T* xi = x + ish * he;
-    T* pi = p + ish * he;
+  const double rr = fold_sum(parts, nparts, sh);
+  int n2 = cur->nshift2;
+  if (cur->count > 0) {
+    const double pp = lane == 0 ? cur->rr : pps[lane] * cur->snorm;
+    const unsigned long long big = __ballot(lane < n2 && pp > cur->prec);
+    if (big) n2 = 64 - __clzll((long long)big);
+  }
+  const double beta = -cur->alpha, alpha = rr / cur->rr;
+  const double alphah = 1.0 + cur->alphap * beta / cur->betap;
+  const double z1 = cur->zeta1[lane], z2 = cur->zeta2[lane];
+  double zeta = 1.0, bs = beta, as = alpha;
+  if (lane > 0 && lane < n2) {
+    zeta = (alphah - cur->csh2[lane] * beta) / z1 + (1.0 - alphah) / z2;
+    zeta = 1.0 / zeta;
+    const double zr = zeta / z1;
+    bs = beta * zr;
+    as = alpha * zr * zr;
+  }
+  const bool ok = finite(alpha) && finite(beta);
+  if (first) {
+    nxt->zeta2[lane] = lane > 0 && lane < n2 ? z1 : z2;
+    nxt->zeta1[lane] = lane > 0 && lane < n2 ? zeta : z1;
+    if (lane == 0) {
+      nxt->rr = rr;
+      nxt->alphap = alpha;
+      nxt->betap = beta;
+      nxt->nshift2 = n2;
+      nxt->count = cur->count + 1;
+      const bool conv = rr * cur->snorm < cur->prec;
+      nxt->nconv = ok && conv ? cur->count : -1;
+      nxt->nan = !ok;
+      nxt->done = !ok || conv;
+    }
+  }
+  if (!ok) return;
+  const int s0 = blockIdx.y * kMsGroup;
+  if (s0 >= n2) return;
+  double b[kMsGroup], a[kMsGroup], z[kMsGroup], acc[kMsGroup];
 #pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      size_t i = (size_t)k * g.stride + hs;
-      const T x_ = xi[i], p_ = pi[i], r_ = r[i];
-      double2 xv = make_double2(x_.x, x_.y), pv = make_double2(p_.x, p_.y);
-      const double2 rv = make_double2(r_.x, r_.y);
-      xv.x = fma(-bs, pv.x, xv.x);
-      xv.y = fma(-bs, pv.y, xv.y);
-      pv.x = fma(pv.x, as, z * rv.x);
-      pv.y = fma(pv.y, as, z * rv.y);
-      xi[i].x = xv.x;
-      xi[i].y = xv.y;
-      pi[i].x = pv.x;
-      pi[i].y = pv.y;
-      acc = fma(pv.x, pv.x, fma(pv.y, pv.y, acc));
-    }
+  for (int k = 0; k < kMsGroup; ++k) {
+    b[k] = __shfl(bs, s0 + k);
+    a[k] = __shfl(as, s0 + k);
+    z[k] = __shfl(zeta, s0 + k);
+    acc[k] = 0.0;
   }
-  acc = block_sum(acc);
-  if (threadIdx.x == 0) partials[(size_t)ish * gridDim.x + blockIdx.x] = acc;
-}
-
-// pp_i, zeta shifts, Nshift2 shrink, stopping test (:79-92, :148-152)
-__global__ void k_ms_tail(const double* __restrict__ partials, int nb, MSScal* S) {
-  if (S->done) return;
-  __shared__ double sums[kMaxShift];
-  for (int ish = 1; ish < S->nshift2; ++ish) {
-    const double* p = partials + (size_t)ish * nb;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) s += p[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) sums[ish] = s;
+  const size_t step = (size_t)gridDim.x * kBlock;
+  for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += step) {
+    const T rv = r[i];
+    T xv[kMsGroup], pv[kMsGroup];
+#pragma unroll
+    for (int k = 0; k < kMsGroup; ++k)
+      if (s0 + k < n2) {
+        xv[k] = ld_stream(x + (s0 + k) * n + i);
+        pv[k] = ld_stream(p + (s0 + k) * n + i);
+      }
+#pragma unroll
+    for (int k = 0; k < kMsGroup; ++k)
+      if (s0 + k < n2) {
+        const double px = pv[k].x, py = pv[k].y;
+        xv[k].x = fma(-b[k], px, (double)xv[k].x);
+        xv[k].y = fma(-b[k], py, (double)xv[k].y);
+        const double qx = fma(px, a[k], z[k] * rv.x), qy = fma(py, a[k], z[k] * rv.y);
+        pv[k].x = qx;
+        pv[k].y = qy;
+        st_stream(x + (s0 + k) * n + i, xv[k]);
+        st_stream(p + (s0 + k) * n + i, pv[k]);
+        acc[k] = fma(qx, qx, fma(qy, qy, acc[k]));
+      }
   }
-  if (threadIdx.x == 0) {
-    for (int ish = 1; ish < S->nshift2; ++ish) {
-      S->pp[ish] = sums[ish] * S->snorm;
-      S->zeta2[ish] = S->zeta1[ish];
-      S->zeta1[ish] = S->zeta[ish];
-    }
-    for (int ish = S->nshift2 - 1; ish >= 0; --ish) {
-      if (S->pp[ish] > S->prec) { S->nshift2 = ish + 1; break; }
-    }
-    S->alphap = S->alpha;
-    S->betap = S->beta;
-    S->count += 1;
-    if (S->rr * S->snorm < S->prec) { S->done = 1; S->nconv = S->count - 1; }
+#pragma unroll
+  for (int k = 0; k < kMsGroup; ++k) {
+    const double v = block_sum(acc[k]);
+    if (threadIdx.x == 0) out[(size_t)(s0 + k) * gridDim.x + blockIdx.x] = v;
   }
 }
 
-// A = D^dag D of the full-index operator D = 1 - kappa H on full fields
-// [2][12][stride] (Fopr_DdagD over Dirac_Wilson, fopr.h:146-153,
-// dirac_wilson.cpp:28-36, 115-118); w: full-field temporary.
-ii_status ddagd_full64(ii_context* ctx, double kappa, const double2* f, double2* out, double2* w,
-                       const int* skip) {
+// |p_i|^2 of the iteration that wrote S, one block per shift
+__global__ void __launch_bounds__(kBlock)
+k_ms_tail(const double* __restrict__ partials, int nb, const MSScal* __restrict__ S,
+          double* __restrict__ pps) {
+  const int i = blockIdx.x;
+  if (S->done || i >= S->nshift2) return;
+  __shared__ double sh[4];
+  const double v = fold_sum(partials + (size_t)i * nb, nb, sh);
+  if (threadIdx.x == 0) pps[i] = v;
+}
+
+// Device scalars of a multishift solve (workspace slot 29): the double-
+// buffered state, then |b|^2, the shifts, |p_i|^2, the constants 1 and 0, and
+// the residuals of the shifts.
+struct MSDev {
+  MSScal* S;
+  double *bb, *sigma, *pps, *consts, *res;
+  MSScal* host;  // pinned
+};
+ii_status ms_dev(ii_context* ctx, MSDev* m) {
+  void *wp = nullptr, *hp = nullptr;
+  II_CHECK(workspace(ctx, 29, 2 * sizeof(MSScal) + (3 * kMaxShift + 8) * sizeof(double), &wp));
+  m->S = (MSScal*)wp;
+  m->bb = (double*)(m->S + 2);
+  m->sigma = m->bb + 4;
+  m->pps = m->sigma + kMaxShift;
+  m->res = m->pps + kMaxShift;
+  m->consts = m->res + kMaxShift;
+  II_CHECK(ensure_host_pin(ctx, sizeof(MSScal), &hp));
+  m->host = (MSScal*)hp;
+  return II_OK;
+}
+
+// The operator A of a multishift solve on fields of T: Dhat^dag Dhat on even
+// half fields (nh = 1, q and t: temporaries), or D^dag D of the full-index
+// D = 1 - kappa H on full fields (nh = 2; Fopr_DdagD over Dirac_Wilson,
+// fopr.h:146-153, dirac_wilson.cpp:28-36, 115-118), which needs no t.
+//   ms_first:  q = D f with partial sums of |q|^2 = <f, A f>
+//   ms_second: r = dv - alpha (D^dag q + shift p) with partial sums of |r|^2,
+//              alpha and the shift term as RUpdFold gives them
+struct MSOp {
+  double kappa;
+  int P;   // II_PREC_DOUBLE or II_PREC_SINGLE
+  int nh;  // half-field blocks per vector
+  SF q, t;
+  int tiles;  // partial sums of one hop
+};
+SF half_of(const MSOp& A, const SF& f, size_t he, int par) {
+  const size_t el = A.P == II_PREC_DOUBLE ? sizeof(double2) : sizeof(float2);
+  return SF{(char*)f.v + (A.nh == 2 ? par : 0) * he * el};
+}
+ii_status ms_first(ii_context* ctx, const MSOp& A, const SF& f, double* part, const int* skip) {
   const size_t he = half_elems(ctx->g);
   HopSpec h;
-  h.a = -kappa;
-  h.xpay = true;
   h.skip = skip;
-  for (int par = 0; par < 2; ++par) {
-    h.out_par = par;
-    II_CHECK(hop64(ctx, h, f + (1 - par) * he, w + par * he, f + par * he, nullptr));
+  if (A.nh == 1) {
+    h.out_par = 1;
+    II_CHECK(hopP(ctx, A.P, h, f, A.t, nullptr, nullptr));
   }
-  h.g5in = h.g5out = true;
-  for (int par = 0; par < 2; ++par) {
+  h.xpay = true;
+  h.epi = kEpiNorm;
+  h.a = A.nh == 1 ? -A.kappa * A.kappa : -A.kappa;
+  for (int par = 0; par < A.nh; ++par) {
     h.out_par = par;
-    II_CHECK(hop64(ctx, h, w + (1 - par) * he, out + par * he, w + par * he, nullptr));
+    h.partials = part + par * A.tiles;
+    const SF x = half_of(A, f, he, par);
+    II_CHECK(hopP(ctx, A.P, h, A.nh == 1 ? A.t : half_of(A, f, he, 1 - par),
+                  half_of(A, A.q, he, par), &x, nullptr));
+  }
+  return II_OK;
+}
+ii_status ms_second(ii_context* ctx, const MSOp& A, const SF& r, const SF& dv, const SF& p,
+                    const RUpdFold& ru, double* part, const int* skip) {
+  const size_t he = half_elems(ctx->g);
+  HopSpec h;
+  h.skip = skip;
+  h.g5in = true;
+  if (A.nh == 1) {
+    h.out_par = 1;
+    II_CHECK(hopP(ctx, A.P, h, A.q, A.t, nullptr, nullptr));
+    h.g5in = false;  // t holds H g5 q
+  }
+  h.g5out = true;
+  h.xpay = true;
+  h.epi = kEpiRUpd;
+  h.a = A.nh == 1 ? -A.kappa * A.kappa : -A.kappa;
+  h.ru = ru;
+  for (int par = 0; par < A.nh; ++par) {
+    h.out_par = par;
+    h.partials = part + par * A.tiles;
+    const SF x = half_of(A, A.q, he, par), d = half_of(A, dv, he, par);
+    h.ru.p = half_of(A, p, he, par).v;
+    II_CHECK(hopP(ctx, A.P, h, A.nh == 1 ? A.t : half_of(A, A.q, he, 1 - par),
+                  half_of(A, r, he, par), &x, &d));
   }
   return II_OK;
 }
 
-__global__ void k_sum2(const double* __restrict__ in, int n, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s += in[i];
-    out[0] = s;
+// Iterates MultiShiftSolver_CG's recursion (multiShiftSolver_CG.cpp:95-152)
+// from x = 0 until |r|^2/|b|^2 < prec or maxiter: six launches an iteration.
+// p: nshift vectors, r: one; m.bb holds |b|^2.  The final state is left in
+// m.host; *conv: whether the test passed.
+template <typename T>
+ii_status ms_iterate(ii_context* ctx, const MSOp& A, const MSDev& m, T* x, T* p, T* r,
+                     const double2* b, const double* shifts, int nshift, double prec, int maxiter,
+                     bool* conv) {
+  const size_t n = half_elems(ctx->g) * A.nh;
+  const int nt = A.tiles * A.nh;  // partial sums of an application of A
+  const int vb = std::min(blocks_for((long)n, 2 * kBlock), kMaxFold);
+  II_CHECK(ensure_partials(ctx, (size_t)2 * nt + (size_t)vb * (nshift + kMsGroup) + 8));
+  double *part = ctx->partials, *part2 = part + nt, *one = part2 + nt, *pv = one + 2;
+  hipLaunchKernelGGL(k_ms_start<T>, dim3(blocks_for((long)n)), dim3(kBlock), 0, ctx->stream, n, b,
+                     x, p, r, nshift);
+  II_HIP(ctx, hipMemcpyAsync(m.sigma, shifts, nshift * sizeof(double), hipMemcpyHostToDevice,
+                             ctx->stream));
+  hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(kMaxShift), 0, ctx->stream, m.S, m.bb, m.sigma,
+                     nshift, prec, m.pps, m.consts);
+  II_HIP(ctx, hipGetLastError());
+  int queued = 0, chunk = 4;
+  *conv = false;
+  double rr0 = -1.0;
+  while (queued < maxiter) {
+    const int k = std::min(chunk, maxiter - queued);
+    for (int it = 0; it < k; ++it, ++queued) {
+      MSScal *cur = m.S + (queued & 1), *nxt = m.S + ((queued + 1) & 1);
+      const double* rp = nullptr;
+      int nr = 0;
+      RUpdFold ru;
+      ru.den2 = m.pps;
+      ru.shift = shifts[0];
+      ru.num = &cur->rr;
+      ru.alpha = &cur->alpha;
+      II_CHECK(ms_first(ctx, A, SF{p}, part, &cur->done));
+      II_CHECK(fold_parts(ctx, part, nt, one, &ru.den, &ru.nden));
+      II_CHECK(ms_second(ctx, A, SF{r}, SF{r}, SF{p}, ru, part2, &cur->done));
+      II_CHECK(fold_parts(ctx, part2, nt, one + 1, &rp, &nr));
+      hipLaunchKernelGGL(k_ms_vec<T>, dim3(vb, (nshift + kMsGroup - 1) / kMsGroup), dim3(kBlock), 0,
+                         ctx->stream, n, x, p, (const T*)r, cur, nxt, rp, nr, m.pps, pv);
+      hipLaunchKernelGGL(k_ms_tail, dim3(nshift), dim3(kBlock), 0, ctx->stream, pv, vb, nxt,
+                         m.pps);
+      II_HIP(ctx, hipGetLastError());
+    }
+    const MSScal& H = *m.host;
+    II_HIP(ctx, hipMemcpyAsync(m.host, m.S + (queued & 1), sizeof(MSScal), hipMemcpyDeviceToHost,
+                               ctx->stream));
+    II_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (H.nan) return set_error(ctx, II_ERR_NAN, "non-finite multishift scalar");
+    if (H.done) { *conv = true; break; }
+    if (rr0 < 0.0) rr0 = 1.0 / H.snorm;
+    chunk = next_chunk(chunk, H.count, std::log(H.rr * H.snorm / H.prec), std::log(rr0 / H.rr));
   }
+  return II_OK;
 }
 
 // multishift on the even Schur system (full = false: x, b even half fields)
@@ -1147,114 +1242,66 @@ ii_status multishift_reference(ii_context* ctx, double kappa, double2* x, const 
   const Geom& g = ctx->g;
   const int nh = full ? 2 : 1;  // half-field blocks per vector
   if (nshift < 1 || nshift > kMaxShift) return set_error(ctx, II_ERR_BAD_ARG, "nshift out of range");
-  int nb = hop_blocks(g);
-  II_CHECK(ensure_partials(ctx, (size_t)nb * nshift + 16));
-  double* part = ctx->partials;
-  void* wp = nullptr;
-  II_CHECK(workspace(ctx, 29, sizeof(MSScal) + (kMaxShift + 8) * sizeof(double), &wp));
-  MSScal* S = (MSScal*)wp;
-  double* aux = (double*)((char*)wp + sizeof(MSScal));  // rr, bb, sigma[...]
-  MSScal* Sh = nullptr;
-  {
-    void* hp = nullptr;
-    II_CHECK(ensure_host_pin(ctx, sizeof(MSScal), &hp));
-    Sh = (MSScal*)hp;
-  }
-  SF fr, fs, fq, ft, fp;
+  MSDev m;
+  II_CHECK(ms_dev(ctx, &m));
+  SF fr, fs, fp;
+  MSOp A;
+  A.kappa = kappa;
+  A.P = II_PREC_DOUBLE;
+  A.nh = nh;
+  A.tiles = hop_dot_parts(g, 1, II_PREC_DOUBLE);
   II_CHECK(fieldP(ctx, 10, 0, nh, &fr));
   II_CHECK(fieldP(ctx, 12, 0, nh, &fs));
-  II_CHECK(fieldP(ctx, 13, 0, nh, &fq));
-  II_CHECK(fieldP(ctx, 14, 0, nh, &ft));
+  II_CHECK(fieldP(ctx, 13, 0, nh, &A.q));
+  II_CHECK(fieldP(ctx, 14, 0, nh, &A.t));
   II_CHECK(fieldP(ctx, 15, 0, nshift * nh, &fp));
-  size_t he = half_elems(g) * nh;
-  double2* p = (double2*)fp.v;
-  // |v|^2 over all nh blocks of a vector into dst (device)
-  auto norm2 = [&](const double2* v, double* dst) -> ii_status {
-    II_CHECK(dot64(ctx, v, v, aux + 8 + kMaxShift - 4, nh));
-    hipLaunchKernelGGL(k_sum2, dim3(1), dim3(64), 0, ctx->stream, aux + 8 + kMaxShift - 4, nh,
-                       dst);
-    II_HIP(ctx, hipGetLastError());
-    return II_OK;
-  };
-  auto apply_A = [&](const double2* f, const int* skip) -> ii_status {
-    if (full) return ddagd_full64(ctx, kappa, f, (double2*)fs.v, (double2*)fq.v, skip);
-    return ddagdP(ctx, 0, kappa, SF{const_cast<double2*>(f)}, fs, fq, ft, nullptr, nullptr, 1,
-                  skip, 0);
-  };
+  const size_t he = half_elems(g) * nh;
   II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-  for (int i = 0; i < nshift; ++i) {
-    II_CHECK(copy64(ctx, p + i * he, b, nh));
-    II_CHECK(zero64(ctx, x + i * he, nh));
-  }
-  II_CHECK(copy64(ctx, (double2*)fr.v, b, nh));
-  II_CHECK(norm2(b, aux));
-  II_CHECK(norm2(b, aux + 1));
-  II_HIP(ctx, hipMemcpyAsync(aux + 2, shifts, nshift * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
-  hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(64), 0, ctx->stream, S, aux, aux + 2, nshift, prec);
+  // |b|^2 over the nh blocks of the vector
+  II_CHECK(dot64(ctx, b, b, m.res, nh));
+  hipLaunchKernelGGL(k_psum, dim3(1), dim3(kFinThreads), 0, ctx->stream, m.res, nh, m.bb);
   II_HIP(ctx, hipGetLastError());
-  const int* skip = &S->done;
-  int queued = 0, chunk = 1;
   bool conv = false;
-  while (queued < maxiter) {
-    int n = std::min(chunk, maxiter - queued);
-    for (int it = 0; it < n; ++it) {
-      II_CHECK(apply_A(p, skip));
-      if (full) {
-        hipLaunchKernelGGL(k_ms_sp<24>, dim3(nb), dim3(kBlock), 0, ctx->stream, g,
-                           (double2*)fs.v, p, S, part);
-        hipLaunchKernelGGL(k_ms_fin_pap, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-        hipLaunchKernelGGL(k_ms_xr<24>, dim3(nb), dim3(kBlock), 0, ctx->stream, g, x, p,
-                           (double2*)fr.v, (const double2*)fs.v, S, part);
-        hipLaunchKernelGGL(k_ms_fin_rr, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-        hipLaunchKernelGGL(k_ms_vec<24>, dim3(nb, nshift), dim3(kBlock), 0, ctx->stream, g, x, p,
-                           (const double2*)fr.v, S, part);
-      } else {
-        hipLaunchKernelGGL(k_ms_sp<12>, dim3(nb), dim3(kBlock), 0, ctx->stream, g,
-                           (double2*)fs.v, p, S, part);
-        hipLaunchKernelGGL(k_ms_fin_pap, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-        hipLaunchKernelGGL(k_ms_xr<12>, dim3(nb), dim3(kBlock), 0, ctx->stream, g, x, p,
-                           (double2*)fr.v, (const double2*)fs.v, S, part);
-        hipLaunchKernelGGL(k_ms_fin_rr, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-        hipLaunchKernelGGL(k_ms_vec<12>, dim3(nb, nshift), dim3(kBlock), 0, ctx->stream, g, x, p,
-                           (const double2*)fr.v, S, part);
-      }
-      hipLaunchKernelGGL(k_ms_tail, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-      II_HIP(ctx, hipGetLastError());
-    }
-    queued += n;
-    II_HIP(ctx, hipMemcpyAsync(Sh, S, sizeof(MSScal), hipMemcpyDeviceToHost, ctx->stream));
-    II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (Sh->nan) return set_error(ctx, II_ERR_NAN, "non-finite multishift scalar");
-    if (Sh->done) { conv = true; break; }
-    chunk = std::min(chunk * 2, 64);
-  }
+  II_CHECK(ms_iterate(ctx, A, m, x, (double2*)fp.v, (double2*)fr.v, b, shifts, nshift, prec,
+                      maxiter, &conv));
   // true residuals (:165-177): diff = max_i |(A + sigma_i) x_i - b|^2 / |b|^2
+  for (int i = 0; i < nshift; ++i) {
+    const SF xi{x + i * he};
+    RUpdFold ru;  // alpha = 1
+    ru.den = m.consts;
+    ru.nden = 1;
+    ru.den2 = m.consts + 1;
+    ru.shift = shifts[i];
+    ru.num = m.consts;
+    ru.alpha = m.bb + 1;
+    double *part = ctx->partials, *part2 = part + nh * A.tiles;
+    II_CHECK(ms_first(ctx, A, xi, part, nullptr));
+    II_CHECK(ms_second(ctx, A, fs, SF{const_cast<double2*>(b)}, xi, ru, part2, nullptr));
+    hipLaunchKernelGGL(k_psum, dim3(1), dim3(kFinThreads), 0, ctx->stream, part2, nh * A.tiles,
+                       m.res + i);
+    II_HIP(ctx, hipGetLastError());
+  }
+  double res[kMaxShift];
+  II_HIP(ctx, hipMemcpyAsync(res, m.res, nshift * sizeof(double), hipMemcpyDeviceToHost,
+                             ctx->stream));
+  II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
   double dmax = -1.0;
   if (per_shift) per_shift->assign(nshift, 0.0);
   for (int i = 0; i < nshift; ++i) {
-    II_CHECK(apply_A(x + i * he, nullptr));
-    II_CHECK(axpby64(ctx, shifts[i], x + i * he, 1.0, (double2*)fs.v, nh));
-    II_CHECK(axpby64(ctx, -1.0, b, 1.0, (double2*)fs.v, nh));
-    II_CHECK(norm2((double2*)fs.v, aux));
-    double h = 0.0;
-    II_HIP(ctx, hipMemcpyAsync(&h, aux, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    double d1 = h * Sh->snorm;
+    const double d1 = res[i] * m.host->snorm;
     if (per_shift) (*per_shift)[i] = std::sqrt(d1);
     if (d1 > dmax) dmax = d1;
   }
-  II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
   float ms = 0.f;
   II_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   if (out) {
-    out->iterations = conv ? Sh->nconv : -1;
+    out->iterations = conv ? m.host->nconv : -1;
     out->diff = dmax;
     out->true_residual = std::sqrt(dmax);
     out->timing_ms = ms;
     out->restarts = 0;
-    out->inner_iterations = Sh->count;
+    out->inner_iterations = m.host->count;
   }
   if (!conv) return set_error(ctx, II_ERR_NOT_CONVERGED, "Not converged.");
   return II_OK;
@@ -1347,67 +1394,23 @@ ii_status multishift_sloppy(ii_context* ctx, double kappa, float2* x32, const do
                             int* iterations) {
   const Geom& g = ctx->g;
   if (!ctx->gauge_lp[II_PREC_SINGLE]) II_CHECK(build_lowprec_gauge(ctx, II_PREC_SINGLE));
-  const int nb = hop_blocks(g);
-  II_CHECK(ensure_partials(ctx, (size_t)nb * nshift + 16));
-  double* part = ctx->partials;
-  void* wp = nullptr;
-  II_CHECK(workspace(ctx, 29, sizeof(MSScal) + (kMaxShift + 8) * sizeof(double), &wp));
-  MSScal* S = (MSScal*)wp;
-  double* aux = (double*)((char*)wp + sizeof(MSScal));
-  MSScal* Sh = nullptr;
-  {
-    void* hp = nullptr;
-    II_CHECK(ensure_host_pin(ctx, sizeof(MSScal), &hp));
-    Sh = (MSScal*)hp;
-  }
-  SF fr, fs, fq, ft, fp;
+  MSDev m;
+  II_CHECK(ms_dev(ctx, &m));
+  SF fr, fp;
+  MSOp A;
+  A.kappa = kappa;
+  A.P = II_PREC_SINGLE;
+  A.nh = 1;
+  A.tiles = hop_dot_parts(g, 1, II_PREC_SINGLE);
   II_CHECK(fieldP(ctx, 32, II_PREC_SINGLE, 1, &fr));
-  II_CHECK(fieldP(ctx, 33, II_PREC_SINGLE, 1, &fs));
-  II_CHECK(fieldP(ctx, 34, II_PREC_SINGLE, 1, &fq));
-  II_CHECK(fieldP(ctx, 35, II_PREC_SINGLE, 1, &ft));
+  II_CHECK(fieldP(ctx, 34, II_PREC_SINGLE, 1, &A.q));
+  II_CHECK(fieldP(ctx, 35, II_PREC_SINGLE, 1, &A.t));
   II_CHECK(fieldP(ctx, 36, II_PREC_SINGLE, nshift, &fp));
-  const size_t he = half_elems(g);
-  float2* p = (float2*)fp.v;
-  float2* r = (float2*)fr.v;
-  II_CHECK(convert_64_to_32(ctx, b64, r, 1));
-  for (int i = 0; i < nshift; ++i) {
-    II_HIP(ctx, hipMemcpyAsync(p + i * he, r, he * sizeof(float2), hipMemcpyDeviceToDevice,
-                               ctx->stream));
-    II_HIP(ctx, hipMemsetAsync(x32 + i * he, 0, he * sizeof(float2), ctx->stream));
-  }
-  II_CHECK(dot64(ctx, b64, b64, aux));
-  II_CHECK(dot64(ctx, b64, b64, aux + 1));
-  II_HIP(ctx, hipMemcpyAsync(aux + 2, shifts, nshift * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
-  hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(64), 0, ctx->stream, S, aux, aux + 2, nshift,
-                     prec1);
-  II_HIP(ctx, hipGetLastError());
-  const int* skip = &S->done;
-  int queued = 0, chunk = 1;
-  while (queued < maxiter) {
-    const int n = std::min(chunk, maxiter - queued);
-    for (int it = 0; it < n; ++it) {
-      II_CHECK(ddagdP(ctx, II_PREC_SINGLE, kappa, SF{p}, fs, fq, ft, nullptr, nullptr, 1, skip,
-                      0));
-      hipLaunchKernelGGL((k_ms_sp<12, float2>), dim3(nb), dim3(kBlock), 0, ctx->stream, g,
-                         (float2*)fs.v, p, S, part);
-      hipLaunchKernelGGL(k_ms_fin_pap, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-      hipLaunchKernelGGL((k_ms_xr<12, float2>), dim3(nb), dim3(kBlock), 0, ctx->stream, g, x32,
-                         p, r, (const float2*)fs.v, S, part);
-      hipLaunchKernelGGL(k_ms_fin_rr, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-      hipLaunchKernelGGL((k_ms_vec<12, float2>), dim3(nb, nshift), dim3(kBlock), 0, ctx->stream,
-                         g, x32, p, (const float2*)r, S, part);
-      hipLaunchKernelGGL(k_ms_tail, dim3(1), dim3(kBlock), 0, ctx->stream, part, nb, S);
-      II_HIP(ctx, hipGetLastError());
-    }
-    queued += n;
-    II_HIP(ctx, hipMemcpyAsync(Sh, S, sizeof(MSScal), hipMemcpyDeviceToHost, ctx->stream));
-    II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (Sh->nan) return set_error(ctx, II_ERR_NAN, "non-finite multishift scalar");
-    if (Sh->done) break;
-    chunk = std::min(chunk * 2, 64);
-  }
-  *iterations = Sh->count;
+  II_CHECK(dot64(ctx, b64, b64, m.bb));
+  bool conv = false;
+  II_CHECK(ms_iterate(ctx, A, m, x32, (float2*)fp.v, (float2*)fr.v, b64, shifts, nshift, prec1,
+                      maxiter, &conv));
+  *iterations = m.host->count;
   return II_OK;
 }
 

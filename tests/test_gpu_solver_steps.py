@@ -1,0 +1,99 @@
+"""The single-rhs solver steps (Solver_CG and MultiShiftSolver_CG on the device)
+where their launches change shape: one tile of 64 sites and less, a ragged last
+tile, and more tiles than a consumer block sums itself (1024); shift counts
+around the groups the vector kernel takes.  The residuals are formed by the
+operator on host arrays, which test_gpu_parity.py pins to the oracle.
+
+Bars: the solvers stop at |r|^2/|b|^2 < prec on the recursion, which drifts
+from the true residual by rounding only (2^-53 times the iteration count and
+the condition number, below 1e-12 here), so the true residual stays below
+1.1 sqrt(prec)."""
+import numpy as np
+import pytest
+
+import iroiro_amd as ii
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+DIMS = [(2, 2, 2, 2), (6, 4, 2, 10), (16, 16, 16, 34)]
+
+
+def operator(dims):
+    lat = orc.Lattice(dims)
+    ctx = ii.Context(dims)
+    D = ii.Dirac_Wilson_EvenOdd(1.0 / (2 * 0.12) - 4.0, lat.apbc(lat.gauge_expH(0.3, 17)), ctx)
+    return ctx, D, ii.Fopr_DdagD(D)
+
+
+@pytest.mark.parametrize("dims", DIMS)
+def test_cg_true_residual(dims):
+    ctx, D, A = operator(dims)
+    b = np.random.default_rng(3).normal(size=D.fsize())
+    x = np.empty_like(b)
+    out = ii.Solver_CG(1e-16, 2000, A).solve(x, b)
+    r = np.linalg.norm(A.mult(x) - b) / np.linalg.norm(b)
+    ctx.close()
+    assert r < 1.1e-8
+    assert abs(out.diff - r) < 1e-3 * r + 1e-13
+
+
+@pytest.mark.parametrize("dims", DIMS)
+def test_cg_stops_at_maxiter(dims):
+    """Every step queued up to maxiter has been taken, and none beyond."""
+    ctx, D, A = operator(dims)
+    b = np.random.default_rng(4).normal(size=D.fsize())
+    xs = []
+    for n in (1, 2):
+        x = np.empty_like(b)
+        with pytest.raises(ii.ConvergenceErr):
+            ii.Solver_CG(1e-300, n, A).solve(x, b)
+        xs.append(x)
+    # the reference's recursion by hand (x0 = b)
+    x, r = b.copy(), b - A.mult(b)
+    p = r.copy()
+    want = []
+    for n in range(2):
+        s = A.mult(p)
+        rr = r @ r
+        alpha = rr / (p @ s)
+        x = x + alpha * p
+        r = r - alpha * s
+        p = r + (r @ r) / rr * p
+        want.append(x.copy())
+    ctx.close()
+    for got, ref in zip(xs, want):
+        assert np.linalg.norm(got - ref) < 1e-12 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dims", DIMS)
+@pytest.mark.parametrize("nshift", [1, 2, 3, 7])
+def test_multishift_true_residuals(dims, nshift):
+    ctx, D, A = operator(dims)
+    b = np.random.default_rng(5).normal(size=D.fsize())
+    shifts = np.geomspace(1e-3, 1.0, nshift)
+    x = [np.empty_like(b) for _ in shifts]
+    so, diff, n = ii.MultiShiftSolver_CG(A, 1e-16, 2000).solve(x, b, shifts)
+    res = [np.linalg.norm(A.mult(v) + s * v - b) / np.linalg.norm(b) for v, s in zip(x, shifts)]
+    ctx.close()
+    # shift 0 stops on its own residual; the others are dropped on |p_i|
+    assert res[0] < 1.1e-8
+    assert abs(so.diff - max(res)) < 1e-3 * max(res) + 1e-13
+    assert max(res) < 1e-6
+
+
+@pytest.mark.parametrize("nshift", [1, 3])
+def test_multishift_full_index(nshift):
+    dims = (6, 4, 2, 10)
+    lat = orc.Lattice(dims)
+    ctx = ii.Context(dims)
+    D = ii.Dirac_Wilson(1.0 / (2 * 0.12) - 4.0, lat.apbc(lat.gauge_expH(0.3, 17)), ctx)
+    A = ii.Fopr_DdagD(D)
+    b = np.random.default_rng(6).normal(size=D.fsize())
+    shifts = np.geomspace(1e-2, 1.0, nshift)
+    x = [np.empty_like(b) for _ in shifts]
+    so, _, _ = ii.MultiShiftSolver_CG(A, 1e-16, 2000).solve(x, b, shifts)
+    res = [np.linalg.norm(A.mult(v) + s * v - b) / np.linalg.norm(b) for v, s in zip(x, shifts)]
+    ctx.close()
+    assert res[0] < 1.1e-8
+    assert abs(so.diff - max(res)) < 1e-3 * max(res) + 1e-13
