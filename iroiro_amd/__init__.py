@@ -392,11 +392,12 @@ class Solver_CG:
         if not isinstance(D, Dirac_Wilson_EvenOdd):
             raise TypeError("Solver_CG on the device supports Fopr_DdagD(Dirac_Wilson_EvenOdd)")
         b = _lib.as_f64(src, D.fsize())
-        x = np.empty(D.fsize())
+        x = _lib.result_f64(sol, D.fsize())
         out = _lib.SolverOutputC()
         st = _lib.load().ii_solver_cg(D.ctx.handle, D.kpp, _lib.dptr(x), _lib.dptr(b), self.prec,
                                       self.MaxIter, ctypes.byref(out))
-        sol[...] = x
+        if x is not sol:
+            sol[...] = x
         D.ctx.check(st, "Solver_CG")
         so = SolverOutput(out)
         so.Msg = "CG solver"
@@ -593,7 +594,7 @@ class RationalSolver_CG:
             raise RuntimeError("[RationalSolver] Rational Approximation not initialized yet")
         D = self._D()
         b = _lib.as_f64(src, D.fsize())
-        x = np.empty(D.fsize())
+        x = _lib.result_f64(sol, D.fsize())
         res = _lib.as_f64(res)
         poles = _lib.as_f64(poles)
         out = _lib.SolverOutputC()
@@ -601,7 +602,8 @@ class RationalSolver_CG:
                                            _lib.dptr(res), _lib.dptr(poles), len(res),
                                            self.MS_Solver_.prec, self.MS_Solver_.MaxIter,
                                            self.precision, ctypes.byref(out))
-        sol[...] = x
+        if x is not sol:
+            sol[...] = x
         if st == _lib.II_ERR_NOT_CONVERGED:
             raise NotConverged(st, "Not converged.")
         D.ctx.check(st, what)
@@ -783,11 +785,12 @@ class Inverter_WilsonLike:
     def invert(self, sol, src):
         D = self.D
         b = _lib.as_f64(src, 24 * D.ctx.V)
-        x = np.empty(24 * D.ctx.V)
+        x = _lib.result_f64(sol, 24 * D.ctx.V)
         out = _lib.SolverOutputC()
         st = _lib.load().ii_eo_invert(D.ctx.handle, D.kpp, _lib.dptr(x), _lib.dptr(b),
                                       self.slv.prec, self.slv.MaxIter, ctypes.byref(out))
-        sol[...] = x
+        if x is not sol:
+            sol[...] = x
         D.ctx.check(st, "Inverter_WilsonLike::invert")
         return SolverOutput(out)
 
@@ -1006,20 +1009,26 @@ class LearnedPreconditioner:
     def loss_grad(self, bs, ys):
         """Loss sum_k |M b_k - y_k|^2/|y_k|^2 and its gradient per layer."""
         nh = 24 * self.ctx.V // 2
-        b = _lib.as_f64(np.concatenate([np.ravel(v) for v in bs]), nh * len(bs))
-        y = _lib.as_f64(np.concatenate([np.ravel(v) for v in ys]), nh * len(ys))
+        bs, ys = [np.ravel(v) for v in bs], [np.ravel(v) for v in ys]
+        if len(bs) != len(ys) or any(v.size != nh for v in bs + ys):
+            bs = _lib.as_f64(np.concatenate(bs), nh * len(bs)).reshape(-1, nh)
+            ys = _lib.as_f64(np.concatenate(ys), nh * len(bs)).reshape(-1, nh)
         sizes = [int(np.prod(self.shape(l))) for l in range(_lib.NET_LAYERS)]
-        f = np.empty(2 * sum(sizes), np.float32)
-        loss = ctypes.c_double()
-        self.ctx.check(self._L().ii_net_loss_grad(self.ctx.handle, len(bs), _lib.dptr(b),
-                                                  _lib.dptr(y), ctypes.byref(loss), _lib.fptr(f)),
-                       "ii_net_loss_grad")
-        c = f.view(np.complex64)
+        total, loss, one = None, 0.0, ctypes.c_double()
+        for b, y in zip(bs, ys):  # one pair a call: no copy that joins them
+            b, y = _lib.as_f64(b), _lib.as_f64(y)
+            f = np.empty(2 * sum(sizes), np.float32)
+            self.ctx.check(self._L().ii_net_loss_grad(self.ctx.handle, 1, _lib.dptr(b),
+                                                      _lib.dptr(y), ctypes.byref(one),
+                                                      _lib.fptr(f)), "ii_net_loss_grad")
+            loss += one.value
+            total = f if total is None else total + f
+        c = total.view(np.complex64)
         grads, off = [], 0
         for l, n in enumerate(sizes):
             grads.append(c[off:off + n].reshape(self.shape(l)))
             off += n
-        return loss.value, grads
+        return loss, grads
 
     def apply(self, r):
         r = _lib.as_f64(r, 24 * self.ctx.V // 2)

@@ -214,6 +214,15 @@ def as_f64(a, n=None):
     return a
 
 
+def result_f64(a, n):
+    """Where a solver writes n doubles for the caller's array `a`: `a` itself
+    if it is such an array in memory, else a new one (to be copied into `a`)."""
+    if (isinstance(a, np.ndarray) and a.dtype == np.float64 and a.size == n and
+            a.flags.c_contiguous and a.flags.writeable):
+        return a
+    return np.empty(n)
+
+
 def check(status, ctx_handle, what):
     if status == II_OK:
         return

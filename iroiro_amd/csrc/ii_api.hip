@@ -92,20 +92,29 @@ ii_status require_gauge(ii_context* ctx) {
 ii_status stage_in(ii_context* ctx, const double* host, size_t n, double** dev) {
   void* p = nullptr;
   II_CHECK(workspace(ctx, 0, n * sizeof(double), &p));
-  II_HIP(ctx, hipMemcpyAsync(p, host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+  II_CHECK(copy_to_device(ctx, p, host, n * sizeof(double)));
   *dev = (double*)p;
   return II_OK;
 }
 ii_status stage_out(ii_context* ctx, double* host, const double* dev, size_t n) {
-  II_HIP(ctx, hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return II_OK;
+  return copy_to_host(ctx, host, dev, n * sizeof(double));
 }
 // A second staging area for outputs (slot 1).
 ii_status stage_buf(ii_context* ctx, size_t n, double** dev) {
   void* p = nullptr;
   II_CHECK(workspace(ctx, 1, n * sizeof(double), &p));
   *dev = (double*)p;
+  return II_OK;
+}
+
+ii_status temp_field(ii_context* ctx, int slot, int subset, int nrhs, ii_field* f) {
+  void* p = nullptr;
+  const size_t n = half_elems(ctx->g) * nrhs * (subset == II_FULL ? 2 : 1);
+  II_CHECK(workspace(ctx, kSlotFields + slot, n * sizeof(double2), &p));
+  f->ctx = ctx;
+  f->subset = subset;
+  f->nrhs = nrhs;
+  f->data = (double2*)p;
   return II_OK;
 }
 
@@ -185,6 +194,7 @@ ii_status ii_context_destroy(ii_context* ctx) {
   if (ctx->scal) (void)hipFree(ctx->scal);
   if (ctx->scal_host) (void)hipHostFree(ctx->scal_host);
   if (ctx->host_pin) (void)hipHostFree(ctx->host_pin);
+  host_pipe_release(ctx);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

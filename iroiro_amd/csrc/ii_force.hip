@@ -258,7 +258,7 @@ static ForcePairs full_pairs(const double2* ee, const double2* eo, const double2
 static ii_status upload_to(ii_context* ctx, int slot, const double* host, size_t n, double** dev) {
   void* p = nullptr;
   II_CHECK(workspace(ctx, slot, n * sizeof(double), &p));
-  II_HIP(ctx, hipMemcpyAsync(p, host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+  II_CHECK(copy_to_device(ctx, p, host, n * sizeof(double)));
   *dev = (double*)p;
   return II_OK;
 }
@@ -268,9 +268,7 @@ static ii_status download_force(ii_context* ctx, const double2* F, double* host)
   void* p = nullptr;
   II_CHECK(workspace(ctx, kWsOut, n * sizeof(double), &p));
   II_CHECK(unpack_gauge_field(ctx, F, (double*)p));
-  II_HIP(ctx, hipMemcpyAsync(host, p, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return II_OK;
+  return copy_to_host(ctx, host, p, n * sizeof(double));
 }
 
 // Two host spinor arrays (half or full) into device fields of slots
@@ -369,10 +367,7 @@ ii_status ii_traceless_antihermite(ii_context* ctx, double* out, const double* i
   hipLaunchKernelGGL(k_traceless_antihermite, dim3(blocks_for(nl)), dim3(kBlock), 0, ctx->stream,
                      d, d, nl);
   II_HIP(ctx, hipGetLastError());
-  II_HIP(ctx, hipMemcpyAsync(out, d, (size_t)18 * nl * sizeof(double), hipMemcpyDeviceToHost,
-                             ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return II_OK;
+  return copy_to_host(ctx, out, d, (size_t)18 * nl * sizeof(double));
 }
 
 ii_status ii_bench_md_force(ii_context* ctx, int nrep, double* force_ms, double* total_ms) {

@@ -92,7 +92,7 @@ struct ii_context {
   int tbc_sign = 1;               // sign of the t-links on the last time slice (r12)
   bool r12_ok = false;
   // workspaces, by slot index (see ii::workspace)
-  static constexpr int kSlots = 96;
+  static constexpr int kSlots = 104;
   ii::Buffer work[kSlots];
   double* partials = nullptr;     // reduction partial sums
   size_t partials_len = 0;
@@ -101,6 +101,7 @@ struct ii_context {
   int nscal = 0;
   void* host_pin = nullptr;       // pinned host block of the multishift scalars
   size_t host_pin_len = 0;
+  void* host_pipe = nullptr;      // pinned slots of the host copies (ii_hostcopy.hip)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // autotuned launch shapes
   ii::HopOrder hop_order;
@@ -156,6 +157,18 @@ ii_status ensure_scalars(ii_context* ctx, int n);
 // Pinned host block of at least `bytes` owned by the context (grows, never
 // shrinks), so solves allocate no pinned memory per call.
 ii_status ensure_host_pin(ii_context* ctx, size_t bytes, void** ptr);
+// Copies between a caller's (pageable) array and the device through pinned
+// slots of the context.  copy_to_device returns when src has been read; the
+// device side is ordered on the context's stream.  copy_to_host follows the
+// stream's work and returns when dst is complete.
+ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t bytes);
+ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes);
+void host_pipe_release(ii_context* ctx);
+// A field of nrhs rhs in workspace slots (kSlotFields ...), for the solvers'
+// inputs and results on host arrays: kept between calls, where a field of its
+// own took an allocation, a clear and a free each.
+constexpr int kSlotFields = 96;
+ii_status temp_field(ii_context* ctx, int slot, int subset, int nrhs, ii_field* f);
 ii_status require_gauge(ii_context* ctx);
 // Entry of every API call on a context: selects its device and clears a
 // stale HIP error left by an earlier, already reported failure.

@@ -1308,8 +1308,7 @@ ii_status ii_net_layer_apply(ii_context* ctx, int layer, int adjoint, const doub
   const size_t nin = (size_t)cin * 24 * g.V, nout = (size_t)cout * 24 * g.V;
   II_CHECK(stage(ctx, N, std::max(nin, nout)));
   // input channels in grad[0] (8-channel capacity), output in grad[1]
-  II_HIP(ctx, hipMemcpyAsync(N->stage, in, nin * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
+  II_CHECK(copy_to_device(ctx, N->stage, in, nin * sizeof(double)));
   hipLaunchKernelGGL(k_net_pack_lex, dim3(blocks_for((long)cin * g.V)), dim3(kBlock), 0,
                      ctx->stream, g, N->stage, N->grad[0], cin);
   II_HIP(ctx, hipGetLastError());
@@ -1317,10 +1316,7 @@ ii_status ii_net_layer_apply(ii_context* ctx, int layer, int adjoint, const doub
   hipLaunchKernelGGL(k_net_unpack_lex, dim3(blocks_for((long)cout * g.V)), dim3(kBlock), 0,
                      ctx->stream, g, N->grad[1], N->stage, cout);
   II_HIP(ctx, hipGetLastError());
-  II_HIP(ctx, hipMemcpyAsync(out, N->stage, nout * sizeof(double), hipMemcpyDeviceToHost,
-                             ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return II_OK;
+  return copy_to_host(ctx, out, N->stage, nout * sizeof(double));
 }
 
 ii_status ii_net_layer_wgrad(ii_context* ctx, int layer, const double* in, const double* grad_out,
@@ -1333,10 +1329,8 @@ ii_status ii_net_layer_wgrad(ii_context* ctx, int layer, const double* in, const
   LayerParams& P = N->L[layer];
   const size_t nin = (size_t)P.cin * 24 * g.V, nout = (size_t)P.cout * 24 * g.V;
   II_CHECK(stage(ctx, N, nin + nout));
-  II_HIP(ctx, hipMemcpyAsync(N->stage, in, nin * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
-  II_HIP(ctx, hipMemcpyAsync(N->stage + nin, grad_out, nout * sizeof(double),
-                             hipMemcpyHostToDevice, ctx->stream));
+  II_CHECK(copy_to_device(ctx, N->stage, in, nin * sizeof(double)));
+  II_CHECK(copy_to_device(ctx, N->stage + nin, grad_out, nout * sizeof(double)));
   hipLaunchKernelGGL(k_net_pack_lex, dim3(blocks_for((long)P.cin * g.V)), dim3(kBlock), 0,
                      ctx->stream, g, N->stage, N->grad[0], P.cin);
   hipLaunchKernelGGL(k_net_pack_lex, dim3(blocks_for((long)P.cout * g.V)), dim3(kBlock), 0,
@@ -1373,10 +1367,8 @@ ii_status ii_net_loss_grad(ii_context* ctx, int npairs, const double* b_even, co
   II_CHECK(zero_grads(ctx, N));
   double L = 0.0;
   for (int k = 0; k < npairs; ++k) {
-    II_HIP(ctx, hipMemcpyAsync(N->stage, b_even + k * nh, nh * sizeof(double),
-                               hipMemcpyHostToDevice, ctx->stream));
-    II_HIP(ctx, hipMemcpyAsync(N->stage + nh, y_even + k * nh, nh * sizeof(double),
-                               hipMemcpyHostToDevice, ctx->stream));
+    II_CHECK(copy_to_device(ctx, N->stage, b_even + k * nh, nh * sizeof(double)));
+    II_CHECK(copy_to_device(ctx, N->stage + nh, y_even + k * nh, nh * sizeof(double)));
     II_CHECK(pack_half_spinor(ctx, N->stage, b64));
     II_CHECK(pack_half_spinor(ctx, N->stage + nh, y64));
     hipLaunchKernelGGL(k_net_to32, dim3(blocks_for(g.Vh)), dim3(kBlock), 0, ctx->stream, g, b64,
@@ -1413,14 +1405,11 @@ ii_status ii_net_apply(ii_context* ctx, const double* r_even, double* z_even) {
   II_CHECK(stage(ctx, N, nh));
   II_CHECK(dev_alloc(ctx, &N->fw[3], he));
   II_CHECK(dev_alloc(ctx, &N->fw[4], he));
-  II_HIP(ctx, hipMemcpyAsync(N->stage, r_even, nh * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
+  II_CHECK(copy_to_device(ctx, N->stage, r_even, nh * sizeof(double)));
   II_CHECK(pack_half_spinor(ctx, N->stage, N->fw[3]));
   II_CHECK(apply_M(ctx, N, N->fw[3], N->fw[4]));
   II_CHECK(unpack_half_spinor(ctx, N->fw[4], N->stage));
-  II_HIP(ctx, hipMemcpyAsync(z_even, N->stage, nh * sizeof(double), hipMemcpyDeviceToHost,
-                             ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  II_CHECK(copy_to_host(ctx, z_even, N->stage, nh * sizeof(double)));
   return II_OK;
 }
 
@@ -1641,8 +1630,7 @@ ii_status ii_fgcr_solve(ii_context* ctx, double kappa, double* x_even, const dou
   II_CHECK(dev_alloc(ctx, &N->fw[3], he));
   II_CHECK(dev_alloc(ctx, &N->fw[4], he));
   double2 *b = N->fw[3], *x = N->fw[4];
-  II_HIP(ctx, hipMemcpyAsync(N->stage, b_even, nh * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
+  II_CHECK(copy_to_device(ctx, N->stage, b_even, nh * sizeof(double)));
   II_CHECK(pack_half_spinor(ctx, N->stage, b));
   II_CHECK(zero64(ctx, x));
   ii_solver_output o{};
@@ -1650,9 +1638,7 @@ ii_status ii_fgcr_solve(ii_context* ctx, double kappa, double* x_even, const dou
   if (out) *out = o;
   II_CHECK(st);
   II_CHECK(unpack_half_spinor(ctx, x, N->stage));
-  II_HIP(ctx, hipMemcpyAsync(x_even, N->stage, nh * sizeof(double), hipMemcpyDeviceToHost,
-                             ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  II_CHECK(copy_to_host(ctx, x_even, N->stage, nh * sizeof(double)));
   if (out) *out = o;
   return II_OK;
 }

@@ -103,13 +103,11 @@ ii_status ii_rational_solve(ii_context* ctx, double kappa, double* sol, const do
   II_CHECK(check_poles(ctx, res, poles, npoles));
   const Geom& g = ctx->g;
   auto t0 = std::chrono::steady_clock::now();
-  ii_field *fb = nullptr, *fx = nullptr, *fs = nullptr;
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fb));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fb};
-  II_CHECK(ii_field_create(ctx, II_EVEN, npoles, &fx));
-  Del d2{fx};
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fs));
-  Del d3{fs};
+  ii_field fb_, fx_, fs_;
+  ii_field *fb = &fb_, *fx = &fx_, *fs = &fs_;
+  II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
+  II_CHECK(temp_field(ctx, 1, II_EVEN, npoles, fx));
+  II_CHECK(temp_field(ctx, 2, II_EVEN, 1, fs));
   II_CHECK(ii_field_upload(fb, 0, src));
   ii_solver_output o{};
   ii_status st = shifted_solutions(ctx, kappa, fx->data, fb->data, poles, npoles, prec, maxiter,
@@ -142,13 +140,11 @@ ii_status ii_action_nf_md_force(ii_context* ctx, double kappa, const double* phi
   II_CHECK(check_poles(ctx, ires, ipoles, npoles));
   const Geom& g = ctx->g;
   const size_t he = half_elems(g);
-  ii_field *fphi = nullptr, *fx = nullptr, *fz = nullptr;
-  II_CHECK(ii_field_create(ctx, II_EVEN, npf, &fphi));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fphi};
-  II_CHECK(ii_field_create(ctx, II_EVEN, npoles, &fx));
-  Del d2{fx};
-  II_CHECK(ii_field_create(ctx, II_EVEN, 2, &fz));  // zeta and an odd temporary
-  Del d3{fz};
+  ii_field fphi_, fx_, fz_;
+  ii_field *fphi = &fphi_, *fx = &fx_, *fz = &fz_;
+  II_CHECK(temp_field(ctx, 0, II_EVEN, npf, fphi));
+  II_CHECK(temp_field(ctx, 1, II_EVEN, npoles, fx));
+  II_CHECK(temp_field(ctx, 2, II_EVEN, 2, fz));  // zeta and an odd temporary
   for (int pf = 0; pf < npf; ++pf) II_CHECK(ii_field_upload(fphi, pf, phi + (size_t)24 * g.Vh * pf));
   // the force accumulates in the device gauge layout
   void* wf = nullptr;
@@ -178,9 +174,7 @@ ii_status ii_action_nf_md_force(ii_context* ctx, double kappa, const double* phi
     }
   }
   II_CHECK(unpack_gauge_field(ctx, F, (double*)wh));
-  II_HIP(ctx, hipMemcpyAsync(force, wh, (size_t)72 * g.V * sizeof(double), hipMemcpyDeviceToHost,
-                             ctx->stream));
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  II_CHECK(copy_to_host(ctx, force, wh, (size_t)72 * g.V * sizeof(double)));
   if (out) *out = o;
   if (worst != II_OK) ctx->err = msg;
   return worst;

@@ -2598,11 +2598,10 @@ ii_status ii_solver_cg(ii_context* ctx, double kappa, double* x, const double* b
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
   const Geom& g = ctx->g;
-  ii_field *fb = nullptr, *fx = nullptr;
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fb));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fb};
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fx));
-  Del d2{fx};
+  ii_field fb_, fx_;
+  ii_field *fb = &fb_, *fx = &fx_;
+  II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
+  II_CHECK(temp_field(ctx, 1, II_EVEN, 1, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
   ii_status st = cg_reference(ctx, kappa, fx->data, fb->data, prec, maxiter, out);
   if (st != II_OK && st != II_ERR_NOT_CONVERGED) return st;
@@ -2620,11 +2619,10 @@ ii_status ii_multishift_cg(ii_context* ctx, double kappa, double* x, const doubl
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
   const Geom& g = ctx->g;
-  ii_field *fb = nullptr, *fx = nullptr;
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fb));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fb};
-  II_CHECK(ii_field_create(ctx, II_EVEN, nshift, &fx));
-  Del d2{fx};
+  ii_field fb_, fx_;
+  ii_field *fb = &fb_, *fx = &fx_;
+  II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
+  II_CHECK(temp_field(ctx, 1, II_EVEN, nshift, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
   ii_status st = multishift_reference(ctx, kappa, fx->data, fb->data, shifts, nshift, prec,
                                       maxiter, out, nullptr, false);
@@ -2644,11 +2642,10 @@ ii_status ii_multishift_mixed(ii_context* ctx, double kappa, double* x, const do
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
   const Geom& g = ctx->g;
-  ii_field *fb = nullptr, *fx = nullptr;
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fb));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fb};
-  II_CHECK(ii_field_create(ctx, II_EVEN, nshift, &fx));
-  Del d2{fx};
+  ii_field fb_, fx_;
+  ii_field *fb = &fb_, *fx = &fx_;
+  II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
+  II_CHECK(temp_field(ctx, 1, II_EVEN, nshift, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
   ii_status st = multishift_mixed_dev(ctx, kappa, fx->data, fb->data, shifts, nshift, tol,
                                       precision, maxiter, out);
@@ -2666,11 +2663,10 @@ ii_status ii_multishift_cg_full(ii_context* ctx, double kappa, double* x, const 
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
   const Geom& g = ctx->g;
-  ii_field *fb = nullptr, *fx = nullptr;
-  II_CHECK(ii_field_create(ctx, II_FULL, 1, &fb));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fb};
-  II_CHECK(ii_field_create(ctx, II_FULL, nshift, &fx));
-  Del d2{fx};
+  ii_field fb_, fx_;
+  ii_field *fb = &fb_, *fx = &fx_;
+  II_CHECK(temp_field(ctx, 0, II_FULL, 1, fb));
+  II_CHECK(temp_field(ctx, 1, II_FULL, nshift, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
   ii_status st = multishift_reference(ctx, kappa, fx->data, fb->data, shifts, nshift, prec,
                                       maxiter, out, nullptr, true);
@@ -2736,15 +2732,12 @@ ii_status ii_eo_invert(ii_context* ctx, double kappa, double* sol, const double*
   II_CHECK(enter(ctx));
   const Geom& g = ctx->g;
   const size_t he = half_elems(g);
-  ii_field *fs = nullptr, *fx = nullptr, *fb = nullptr, *fy = nullptr;
-  II_CHECK(ii_field_create(ctx, II_FULL, 1, &fs));
-  struct Del { ii_field* f; ~Del() { if (f) ii_field_destroy(f); } } d1{fs};
-  II_CHECK(ii_field_create(ctx, II_FULL, 1, &fx));
-  Del d2{fx};
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fb));
-  Del d3{fb};
-  II_CHECK(ii_field_create(ctx, II_EVEN, 1, &fy));
-  Del d4{fy};
+  ii_field fs_, fx_, fb_, fy_;
+  ii_field *fs = &fs_, *fx = &fx_, *fb = &fb_, *fy = &fy_;
+  II_CHECK(temp_field(ctx, 0, II_FULL, 1, fs));
+  II_CHECK(temp_field(ctx, 1, II_FULL, 1, fx));
+  II_CHECK(temp_field(ctx, 2, II_EVEN, 1, fb));
+  II_CHECK(temp_field(ctx, 3, II_EVEN, 1, fy));
   II_CHECK(ii_field_upload(fs, 0, src));
   double2* se = fs->data;
   double2* so = fs->data + he;

@@ -1,0 +1,26 @@
+"""Host arrays through the library's staged copies, byte for byte: below the
+size the runtime copies itself, in one and several pieces of one thread, and in
+the pieces of two threads with a last piece of odd size."""
+import numpy as np
+import pytest
+
+import iroiro_amd as ii
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2, 2), (4, 4, 4, 8), (6, 4, 2, 10), (8, 8, 8, 16),
+                                  (14, 10, 12, 18), (22, 14, 18, 26)])
+def test_field_and_gauge_round_trip(dims):
+    ctx = ii.Context(dims)
+    f = ii.DeviceField(ctx, "full", 2)
+    rng = np.random.default_rng(1)
+    a, b = rng.normal(size=f.size), rng.normal(size=f.size)
+    f.upload(0, a)
+    f.upload(1, b)
+    assert np.array_equal(f.download(1), b)
+    assert np.array_equal(f.download(0), a)
+    u = rng.normal(size=72 * ctx.V)
+    ctx.upload_gauge(u)
+    assert np.array_equal(ctx.download_gauge(), u)
+    ctx.close()
