@@ -26,7 +26,8 @@ namespace ii {
 // 24-term site sums in FP32, the sums over sites in FP64.
 template <int EPI, typename R, typename C, typename SpX, typename StOut>
 __device__ __forceinline__ void hop_epilogue(C o[12], const C* xs, int hs, const SpX& dr,
-                                             const StOut& outr, double alpha, double ds[3]) {
+                                             const StOut& outr, double alpha, double shift,
+                                             const SpX& pr, double ds[3]) {
   constexpr bool kF64 = std::is_same<R, double>::value;
   if constexpr (EPI == kEpiDot) {
     if constexpr (kF64) {
@@ -59,6 +60,15 @@ __device__ __forceinline__ void hop_epilogue(C o[12], const C* xs, int hs, const
   } else if constexpr (EPI == kEpiRUpd) {
     const R sc = (R)dr.scale(hs), al = (R)alpha;
     R sd = R(0);
+    if (shift != 0.0) {
+      const R sh = (R)shift * (R)pr.scale(hs);
+#pragma unroll
+      for (int k = 0; k < 12; ++k) {
+        auto pv = pr.ld(hs, k);
+        o[k].x = fma(sh, (R)pv.x, o[k].x);
+        o[k].y = fma(sh, (R)pv.y, o[k].y);
+      }
+    }
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
       auto dvv = dr.ld(hs, k);
@@ -104,7 +114,7 @@ __global__ void __launch_bounds__(kBlock)
 k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
       typename SpIn::R a, bool tbc_flip, double* __restrict__ partials,
       const int* __restrict__ skip, int skip_stride, HopOrder order,
-      const double* __restrict__ coef, int coef_stride) {
+      const double* __restrict__ coef, int coef_stride, const double* __restrict__ sig, SpX px) {
   using C = typename SpIn::C;
   const int nblk = gridDim.x;
   const int base = hop_block_base(g, order, blockIdx.x, nblk, kBlock);
@@ -137,7 +147,8 @@ k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
       }
     }
     hop_epilogue<EPI, typename SpIn::R>(o, xsv, hs, dv.rhs(rhs), out.rhs(rhs),
-                                        EPI == kEpiRUpd ? coef[rhs * coef_stride] : 0.0, dsum);
+                                        EPI == kEpiRUpd ? coef[rhs * coef_stride] : 0.0,
+                                        EPI == kEpiRUpd && sig ? sig[rhs] : 0.0, px.rhs(rhs), dsum);
   }
   constexpr int NS = epi_sums(EPI);
   const size_t plane = (size_t)gridDim.y * nblk;
@@ -207,7 +218,7 @@ __global__ void __launch_bounds__(256)
 k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
             typename SpIn::R a, bool tbc_flip, double* __restrict__ partials,
             const int* __restrict__ skip, HopOrder order, const double* __restrict__ coef,
-            RUpdFold ru) {
+            RUpdFold ru, const double* __restrict__ sig, SpX sp) {
   using C = typename SpIn::C;
   using R = typename SpIn::R;
   __shared__ C part[4][12][64];  // [dimension][3 spin + colour][site]
@@ -258,7 +269,6 @@ k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
   }
   __syncthreads();
   double alpha = 0.0, shift = 0.0;
-  SpX sp = dv;
   if constexpr (EPI == kEpiRUpd) {
     if (ru.den) {
       double d = dsh[0] + dsh[1] + dsh[2] + dsh[3];
@@ -271,6 +281,7 @@ k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
       if (blockIdx.x == 0 && threadIdx.x == 0) *ru.alpha = alpha;
     } else {
       alpha = coef[0];
+      if (sig) shift = sig[0];
     }
   }
   double dsum[3] = {0.0, 0.0, 0.0};
@@ -316,7 +327,8 @@ __global__ void __launch_bounds__(MAXT)
 k_hop_mrhs(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
            typename SpIn::R a, bool tbc_flip, double* __restrict__ partials,
            const int* __restrict__ skip, int skip_stride, int nrhs, HopOrder order,
-           const double* __restrict__ coef, int coef_stride) {
+           const double* __restrict__ coef, int coef_stride, const double* __restrict__ sig,
+           SpX px) {
   using C = typename SpIn::C;
   using UC = typename Gauge::C;
   // FP16 fields and links: colour products with v_dot2_f32_f16 on links
@@ -444,7 +456,8 @@ k_hop_mrhs(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
       }
     }
     hop_epilogue<EPI, typename SpIn::R>(o, xsv, hs, dv.rhs(rhs), out.rhs(rhs),
-                                        EPI == kEpiRUpd ? coef[rhs * coef_stride] : 0.0, dsum);
+                                        EPI == kEpiRUpd ? coef[rhs * coef_stride] : 0.0,
+                                        EPI == kEpiRUpd && sig ? sig[rhs] : 0.0, px.rhs(rhs), dsum);
   }
   constexpr int NS = epi_sums(EPI);
   const size_t plane = (size_t)nrhs * ntile;
@@ -490,6 +503,12 @@ ii_status launch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, const 
                      const SpX& x, const SpX& dv, typename SpIn::R a, const HopSpec& h) {
   const Geom& g = ctx->g;
   bool flip = ctx->tbc_sign < 0;
+  SpX px = dv;  // the shift term's field
+  if (h.sig) {
+    px.p = (decltype(px.p))h.p;
+    if constexpr (SpIn::kScaled) px.nrm = h.p_nrm;
+    if constexpr (std::is_same<SpX, SpF64>::value) px.rs = 0;
+  }
   if (h.nrhs == 1) {
     constexpr int bs = SpIn::kScaled ? kBlock : 64;  // sites per block
     const HopOrder o = ctx->hop_order.mode == 1 ? strip_order(g, ctx->hop_order.W, bs) : HopOrder();
@@ -497,11 +516,12 @@ ii_status launch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, const 
     if constexpr (SpIn::kScaled)
       hipLaunchKernelGGL((k_hop<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX>), grid,
                          dim3(kBlock), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a,
-                         flip, h.partials, h.skip, h.skip_stride, o, h.coef, h.coef_stride);
+                         flip, h.partials, h.skip, h.skip_stride, o, h.coef, h.coef_stride, h.sig,
+                         px);
     else
       hipLaunchKernelGGL((k_hop_split<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX>), grid,
                          dim3(kBlock), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par, a,
-                         flip, h.partials, h.skip, o, h.coef, h.ru);
+                         flip, h.partials, h.skip, o, h.coef, h.ru, h.sig, px);
   } else if constexpr (GaugePrec<Gauge>::value < 0) {
     return set_error(ctx, II_ERR_STATE, "this gauge form serves single-rhs hops only");
   } else {
@@ -516,7 +536,7 @@ ii_status launch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, const 
     hipLaunchKernelGGL((k_hop_mrhs<G5IN, G5OUT, XPAY, EPI, SpIn, Gauge, StOut, SpX, TS, MAXT>),
                        grid, dim3(TS, rb), 0, ctx->stream, g, in, gauge, out, x, dv, h.out_par,
                        a, flip, h.partials, h.skip, h.skip_stride, h.nrhs, ord, h.coef,
-                       h.coef_stride);
+                       h.coef_stride, h.sig, px);
   }
   II_HIP(ctx, hipGetLastError());
   return II_OK;
@@ -535,6 +555,8 @@ ii_status dispatch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, cons
       (h.nrhs != 1 || SpIn::kScaled || h.ru.nden > kMaxFold || !h.ru.num || !h.ru.alpha ||
        (h.ru.shift != 0.0 && (!h.ru.p || !h.ru.den2))))
     return set_error(ctx, II_ERR_BAD_ARG, "bad folded residual update");
+  if (h.sig && (h.epi != kEpiRUpd || h.ru.den || !h.p || (SpIn::kScaled && !h.p_nrm)))
+    return set_error(ctx, II_ERR_BAD_ARG, "bad shift term of a residual update");
   if (h.epi == kEpiRUpd && !h.coef && !h.ru.den)
     return set_error(ctx, II_ERR_BAD_ARG, "residual-update hop without its scalars");
   const int sel = (h.g5in ? 32 : 0) | (h.g5out ? 16 : 0) | (h.xpay ? 8 : 0) | h.epi;
@@ -759,7 +781,7 @@ ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* o
   SpF64 sin{in, g.stride, rs};
   StF64 so{out, g.stride};
   SpF64 sx{x ? x : in, g.stride, rs};
-  SpF64 sd{dv ? dv : in, g.stride, rs};
+  SpF64 sd{dv ? dv : in, g.stride, h.dv_shared ? -1 : rs};
   const unsigned long long gb = (unsigned long long)72 * g.stride * sizeof(double2);
   if (h.nrhs == 1 && links_cached(gb))
     return dispatch_hop(ctx, sin, GaugeF64Flat<0>{ctx->gauge64, g.stride}, so, sx, sd, h);

@@ -54,6 +54,13 @@ struct HopSpec {
   const double* coef = nullptr;  // kEpiRUpd: alpha of rhs r at coef[r * coef_stride]
   int coef_stride = 0;
   RUpdFold ru;                   // kEpiRUpd, single rhs: used when ru.den is set
+  // kEpiRUpd: r = dv - alpha (o + sig[rhs] p), sig one device value per rhs
+  // (null: no shift), p a field in the hop's precision like dv (16-bit: p_nrm
+  // its norms)
+  const double* sig = nullptr;
+  const void* p = nullptr;
+  const float* p_nrm = nullptr;
+  bool dv_shared = false;        // FP64: one dv for every rhs
   int nrhs = 1;
   double* partials = nullptr;
   // optional per-rhs skip flags: rhs r is skipped when skip[r * skip_stride] != 0

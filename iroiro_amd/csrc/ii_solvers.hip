@@ -56,8 +56,11 @@ constexpr int kFinThreads = 1024;
 // pap -> alpha = rr/pap; with ahist, alpha is also kept at
 // ahist[rhs * astride + aidx] (0 for a finished rhs) for the deferred
 // solution update
+// (sig: pap += sig[rhs] |p|^2, from the npp partial sums per rhs at pp)
 __global__ void k_fin_pap(const double* __restrict__ partials, int nb, RUScal* __restrict__ sc,
-                          double* __restrict__ ahist, int aidx, int astride) {
+                          double* __restrict__ ahist, int aidx, int astride,
+                          const double* __restrict__ sig = nullptr,
+                          const double* __restrict__ pp = nullptr, int npp = 0) {
   RUScal& S = sc[blockIdx.x];
   double* ah = ahist ? ahist + (size_t)blockIdx.x * astride + aidx : nullptr;
   if (S.done) {
@@ -67,6 +70,11 @@ __global__ void k_fin_pap(const double* __restrict__ partials, int nb, RUScal* _
   const double* p = partials + (size_t)blockIdx.x * nb;
   double s = 0.0;
   for (int i = threadIdx.x; i < nb; i += blockDim.x) s += p[i];
+  if (sig) {
+    double t = 0.0;
+    for (int i = threadIdx.x; i < npp; i += blockDim.x) t += pp[(size_t)blockIdx.x * npp + i];
+    s = fma(sig[blockIdx.x], t, s);
+  }
   s = block_sum(s);
   if (threadIdx.x == 0) {
     S.pap = s;
@@ -188,22 +196,35 @@ k_cg_xr(Geom g, SpP p, SpS s, SpR rr_, StR rw, SpY yr, StY yw, RUScal* __restric
   if (threadIdx.x == 0) partials[(size_t)rhs * gridDim.x + blockIdx.x] = acc;
 }
 
-// p = r + beta p        (solver_CG.cpp:152-153: p = p*cr + r)
-template <typename SpR, typename SpP, typename StP>
+// p = r + beta p        (solver_CG.cpp:152-153: p = p*cr + r); NORM: partial
+// sums of |p|^2
+template <bool NORM, typename SpR, typename SpP, typename StP>
 __global__ void __launch_bounds__(kBlock)
-k_cg_p(Geom g, SpR r, SpP pr, StP pw, const RUScal* __restrict__ sc) {
+k_cg_p(Geom g, SpR r, SpP pr, StP pw, const RUScal* __restrict__ sc,
+       double* __restrict__ partials) {
   const int rhs = blockIdx.y;
   const RUScal& S = sc[rhs];
   if (S.done) return;
   const double b = S.beta;
   const int hs = blockIdx.x * blockDim.x + threadIdx.x;
-  if (hs >= g.Vh) return;
-  double rv[24], pv[24];
-  ld_site(r.rhs(rhs), hs, rv);
-  ld_site(pr.rhs(rhs), hs, pv);
+  if (!NORM && hs >= g.Vh) return;
+  double acc = 0.0;
+  if (hs < g.Vh) {
+    double rv[24], pv[24];
+    ld_site(r.rhs(rhs), hs, rv);
+    ld_site(pr.rhs(rhs), hs, pv);
 #pragma unroll
-  for (int k = 0; k < 24; ++k) pv[k] = fma(pv[k], b, rv[k]);
-  st_site(pw.rhs(rhs), hs, pv);
+    for (int k = 0; k < 24; ++k) pv[k] = fma(pv[k], b, rv[k]);
+    if (NORM) {
+#pragma unroll
+      for (int k = 0; k < 24; ++k) acc = fma(pv[k], pv[k], acc);
+    }
+    st_site(pw.rhs(rhs), hs, pv);
+  }
+  if (NORM) {
+    acc = block_sum(acc);
+    if (threadIdx.x == 0) partials[(size_t)rhs * gridDim.x + blockIdx.x] = acc;
+  }
 }
 
 // Deferred solution update y += sum_j alpha_j p_j over up to kDefer stored
@@ -268,31 +289,6 @@ k_convert(Geom g, SpA a, StB b, const int* __restrict__ skip, int skip_stride) {
   double v[24];
   ld_site(a.rhs(rhs), hs, v);
   st_site(b.rhs(rhs), hs, v);
-}
-
-// y64 += ys ; ys = 0  (reliable update accumulation), masked
-template <typename SpY, typename StY>
-__global__ void __launch_bounds__(kBlock)
-k_accum(Geom g, SpY ys, StY yz, double2* __restrict__ y64, const int* __restrict__ skip,
-        int skip_stride) {
-  const int rhs = blockIdx.y;
-  if (skip && skip[rhs * skip_stride]) return;
-  const int hs = blockIdx.x * blockDim.x + threadIdx.x;
-  if (hs >= g.Vh) return;
-  double v[24];
-  ld_site(ys.rhs(rhs), hs, v);
-  double2* y = y64 + (size_t)rhs * 12 * g.stride;
-#pragma unroll
-  for (int k = 0; k < 12; ++k) {
-    double2 o = y[(size_t)k * g.stride + hs];
-    o.x += v[2 * k];
-    o.y += v[2 * k + 1];
-    y[(size_t)k * g.stride + hs] = o;
-  }
-  double z[24];
-#pragma unroll
-  for (int k = 0; k < 24; ++k) z[k] = 0.0;
-  st_site(yz.rhs(rhs), hs, z);
 }
 
 // masked |a|^2 partials (FP64)
@@ -436,12 +432,14 @@ ii_status ddagdP(ii_context* ctx, int P, double kappa, const SF& f, const SF& ou
 //   alpha = rr / |q|^2                                   (k_fin_pap; ahist)
 //   r -= alpha Dhat^dag q, with partial sums of |r|^2   (fourth hop, kEpiRUpd)
 // A p itself is never stored; the k_fin_rr that follows reads the |r|^2
-// partials (hop_dot_parts per rhs).
+// partials (hop_dot_parts per rhs).  With sig (one shift per rhs) the operator
+// is A + sig: <p, (A + sig) p> = |q|^2 + sig |p|^2 (pnorm: hop_blocks partial
+// sums of |p|^2 per rhs) and r -= alpha (Dhat^dag q + sig p).
 static_assert(sizeof(RUScal) % sizeof(double) == 0, "RUScal is read as a double array");
 ii_status ddagd_cg_fused(ii_context* ctx, int P, double kappa, const SF& p, const SF& r,
                          const SF& q, const SF& t, RUScal* sc, double* partials, int nrhs,
                          const int* skip, int skip_stride, double* ahist, int aidx,
-                         int astride) {
+                         int astride, const double* sig = nullptr, const double* pnorm = nullptr) {
   HopSpec h;
   h.nrhs = nrhs;
   h.skip = skip;
@@ -456,7 +454,8 @@ ii_status ddagd_cg_fused(ii_context* ctx, int P, double kappa, const SF& p, cons
   h.partials = partials;
   II_CHECK(hopP(ctx, P, h, t, q, &p, nullptr));  // q = Dhat p, |q|^2
   hipLaunchKernelGGL(k_fin_pap, dim3(nrhs), dim3(kFinThreads), 0, ctx->stream, partials,
-                     hop_dot_parts(ctx->g, nrhs, P), sc, ahist, aidx, astride);
+                     hop_dot_parts(ctx->g, nrhs, P), sc, ahist, aidx, astride, sig, pnorm,
+                     hop_blocks(ctx->g));
   h.out_par = 1;
   h.a = 1.0;
   h.xpay = false;
@@ -471,43 +470,37 @@ ii_status ddagd_cg_fused(ii_context* ctx, int P, double kappa, const SF& p, cons
   h.epi = kEpiRUpd;
   h.coef = &sc[0].alpha;
   h.coef_stride = (int)(sizeof(RUScal) / sizeof(double));
+  h.sig = sig;
+  h.p = p.v;
+  h.p_nrm = p.nrm;
   return hopP(ctx, P, h, t, r, &q, &r);  // r -= alpha Dhat^dag q, |r|^2
 }
 
-template <int P>
-ii_status cg_step_blas(ii_context* ctx, const SF& p, const SF& s, const SF& r, const SF& y,
-                       int ytype, RUScal* sc, int nrhs, double* partials, int nb) {
+// y += alpha p; r -= alpha s; |r|^2 partials, FP64
+ii_status cg_blas64(ii_context* ctx, const SF& p, const SF& s, const SF& r, const SF& y,
+                    RUScal* sc, int nrhs, double* partials, int nb) {
   const Geom& g = ctx->g;
-  using A = Acc<P>;
-  dim3 grid(nb, nrhs);
-  if (ytype == II_PREC_DOUBLE) {
-    hipLaunchKernelGGL((k_cg_xr<typename A::Sp, typename A::Sp, typename A::Sp, typename A::St,
-                                SpF64, StF64>),
-                       grid, dim3(kBlock), 0, ctx->stream, g, A::sp(p, g.stride),
-                       A::sp(s, g.stride), A::sp(r, g.stride), A::st(r, g.stride),
-                       Acc<II_PREC_DOUBLE>::sp(y, g.stride), Acc<II_PREC_DOUBLE>::st(y, g.stride),
-                       sc, partials);
-  } else {
-    hipLaunchKernelGGL((k_cg_xr<typename A::Sp, typename A::Sp, typename A::Sp, typename A::St,
-                                SpF32, StF32>),
-                       grid, dim3(kBlock), 0, ctx->stream, g, A::sp(p, g.stride),
-                       A::sp(s, g.stride), A::sp(r, g.stride), A::st(r, g.stride),
-                       Acc<II_PREC_SINGLE>::sp(y, g.stride), Acc<II_PREC_SINGLE>::st(y, g.stride),
-                       sc, partials);
-  }
+  using A = Acc<0>;
+  hipLaunchKernelGGL((k_cg_xr<SpF64, SpF64, SpF64, StF64, SpF64, StF64>), dim3(nb, nrhs),
+                     dim3(kBlock), 0, ctx->stream, g, A::sp(p, g.stride), A::sp(s, g.stride),
+                     A::sp(r, g.stride), A::st(r, g.stride), A::sp(y, g.stride),
+                     A::st(y, g.stride), sc, partials);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
 }
-
-// p_out = r + beta p_in (p_out may be p_in)
 template <int P>
 ii_status cg_p_update(ii_context* ctx, const SF& r, const SF& p, const SF& pout, RUScal* sc,
-                      int nrhs) {
+                      int nrhs, double* pnorm) {
   const Geom& g = ctx->g;
   using A = Acc<P>;
-  hipLaunchKernelGGL((k_cg_p<typename A::Sp, typename A::Sp, typename A::St>),
-                     dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g,
-                     A::sp(r, g.stride), A::sp(p, g.stride), A::st(pout, g.stride), sc);
+  if (pnorm)
+    hipLaunchKernelGGL((k_cg_p<true, typename A::Sp, typename A::Sp, typename A::St>),
+                       dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g,
+                       A::sp(r, g.stride), A::sp(p, g.stride), A::st(pout, g.stride), sc, pnorm);
+  else
+    hipLaunchKernelGGL((k_cg_p<false, typename A::Sp, typename A::Sp, typename A::St>),
+                       dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g,
+                       A::sp(r, g.stride), A::sp(p, g.stride), A::st(pout, g.stride), sc, pnorm);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
 }
@@ -575,22 +568,14 @@ ii_status norm2P(ii_context* ctx, int P, const SF& a, int nrhs, const int* skip,
   }
 }
 
-ii_status cg_blas_P(ii_context* ctx, int P, const SF& p, const SF& s, const SF& r, const SF& y,
-                    int ytype, RUScal* sc, int nrhs, double* partials, int nb) {
-  switch (P) {
-    case 0: return cg_step_blas<0>(ctx, p, s, r, y, ytype, sc, nrhs, partials, nb);
-    case 1: return cg_step_blas<1>(ctx, p, s, r, y, ytype, sc, nrhs, partials, nb);
-    case 2: return cg_step_blas<2>(ctx, p, s, r, y, ytype, sc, nrhs, partials, nb);
-    default: return cg_step_blas<3>(ctx, p, s, r, y, ytype, sc, nrhs, partials, nb);
-  }
-}
 ii_status cg_p_P(ii_context* ctx, int P, const SF& r, const SF& p, const SF& pout, RUScal* sc,
-                 int nrhs) {
+                 int nrhs,
+                 double* pnorm = nullptr) {
   switch (P) {
-    case 0: return cg_p_update<0>(ctx, r, p, pout, sc, nrhs);
-    case 1: return cg_p_update<1>(ctx, r, p, pout, sc, nrhs);
-    case 2: return cg_p_update<2>(ctx, r, p, pout, sc, nrhs);
-    default: return cg_p_update<3>(ctx, r, p, pout, sc, nrhs);
+    case 0: return cg_p_update<0>(ctx, r, p, pout, sc, nrhs, pnorm);
+    case 1: return cg_p_update<1>(ctx, r, p, pout, sc, nrhs, pnorm);
+    case 2: return cg_p_update<2>(ctx, r, p, pout, sc, nrhs, pnorm);
+    default: return cg_p_update<3>(ctx, r, p, pout, sc, nrhs, pnorm);
   }
 }
 ii_status cg_flush_P(ii_context* ctx, int P, const SF* ring, const int* slots, int n,
@@ -1315,11 +1300,10 @@ ii_status multishift_reference(ii_context* ctx, double kappa, double2* x, const 
 // reliable-update CG (inner precision P, FP64 true residuals) until
 // |b - (A + sigma_i) x_i| <= tol |b|.
 
-// s += sigma_r p ; partial <p, s>   (per rhs shift of the batched CG)
-template <typename SpP, typename SpS, typename StS>
+// s += sigma_r p ; partial <p, s>   (per rhs shift of the batched FP64 CG)
 __global__ void __launch_bounds__(kBlock)
-k_sp_shift(Geom g, SpP p, SpS s, StS sw, const double* __restrict__ sig, RUScal* __restrict__ sc,
-           double* __restrict__ partials) {
+k_sp_shift(Geom g, SpF64 p, SpF64 s, StF64 sw, const double* __restrict__ sig,
+           RUScal* __restrict__ sc, double* __restrict__ partials) {
   const int rhs = blockIdx.y;
   if (sc[rhs].done) return;
   const double sg = sig[rhs];
@@ -1339,53 +1323,15 @@ k_sp_shift(Geom g, SpP p, SpS s, StS sw, const double* __restrict__ sig, RUScal*
   acc = block_sum(acc);
   if (threadIdx.x == 0) partials[(size_t)rhs * gridDim.x + blockIdx.x] = acc;
 }
-
-// rho = b - q - sigma_r y ; partial |rho|^2, masked (FP64; one b for all rhs)
-__global__ void __launch_bounds__(kBlock)
-k_resid_shift(Geom g, const double2* __restrict__ b, const double2* __restrict__ q,
-              const double2* __restrict__ y, const double* __restrict__ sig,
-              double2* __restrict__ rho, const int* __restrict__ skip, int skip_stride,
-              double* __restrict__ partials) {
-  const int rhs = blockIdx.y;
-  if (skip && skip[rhs * skip_stride]) return;
-  const double sg = sig[rhs];
-  const int hs = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0.0;
-  if (hs < g.Vh) {
-    const size_t off = (size_t)rhs * 12 * g.stride + hs;
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-      const size_t i = (size_t)k * g.stride;
-      const double2 bv = b[i + hs], qv = q[off + i], yv = y[off + i];
-      const double2 d = make_double2(bv.x - qv.x - sg * yv.x, bv.y - qv.y - sg * yv.y);
-      rho[off + i] = d;
-      acc = fma(d.x, d.x, fma(d.y, d.y, acc));
-    }
-  }
-  acc = block_sum(acc);
-  if (threadIdx.x == 0) partials[(size_t)rhs * gridDim.x + blockIdx.x] = acc;
-}
-
-template <int P>
-ii_status sp_shift_t(ii_context* ctx, const SF& p, const SF& s, const double* sig, RUScal* sc,
+ii_status sp_shift64(ii_context* ctx, const SF& p, const SF& s, const double* sig, RUScal* sc,
                      int nrhs, double* partials) {
   const Geom& g = ctx->g;
-  using A = Acc<P>;
-  hipLaunchKernelGGL((k_sp_shift<typename A::Sp, typename A::Sp, typename A::St>),
-                     dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g,
+  using A = Acc<0>;
+  hipLaunchKernelGGL(k_sp_shift, dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g,
                      A::sp(p, g.stride), A::sp(s, g.stride), A::st(s, g.stride), sig, sc,
                      partials);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
-}
-ii_status sp_shift_P(ii_context* ctx, int P, const SF& p, const SF& s, const double* sig,
-                     RUScal* sc, int nrhs, double* partials) {
-  switch (P) {
-    case 0: return sp_shift_t<0>(ctx, p, s, sig, sc, nrhs, partials);
-    case 1: return sp_shift_t<1>(ctx, p, s, sig, sc, nrhs, partials);
-    case 2: return sp_shift_t<2>(ctx, p, s, sig, sc, nrhs, partials);
-    default: return sp_shift_t<3>(ctx, p, s, sig, sc, nrhs, partials);
-  }
 }
 
 // Stage 1 (FP32 vectors): x32 receives nshift FP32 half fields.
@@ -1415,19 +1361,23 @@ ii_status multishift_sloppy(ii_context* ctx, double kappa, float2* x32, const do
 }
 
 // Stage 2: batched reliable-update CG on (A + sigma_r) x_r = b for all r,
-// starting from x64 (in/out, nrhs FP64 half fields).
+// starting from x64 (in/out, nrhs FP64 half fields).  The sloppy precisions
+// take the propagator's fused steps with the shift in their scalars and
+// epilogues (ddagd_cg_fused), its deferred solution update and its joined
+// reliable updates; the FP64 residual of an update is its last hop's epilogue.
 ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, int nrhs,
                          const double2* b64, double2* x64, double tol, int P, int maxiter,
                          ii_solver_output* outs) {
   const Geom& g = ctx->g;
   if (P != II_PREC_DOUBLE && !ctx->gauge_lp[P]) II_CHECK(build_lowprec_gauge(ctx, P));
   const bool lo = P != II_PREC_DOUBLE;
-  const int ytype = lo ? II_PREC_SINGLE : II_PREC_DOUBLE;
   const double delta = lo ? 0.1 : 0.0;
-  const int nb = hop_blocks(g);
-  II_CHECK(ensure_partials(ctx, (size_t)std::max(nb, hop_dot_parts(g, nrhs, P)) * nrhs + 16));
+  const int nb = hop_blocks(g), nh = hop_dot_parts(g, nrhs, P);
+  const int nhd = hop_dot_parts(g, nrhs, II_PREC_DOUBLE);
+  const size_t np = (size_t)std::max(std::max(nb, nh), nhd) * nrhs;
+  II_CHECK(ensure_partials(ctx, 2 * np + 16));
   II_CHECK(ensure_ru_scalars(ctx, nrhs));
-  double* part = ctx->partials;
+  double *part = ctx->partials, *pnorm = part + np;  // pnorm: |p|^2 of the current directions
   RUScal* sc = dev_scal(ctx);
   const int ss = kScalInts;
   const int* skip_it = &sc[0].done;
@@ -1437,22 +1387,25 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   double* sig = (double*)auxp;
   double* rr0 = sig + nrhs;
   double* bb = rr0 + nrhs;
-  II_HIP(ctx, hipMemcpyAsync(sig, shifts, nrhs * sizeof(double), hipMemcpyHostToDevice,
-                             ctx->stream));
-  SF q64, t64, u64, rho, ps, rs, ss_, qs, ts, ys;
-  II_CHECK(fieldP(ctx, 38, 0, nrhs, &q64));  // (A) y
-  II_CHECK(fieldP(ctx, 39, 0, nrhs, &t64));  // Dhat y, intermediate
+  double* one = bb + nrhs;  // the device scalar 1.0 (alpha of rho = b - (A + sigma) x)
+  SF t64, u64, rho, ps, rs, ss_, qs, ts, ys;
+  II_CHECK(fieldP(ctx, 39, 0, nrhs, &t64));  // Dhat x, intermediate
   II_CHECK(fieldP(ctx, 41, 0, nrhs, &u64));  // odd temporary
   II_CHECK(fieldP(ctx, 40, 0, nrhs, &rho));
+  const int nring = lo ? kDefer + 1 : 1;
+  std::vector<SF> ring(nring);
+  double* ahist = nullptr;
   if (lo) {
-    II_CHECK(fieldP(ctx, 50, P, nrhs, &ps));
+    for (int i = 0; i < nring; ++i) II_CHECK(fieldP(ctx, i ? 63 + i : 50, P, nrhs, &ring[i]));
     II_CHECK(fieldP(ctx, 51, P, nrhs, &rs));
-    II_CHECK(fieldP(ctx, 52, P, nrhs, &ss_));
     II_CHECK(fieldP(ctx, 53, P, nrhs, &qs));
     II_CHECK(fieldP(ctx, 54, P, nrhs, &ts));
     II_CHECK(fieldP(ctx, 55, II_PREC_SINGLE, nrhs, &ys));
+    void* v = nullptr;
+    II_CHECK(workspace(ctx, 62, sizeof(double) * nring * nrhs, &v));
+    ahist = (double*)v;
   } else {
-    II_CHECK(fieldP(ctx, 50, 0, nrhs, &ps));
+    II_CHECK(fieldP(ctx, 50, 0, nrhs, &ring[0]));
     rs = rho;
     II_CHECK(fieldP(ctx, 52, 0, nrhs, &ss_));
     qs = t64;
@@ -1460,44 +1413,100 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
     ys = SF{x64};
   }
   auto t0 = std::chrono::steady_clock::now();
-  // initial true residual rho = b - (A + sigma) x and |b|^2
-  II_CHECK(ddagdP(ctx, 0, kappa, SF{x64}, q64, t64, u64, nullptr, nullptr, nrhs, nullptr, 0));
-  hipLaunchKernelGGL(k_resid_shift, dim3(nb, nrhs), dim3(kBlock), 0, ctx->stream, g, b64,
-                     (const double2*)q64.v, (const double2*)x64, sig, (double2*)rho.v, nullptr,
-                     0, part);
-  II_HIP(ctx, hipGetLastError());
-  II_CHECK(finalize_sums(ctx, part, nb, rr0, nrhs));
+  // rho = b - (A + sigma) x with the partial sums of |rho|^2, for the rhs not
+  // masked by skip
+  auto residual = [&](const int* skip, int stride) -> ii_status {
+    HopSpec h;
+    h.nrhs = nrhs;
+    h.skip = skip;
+    h.skip_stride = stride;
+    h.out_par = 1;
+    II_CHECK(hopP(ctx, 0, h, SF{x64}, u64, nullptr, nullptr));
+    h.out_par = 0;
+    h.a = -kappa * kappa;
+    h.xpay = true;
+    const SF xf{x64};
+    II_CHECK(hopP(ctx, 0, h, u64, t64, &xf, nullptr));  // Dhat x
+    h.out_par = 1;
+    h.a = 1.0;
+    h.xpay = false;
+    h.g5in = true;
+    II_CHECK(hopP(ctx, 0, h, t64, u64, nullptr, nullptr));
+    h.out_par = 0;
+    h.a = -kappa * kappa;
+    h.xpay = true;
+    h.g5in = false;
+    h.g5out = true;
+    h.epi = kEpiRUpd;
+    h.coef = one;
+    h.sig = sig;
+    h.p = x64;
+    h.dv_shared = true;
+    h.partials = part;
+    const SF bf{const_cast<double2*>(b64)};
+    return hopP(ctx, 0, h, u64, rho, &t64, &bf);
+  };
+  // |b|^2 of every rhs, the shifts and the constant
   {
-    double h = 0.0;
+    std::vector<double> hb(3 * nrhs + 1, 1.0);
     II_CHECK(dot64(ctx, b64, b64, bb));
-    II_HIP(ctx, hipMemcpyAsync(&h, bb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    II_HIP(ctx, hipMemcpyAsync(&hb[0], bb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    std::vector<double> hb(nrhs, h);
-    II_HIP(ctx, hipMemcpyAsync(bb, hb.data(), nrhs * sizeof(double), hipMemcpyHostToDevice,
+    const double h = hb[0];
+    for (int k = 0; k < nrhs; ++k) {
+      hb[k] = shifts[k];
+      hb[nrhs + k] = 0.0;
+      hb[2 * nrhs + k] = h;
+    }
+    II_HIP(ctx, hipMemcpyAsync(sig, hb.data(), hb.size() * sizeof(double), hipMemcpyHostToDevice,
                                ctx->stream));
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
   }
+  II_CHECK(residual(nullptr, 0));
+  II_CHECK(finalize_sums(ctx, part, nhd, rr0, nrhs));
   hipLaunchKernelGGL(k_scal_init, dim3(nrhs), dim3(64), 0, ctx->stream, sc, rr0, bb, 0.0, tol,
                      delta, 1);
   II_HIP(ctx, hipGetLastError());
+  int pos = 0;            // ring slot of the current search directions
+  std::vector<int> pend;  // ring slots whose alpha p is not yet in ys
+  auto flush = [&](bool fold, const int* skip) -> ii_status {
+    if (!fold && pend.empty()) return II_OK;
+    II_CHECK(cg_flush_P(ctx, P, ring.data(), pend.data(), (int)pend.size(), ahist, nring, ys, nrhs,
+                        fold ? x64 : nullptr, skip, ss));
+    pend.clear();
+    return II_OK;
+  };
   if (lo) {
     II_CHECK(convertP(ctx, 0, P, rho, rs, nrhs));
-    II_CHECK(convertP(ctx, 0, P, rho, ps, nrhs));
+    II_CHECK(convertP(ctx, 0, P, rho, ring[0], nrhs));
+    II_CHECK(norm2P(ctx, P, ring[0], nrhs, nullptr, 0, pnorm));
     II_HIP(ctx, hipMemsetAsync(ys.v, 0, field_bytes(g, II_PREC_SINGLE) * nrhs, ctx->stream));
   } else {
-    II_CHECK(copy64(ctx, (double2*)ps.v, (double2*)rho.v, nrhs));
+    II_CHECK(copy64(ctx, (double2*)ring[0].v, (double2*)rho.v, nrhs));
   }
   int its = 0, chunk = 1;
   bool all_done = false;
   while (its < maxiter && !all_done) {
     for (int i = 0; i < chunk; ++i) {
-      II_CHECK(ddagdP(ctx, P, kappa, ps, ss_, qs, ts, nullptr, nullptr, nrhs, skip_it, ss));
-      II_CHECK(sp_shift_P(ctx, P, ps, ss_, sig, sc, nrhs, part));
-      hipLaunchKernelGGL(k_fin_pap, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc,
-                         nullptr, 0, 0);
-      II_CHECK(cg_blas_P(ctx, P, ps, ss_, rs, ys, ytype, sc, nrhs, part, nb));
-      hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc, 1);
-      II_CHECK(cg_p_P(ctx, P, rs, ps, ps, sc, nrhs));
+      const SF& p = ring[pos];
+      if (lo) {
+        II_CHECK(ddagd_cg_fused(ctx, P, kappa, p, rs, qs, ts, sc, part, nrhs, skip_it, ss, ahist,
+                                pos, nring, sig, pnorm));
+        hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kFinThreads), 0, ctx->stream, part, nh, sc,
+                           1);
+        pend.push_back(pos);
+        pos = (pos + 1) % nring;
+        II_CHECK(cg_p_P(ctx, P, rs, p, ring[pos], sc, nrhs, pnorm));
+        if ((int)pend.size() == kDefer) II_CHECK(flush(false, nullptr));
+      } else {
+        II_CHECK(ddagdP(ctx, P, kappa, p, ss_, qs, ts, nullptr, nullptr, nrhs, skip_it, ss));
+        II_CHECK(sp_shift64(ctx, p, ss_, sig, sc, nrhs, part));
+        hipLaunchKernelGGL(k_fin_pap, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc,
+                           nullptr, 0, 0);
+        II_CHECK(cg_blas64(ctx, p, ss_, rs, ys, sc, nrhs, part, nb));
+        hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc, 1);
+        II_CHECK(cg_p_P(ctx, P, rs, p, p, sc, nrhs));
+      }
     }
     its += chunk;
     II_CHECK(read_scalars(ctx, nrhs));
@@ -1512,35 +1521,24 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
     if (all_done) break;
     if (any_upd) {
       if (lo) {
-        hipLaunchKernelGGL((k_accum<SpF32, StF32>), dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0,
-                           ctx->stream, g, Acc<1>::sp(ys, g.stride), Acc<1>::st(ys, g.stride),
-                           x64, skip_ru, ss);
-        II_HIP(ctx, hipGetLastError());
+        II_CHECK(join_updates(ctx, nrhs));
+        II_CHECK(flush(true, skip_ru));
       }
-      II_CHECK(ddagdP(ctx, 0, kappa, SF{x64}, q64, t64, u64, nullptr, nullptr, nrhs, skip_ru,
-                      ss));
-      hipLaunchKernelGGL(k_resid_shift, dim3(nb, nrhs), dim3(kBlock), 0, ctx->stream, g, b64,
-                         (const double2*)q64.v, (const double2*)x64, sig, (double2*)rho.v,
-                         skip_ru, ss, part);
-      hipLaunchKernelGGL(k_fin_rho, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc);
-      hipLaunchKernelGGL(k_norm2_masked, dim3(nb, nrhs), dim3(kBlock), 0, ctx->stream, g,
-                         (const double2*)rho.v, skip_ru, ss, part);
+      II_CHECK(residual(skip_ru, ss));
+      // |rho|^2 decides, and is the new |r|^2 of the rhs that go on
+      hipLaunchKernelGGL(k_fin_rho, dim3(nrhs), dim3(kFinThreads), 0, ctx->stream, part, nhd, sc);
       if (lo) II_CHECK(convertP(ctx, 0, P, rho, rs, nrhs, skip_ru, ss));
-      hipLaunchKernelGGL(k_fin_ru, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc);
+      hipLaunchKernelGGL(k_fin_ru, dim3(nrhs), dim3(kFinThreads), 0, ctx->stream, part, nhd, sc);
       II_HIP(ctx, hipGetLastError());
       // restart the search direction where the recursion broke (keep_p == 0)
-      II_CHECK(convertP(ctx, 0, P, rho, ps, nrhs, &sc[0].keep_p, ss));
+      II_CHECK(convertP(ctx, 0, P, rho, ring[pos], nrhs, &sc[0].keep_p, ss));
+      if (lo) II_CHECK(norm2P(ctx, P, ring[pos], nrhs, nullptr, 0, pnorm));
       chunk = 1;
     } else {
       chunk = std::min(chunk * 2, 8);
     }
   }
-  if (lo) {
-    hipLaunchKernelGGL((k_accum<SpF32, StF32>), dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0,
-                       ctx->stream, g, Acc<1>::sp(ys, g.stride), Acc<1>::st(ys, g.stride), x64,
-                       nullptr, 0);
-    II_HIP(ctx, hipGetLastError());
-  }
+  if (lo) II_CHECK(flush(true, nullptr));
   II_CHECK(read_scalars(ctx, nrhs));
   const double ms =
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1600,7 +1598,6 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
   // sloppy fields
   SF ps, rs, ss_, qs, ts, ys;
   const bool lo = P != II_PREC_DOUBLE;
-  const int ytype = lo ? II_PREC_SINGLE : II_PREC_DOUBLE;
   if (lo) {
     II_CHECK(fieldP(ctx, 50, P, batch, &ps));
     II_CHECK(fieldP(ctx, 51, P, batch, &rs));  // (A p is not stored: fused CG step)
@@ -1701,7 +1698,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
         II_CHECK(ddagdP(ctx, P, kappa, p, ss_, qs, ts, &p, part, nr, skip_it, ss));
         hipLaunchKernelGGL(k_fin_pap, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part,
                            hop_dot_parts(g, nr, P), sc, nullptr, 0, 0);
-        II_CHECK(cg_blas_P(ctx, P, p, ss_, rs, ys, ytype, sc, nr, part, nb));
+        II_CHECK(cg_blas64(ctx, p, ss_, rs, ys, sc, nr, part, nb));
         hipLaunchKernelGGL(k_fin_rr, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part, nb, sc, 1);
       }
       return cg_p_P(ctx, P, rs, p, ring[(cur + 1) % nring], sc, nr);

@@ -94,13 +94,13 @@ struct SpF64 {
   static constexpr bool kScaled = false;
   const double2* __restrict__ p;
   int stride;
-  int rs = 0;  // elements between rhs (0: 12 * stride, back to back)
+  int rs = 0;  // elements between rhs (0: 12 * stride, back to back; -1: one for all)
   __device__ __forceinline__ C ld(int site, int comp) const {
     return ld_at(p, (uint32_t)(comp * stride), (uint32_t)site);
   }
   __device__ __forceinline__ R scale(int) const { return 1.0; }
   __device__ __forceinline__ SpF64 rhs(int r) const {
-    return SpF64{p + (size_t)r * (rs ? rs : 12 * stride), stride, rs};
+    return SpF64{p + (size_t)r * (rs < 0 ? 0 : rs ? rs : 12 * stride), stride, rs};
   }
 };
 struct StF64 {

@@ -97,3 +97,21 @@ def test_multishift_full_index(nshift):
     ctx.close()
     assert res[0] < 1.1e-8
     assert abs(so.diff - max(res)) < 1e-3 * max(res) + 1e-13
+
+
+@pytest.mark.parametrize("precision", ["double", "single", "half"])
+@pytest.mark.parametrize("nshift", [1, 2, 13])
+def test_mixed_multishift_true_residuals(precision, nshift):
+    """One shift takes the single-rhs hops, 13 more than one block row of the
+    multi-rhs hop; shift 0 among them leaves the shift term out.  The solver
+    stops on the FP64 true residual: the bar is its tolerance."""
+    ctx, D, A = operator((6, 4, 4, 10))
+    b = np.random.default_rng(7).normal(size=D.fsize())
+    shifts = np.concatenate([[0.0], np.geomspace(1e-2, 1.0, nshift)])[:nshift]
+    x = [np.empty_like(b) for _ in shifts]
+    outs = ii.MultiShiftSolver_Mixed(A, tol=1e-10, precision=precision).solve(x, b, shifts)
+    res = [np.linalg.norm(A.mult(v) + s * v - b) / np.linalg.norm(b) for v, s in zip(x, shifts)]
+    ctx.close()
+    for o, r in zip(outs, res):
+        assert r <= 1.001e-10
+        assert abs(o.true_residual - r) < 1e-3 * r + 1e-14
