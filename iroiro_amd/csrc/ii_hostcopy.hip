@@ -3,8 +3,8 @@
 // The runtime moves pageable memory at 15 (1.6 MB) to 30 GB/s up and 14 to 17
 // GB/s down; the link takes 56 GB/s from pinned memory in pieces of some MiB
 // (21 GB/s in pieces of 512 KiB, 30 in 1 MiB).  Here the bytes go through
-// pinned slots of the context: a thread moves one piece between the caller's
-// array and a slot while its other slot is on the link.  One thread copies 28
+// pinned slots: a thread moves one piece between the caller's array and a slot
+// while its other slot is on the link.  One thread copies 28
 // GB/s, so a large copy takes two (three and four were no faster); the second
 // is started for the call and joined before it returns.  127 MB: 29 -> 43 GB/s
 // up, 17 -> 44 GB/s down; 25 MB: 32 -> 37 and 17 -> 32; 1.6 MB: 15 -> 18 and
@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -33,34 +34,50 @@ constexpr size_t kDirect = (size_t)64 << 10;
 
 }  // namespace
 
+// The pinned slots of a device, 16 MiB, shared by its contexts (pinning them
+// takes about 10 ms, which every context would pay): allocated at the first
+// copy that needs them, freed with the last context that used them.  A copy
+// holds `mu` throughout; a slot whose piece is still on its way to the device,
+// on whichever context's stream, is waited for through its event.
 struct HostPipe {
+  std::mutex mu;
   char* pin = nullptr;
   hipEvent_t ev[2 * kPipeThreads] = {};
+  int users = 0;
+  void free_slots() {
+    for (auto& e : ev) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+  }
 };
+constexpr int kPipeDevices = 64;  // as many as noalloc_setup lets a context be created on
+static HostPipe g_pipe[kPipeDevices];
 
 void host_pipe_release(ii_context* ctx) {
   HostPipe* H = static_cast<HostPipe*>(ctx->host_pipe);
   if (!H) return;
-  for (auto& e : H->ev)
-    if (e) (void)hipEventDestroy(e);
-  if (H->pin) (void)hipHostFree(H->pin);
-  delete H;
+  std::lock_guard<std::mutex> lock(H->mu);
+  if (--H->users == 0) H->free_slots();
   ctx->host_pipe = nullptr;
 }
 
-static ii_status host_pipe(ii_context* ctx, HostPipe** out) {
-  if (!ctx->host_pipe) {
-    ctx->host_pipe = new HostPipe();
-    HostPipe* H = static_cast<HostPipe*>(ctx->host_pipe);
+// the device's slots, H->mu held
+static ii_status host_pipe(ii_context* ctx, HostPipe* H) {
+  if (ctx->host_pipe) return II_OK;
+  if (!H->pin) {
     bool ok = hipHostMalloc((void**)&H->pin, 2 * kPipeThreads * kPieceMax) == hipSuccess;
     for (auto& e : H->ev)
       ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
-      host_pipe_release(ctx);
+      H->free_slots();
       return set_error(ctx, II_ERR_DEVICE, "pinned staging memory");
     }
   }
-  *out = static_cast<HostPipe*>(ctx->host_pipe);
+  ++H->users;
+  ctx->host_pipe = H;
   return II_OK;
 }
 
@@ -106,8 +123,9 @@ ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t byt
     II_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return II_OK;
   }
-  HostPipe* H = nullptr;
-  II_CHECK(host_pipe(ctx, &H));
+  HostPipe* H = &g_pipe[ctx->device];
+  std::lock_guard<std::mutex> lock(H->mu);
+  II_CHECK(host_pipe(ctx, H));
   return run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first = 0, len = 0;
     for (int i = 0; take(&first, &len); ++i) {
@@ -129,8 +147,9 @@ ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return II_OK;
   }
-  HostPipe* H = nullptr;
-  II_CHECK(host_pipe(ctx, &H));
+  HostPipe* H = &g_pipe[ctx->device];
+  std::lock_guard<std::mutex> lock(H->mu);
+  II_CHECK(host_pipe(ctx, H));
   return run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first[2] = {0, 0}, len[2] = {0, 0};
     auto request = [&](int b) {

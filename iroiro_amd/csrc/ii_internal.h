@@ -101,7 +101,7 @@ struct ii_context {
   int nscal = 0;
   void* host_pin = nullptr;       // pinned host block of the multishift scalars
   size_t host_pin_len = 0;
-  void* host_pipe = nullptr;      // pinned slots of the host copies (ii_hostcopy.hip)
+  void* host_pipe = nullptr;      // the device's pinned slots, once used (ii_hostcopy.hip)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // autotuned launch shapes
   ii::HopOrder hop_order;
@@ -157,8 +157,8 @@ ii_status ensure_scalars(ii_context* ctx, int n);
 // Pinned host block of at least `bytes` owned by the context (grows, never
 // shrinks), so solves allocate no pinned memory per call.
 ii_status ensure_host_pin(ii_context* ctx, size_t bytes, void** ptr);
-// Copies between a caller's (pageable) array and the device through pinned
-// slots of the context.  copy_to_device returns when src has been read; the
+// Copies between a caller's (pageable) array and the device through the
+// device's pinned slots.  copy_to_device returns when src has been read; the
 // device side is ordered on the context's stream.  copy_to_host follows the
 // stream's work and returns when dst is complete.
 ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t bytes);

@@ -18,7 +18,9 @@
 // [[Re W, -Im W], [Im W, Re W]] of the channel-spin mixing matrix of the
 // path, pre-arranged per lane (8 bf16 = 16 bytes) and staged in LDS once per
 // block.  C rows are (out channel, spin, re/im), accumulated in FP32 over
-// the 9 paths.  The adjoint layer is the same kernel with the paths
+// the 9 paths, the next path's loads requested before a path's products (8x8
+// at 16^3x32 158 -> 144 us, 1x8 83 -> 69 us; the FP32 transports' VALU work, 400
+// instructions a path and lane, is 70% of the time that is left).  The adjoint layer is the same kernel with the paths
 // mirrored and W -> W^dag (channel-transposed): T_{+mu}^dag = T_{-mu}.
 //
 // Weight gradient: FP32 matrix cores, gw[d][o][i] = sum_{x,c} g[o](x)
@@ -173,61 +175,113 @@ struct LayerArgs {
   int tiles_per_block;
 };
 
-// Transported 4-spinor of a channel field at one site: w = M v with M = 1,
-// U or U^dag.  The buffer base is the whole activation array (uniform), the
-// scalar offset `soff` must be wave-uniform (component blocks), and the
-// per-lane element offset `loff` carries the channel and the site, so no
-// load needs a per-lane descriptor or scalar offset.
-__device__ __forceinline__ void net_transport(const float2* __restrict__ base, uint32_t soff,
-                                              int stride, uint32_t loff, bool has_link, bool dag,
-                                              const float2 U[3][3], float2 w[4][3]) {
-  float2 v[4][3];
+// A path's neighbour spinors of the lane's channels (q, and 4 + q where the
+// layer has 8 input channels) and its link, as loaded.  The buffer base is the
+// whole activation array (uniform), the scalar offset must be wave-uniform
+// (component blocks), and the per-lane element offset carries the channel and
+// the site, so no load needs a per-lane descriptor or scalar offset.
+template <int KB>
+struct LayerRaw {
+  float2 v[KB][12];  // [3 spin + colour]
+  float2 u[6];       // r12 link
+  bool flip;         // the link carries the time boundary's sign
+};
+template <int CIN, int D>
+__device__ __forceinline__ void layer_request(const LayerArgs& a, int par, int s, int q,
+                                              const SiteCoord& sc, LayerRaw<frag_kb(CIN)>& r) {
+  const Geom& g = a.g;
+  constexpr int mu = D == 0 ? 0 : (D - 1) >> 1;
+  constexpr bool fw = D > 0 && ((D - 1) & 1) == 0;
+  const int nb = D == 0 ? s : neighbour(g, sc, s, mu, fw);
+  if constexpr (D > 0) {
+    const uint32_t base = (uint32_t)(((fw ? par : 1 - par) * 4 + mu) * 6 * g.stride);
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+    for (int k = 0; k < 6; ++k)
+      r.u[k] = ld_at(a.gauge, base + (uint32_t)(k * g.stride), (uint32_t)(fw ? s : nb));
+    r.flip = a.flip && mu == 3 && sc.t == (fw ? g.L[3] - 1 : 0);
+  }
+  const uint32_t soff = (uint32_t)((D == 0 ? par : 1 - par) * 12 * g.stride);
 #pragma unroll
-    for (int c = 0; c < 3; ++c) v[t][c] = ld_at(base, soff + (uint32_t)((3 * t + c) * stride), loff);
-  if (!has_link) {
+  for (int kb = 0; kb < frag_kb(CIN); ++kb) {
+    const int ch = 4 * kb + q;
+    if (ch < CIN) {
+      const uint32_t loff = (uint32_t)(ch * (size_t)24 * g.stride + nb);
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int k = 0; k < 12; ++k) r.v[kb][k] = ld_at(a.in, soff + (uint32_t)(k * g.stride), loff);
+    }
+  }
+}
+// The path's B operands: w = M v with M = 1, U or U^dag, rounded to bfloat16.
+template <int CIN, int D>
+__device__ __forceinline__ void layer_operands(const LayerRaw<frag_kb(CIN)>& r, int q,
+                                               bf16x8 B[3][frag_kb(CIN)]) {
+  constexpr bool dag = D > 0 && ((D - 1) & 1) == 1;
+  float2 U[3][3];
+  if constexpr (D > 0) {
 #pragma unroll
-      for (int c = 0; c < 3; ++c) w[t][c] = v[t][c];
-    return;
+    for (int k = 0; k < 6; ++k) U[k / 3][k % 3] = r.u[k];
+    r12_third_row(U, r.flip);
   }
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int kb = 0; kb < frag_kb(CIN); ++kb) {
+    const bool live = 4 * kb + q < CIN;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      float2 acc = make_float2(0.f, 0.f);
+    for (int c = 0; c < 3; ++c) {
+      bf16x8 b;
 #pragma unroll
-      for (int b = 0; b < 3; ++b) {
-        if (dag) cmacc(acc, U[b][a], v[t][b]);
-        else cmac(acc, U[a][b], v[t][b]);
+      for (int t = 0; t < 4; ++t) {
+        float2 w = make_float2(0.f, 0.f);
+        if (live) {
+          if constexpr (D == 0) {
+            w = r.v[kb][3 * t + c];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+              if (dag) cmacc(w, U[e][c], r.v[kb][3 * t + e]);
+              else cmac(w, U[c][e], r.v[kb][3 * t + e]);
+            }
+          }
+        }
+        b[2 * t] = (__bf16)w.x;
+        b[2 * t + 1] = (__bf16)w.y;
       }
-      w[t][a] = acc;
+      B[c][kb] = b;
     }
+  }
 }
 
-// Path d of half site s (parity par): neighbour half index (in parity
-// par ^ (d > 0)) and link.
-__device__ __forceinline__ int net_path(const Geom& g, const GaugeF32r12& gauge, int flip, int d,
-                                        int par, int s, const SiteCoord& sc, float2 U[3][3],
-                                        bool& dag) {
-  dag = false;
-  if (d == 0) return s;
-  const int mu = (d - 1) >> 1;
-  const bool fw = ((d - 1) & 1) == 0;
-  const int nb = neighbour(g, sc, s, mu, fw);
-  if (fw) {
-    gauge.ld(par, mu, s, flip && mu == 3 && sc.t == g.L[3] - 1, U);
-  } else {
-    gauge.ld(1 - par, mu, nb, flip && mu == 3 && sc.t == 0, U);
-    dag = true;
+// Paths D, D + 1, ...: the next path's loads are requested before this path's
+// products.
+template <int CIN, int COUT, int D>
+__device__ __forceinline__ void layer_paths(const LayerArgs& a, const uint4* sA, int par, int s,
+                                            int q, int lane, const SiteCoord& sc,
+                                            const LayerRaw<frag_kb(CIN)>& cur,
+                                            f32x4 acc[3][frag_mb(COUT)]) {
+  constexpr int MB = frag_mb(COUT), KB = frag_kb(CIN);
+  LayerRaw<KB> nxt;
+  if constexpr (D + 1 < kPaths) {
+    layer_request<CIN, D + 1>(a, par, s, q, sc, nxt);
+    asm volatile("" ::: "memory");  // not sunk below the products
   }
-  return nb;
+  bf16x8 B[3][KB];
+  layer_operands<CIN, D>(cur, q, B);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const uint4 araw = sA[((D * MB + mb) * KB + kb) * 64 + lane];
+      bf16x8 A;
+      __builtin_memcpy(&A, &araw, 16);
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[c][kb], acc[c][mb], 0, 0, 0);
+    }
+  if constexpr (D + 1 < kPaths)
+    layer_paths<CIN, COUT, D + 1>(a, sA, par, s, q, lane, sc, nxt, acc);
 }
 
 template <int CIN, int COUT>
-__global__ void __launch_bounds__(kLayerThreads) k_net_layer(LayerArgs a) {
+__global__ void __launch_bounds__(kLayerThreads, 2) k_net_layer(LayerArgs a) {
   constexpr int MB = frag_mb(COUT), KB = frag_kb(CIN);
   constexpr int NF = frag_count(CIN, COUT);
   __shared__ uint4 sA[NF];
@@ -239,7 +293,6 @@ __global__ void __launch_bounds__(kLayerThreads) k_net_layer(LayerArgs a) {
   const int tpp = (g.Vh + 15) >> 4;
   const int ntiles = tpp * a.npar;
   const size_t cs = (size_t)24 * g.stride;
-  const GaugeF32r12 gauge{a.gauge, g.stride};
   const int t_begin = blockIdx.x * a.tiles_per_block;
   const int t_end = min(t_begin + a.tiles_per_block, ntiles);
   for (int tile = t_begin + wave; tile < t_end; tile += kLayerThreads / 64) {
@@ -256,48 +309,9 @@ __global__ void __launch_bounds__(kLayerThreads) k_net_layer(LayerArgs a) {
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[c][mb][r] = 0.0f;
-#pragma unroll 1
-    for (int d = 0; d < kPaths; ++d) {
-      float2 U[3][3];
-      bool dag;
-      const int nb = net_path(g, gauge, a.flip, d, par, s, sc, U, dag);
-      const uint32_t soff = (uint32_t)((d == 0 ? par : 1 - par) * 12 * g.stride);
-      bf16x8 B[3][KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int ch = 4 * kb + q;
-        float2 w[4][3];
-        if (ch >= CIN) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) w[t][c] = make_float2(0.f, 0.f);
-        } else {
-          net_transport(a.in, soff, g.stride, (uint32_t)(ch * cs + nb), d != 0, dag, U, w);
-        }
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          bf16x8 b;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            b[2 * t] = (__bf16)w[t][c].x;
-            b[2 * t + 1] = (__bf16)w[t][c].y;
-          }
-          B[c][kb] = b;
-        }
-      }
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const uint4 araw = sA[((d * MB + mb) * KB + kb) * 64 + lane];
-          bf16x8 A;
-          __builtin_memcpy(&A, &araw, 16);
-#pragma unroll
-          for (int c = 0; c < 3; ++c)
-            acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[c][kb], acc[c][mb], 0, 0, 0);
-        }
-    }
+    LayerRaw<KB> raw;
+    layer_request<CIN, 0>(a, par, s, q, sc, raw);
+    layer_paths<CIN, COUT, 0>(a, sA, par, s, q, lane, sc, raw, acc);
     if (valid) {
       // C row 4q + r of block mb = (channel 2mb + q/2, spin 2(q&1) + r/2, re/im r&1)
 #pragma unroll
@@ -535,31 +549,38 @@ k_net_wgrad(Geom g, const float2* __restrict__ T, const float2* __restrict__ Lf,
     }
 }
 
-// gacc[e] += scale * sum_p partial[p][e], fixed order, FP64 sum: 64 entries a
-// block, 16 threads an entry (one thread an entry left 5 blocks summing 8192
-// partials each: 2.4 ms for a one-channel layer, now 22 us).
+// gacc[e] += scale * sum_p partial[p][e], fixed order, FP64 sum: 16 entries a
+// block (128-byte rows of a partial), 64 threads an entry.  One thread an entry
+// left 5 blocks summing 8192 partials each: 2.4 ms for a one-channel layer;
+// 64 entries a block took 22 us.
+constexpr int kRedEntries = 16;
 __global__ void __launch_bounds__(1024)
 k_net_wreduce(const float2* __restrict__ partial, int np, int ne, float scale,
               float2* __restrict__ gacc) {
-  __shared__ double2 part[16][64];
-  const int e = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
+  constexpr int SL = 1024 / kRedEntries;
+  __shared__ double2 part[SL][kRedEntries];
+  const int l = threadIdx.x % kRedEntries, sl = threadIdx.x / kRedEntries;
+  const int e = blockIdx.x * kRedEntries + l;
   double sr = 0.0, si = 0.0;
   if (e < ne)
-    for (int p = sl; p < np; p += 16) {
+    for (int p = sl; p < np; p += SL) {
       const float2 v = partial[(size_t)p * ne + e];
       sr += v.x;
       si += v.y;
     }
-  part[sl][threadIdx.x & 63] = make_double2(sr, si);
+  part[sl][l] = make_double2(sr, si);
   __syncthreads();
-  if (sl > 0 || e >= ne) return;
-  for (int k = 1; k < 16; ++k) {
-    sr += part[k][threadIdx.x].x;
-    si += part[k][threadIdx.x].y;
+  for (int h = SL / 2; h > 0; h /= 2) {
+    if (sl < h) {
+      part[sl][l].x += part[sl + h][l].x;
+      part[sl][l].y += part[sl + h][l].y;
+    }
+    __syncthreads();
   }
+  if (sl > 0 || e >= ne) return;
   float2 a = gacc[e];
-  a.x += (float)(scale * sr);
-  a.y += (float)(scale * si);
+  a.x += (float)(scale * part[0][l].x);
+  a.y += (float)(scale * part[0][l].y);
   gacc[e] = a;
 }
 
@@ -721,13 +742,16 @@ k_cdot(Geom g, const double2* __restrict__ a, const double2* __restrict__ b,
     part[2 * blockIdx.x + 1] = im;
   }
 }
-__global__ void k_cdot_fin(const double* __restrict__ part, int nb, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double re = 0.0, im = 0.0;
-    for (int i = 0; i < nb; ++i) {
-      re += part[2 * i];
-      im += part[2 * i + 1];
-    }
+__global__ void __launch_bounds__(kBlock)
+k_cdot_fin(const double* __restrict__ part, int nb, double* __restrict__ out) {
+  double re = 0.0, im = 0.0;
+  for (int i = threadIdx.x; i < nb; i += kBlock) {
+    re += part[2 * i];
+    im += part[2 * i + 1];
+  }
+  re = block_sum(re);
+  im = block_sum(im);
+  if (threadIdx.x == 0) {
     out[0] = re;
     out[1] = im;
   }
@@ -799,16 +823,17 @@ ii_status run_layer(ii_context* ctx, Net* N, int l, bool adj, const float2* in, 
   return set_error(ctx, II_ERR_STATE, "unsupported layer shape");
 }
 
-// Weight gradient of one layer added to gacc: at most kWgBlocks blocks, so
-// that a block's FP32 sums stay as short as 2048 sites at 32^3x64.
-constexpr int kWgBlocks = 1024;
+// Weight gradient of one layer added to gacc.  The number of blocks bounds the
+// length of their FP32 sums: 2048 sites a block for 8x8 channels at 32^3x64,
+// half of that for one channel, whose partials are an eighth.
 template <int CT>
 ii_status launch_wgrad(ii_context* ctx, Net* N, const float2* T, const float2* Lf, bool swap,
                        float2* gacc, float scale) {
   const Geom& g = ctx->g;
   constexpr int ne = kPaths * CT * 8 * 16;
   const int nq = 2 * g.Vh, stages = (nq + kWgSites - 1) / kWgSites;
-  const int spb = (stages + kWgBlocks - 1) / kWgBlocks * kWgSites;
+  constexpr int kMaxBlocks = CT == 8 ? 1024 : 2048;
+  const int spb = (stages + kMaxBlocks - 1) / kMaxBlocks * kWgSites;
   const int nblk = (nq + spb - 1) / spb;
   const size_t need = (size_t)nblk * ne;
   if (need > N->partial_len) {
@@ -821,7 +846,7 @@ ii_status launch_wgrad(ii_context* ctx, Net* N, const float2* T, const float2* L
                      (const float2*)ctx->gauge_lp[II_PREC_SINGLE], ctx->tbc_sign < 0, swap ? 1 : 0,
                      spb, (float*)N->partial);
   II_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL(k_net_wreduce, dim3((ne + 63) / 64), dim3(1024), 0, ctx->stream, N->partial,
+  hipLaunchKernelGGL(k_net_wreduce, dim3((ne + kRedEntries - 1) / kRedEntries), dim3(1024), 0, ctx->stream, N->partial,
                      nblk, ne, scale, gacc);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
@@ -994,7 +1019,7 @@ ii_status cdot(ii_context* ctx, Net* N, const double2* a, const double2* b, doub
   const Geom& g = ctx->g;
   const int nb = std::min(kRedBlocksMax, blocks_for(g.Vh));
   hipLaunchKernelGGL(k_cdot, dim3(nb), dim3(kBlock), 0, ctx->stream, g, a, b, N->dpart);
-  hipLaunchKernelGGL(k_cdot_fin, dim3(1), dim3(64), 0, ctx->stream, N->dpart, nb,
+  hipLaunchKernelGGL(k_cdot_fin, dim3(1), dim3(kBlock), 0, ctx->stream, N->dpart, nb,
                      N->dpart + 2 * kRedBlocksMax);
   II_HIP(ctx, hipGetLastError());
   II_HIP(ctx, hipMemcpyAsync(N->dhost, N->dpart + 2 * kRedBlocksMax, 2 * sizeof(double),
