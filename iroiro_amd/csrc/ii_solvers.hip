@@ -1573,7 +1573,11 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
   const int maxiter = prm->maxiter > 0 ? prm->maxiter : 100000;
   const size_t he = half_elems(g);
   const int nb = hop_blocks(g);
-  II_CHECK(ensure_partials(ctx, (size_t)std::max(nb, hop_dot_parts(g, batch, P)) * batch + 16));
+  // room for the vector kernels, the hops of either precision (one rhs: the
+  // FP64 hop writes a partial per 64 sites) and dot64, which must not move it
+  const int nhd = hop_dot_parts(g, batch, II_PREC_DOUBLE);
+  II_CHECK(ensure_partials(ctx, (size_t)batch * std::max({nb, hop_dot_parts(g, batch, P), nhd,
+                                                          2 * kRedBlocksMax}) + 16));
   II_CHECK(ensure_ru_scalars(ctx, batch));
   double* part = ctx->partials;
   RUScal* sc = dev_scal(ctx);
@@ -2268,7 +2272,9 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
   const int nb = hop_blocks(g);                   // BLAS partials per rhs
   const int nh = hop_dot_parts(g, batch, P);      // hop partials per rhs
   const int nhd = hop_dot_parts(g, batch, II_PREC_DOUBLE);
-  II_CHECK(ensure_partials(ctx, (size_t)3 * std::max(std::max(nb, nh), nhd) * batch + 16));
+  // dot64 must not move the partials either
+  II_CHECK(ensure_partials(
+      ctx, (size_t)batch * std::max(3 * std::max({nb, nh, nhd}), 2 * kRedBlocksMax) + 16));
   II_CHECK(ensure_ru_scalars(ctx, batch));
   double* part = ctx->partials;
   RUScal* sc = dev_scal(ctx);
