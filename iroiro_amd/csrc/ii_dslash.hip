@@ -774,14 +774,14 @@ ii_status tune_mrhs(ii_context* ctx, int P, int nrhs) {
 static bool links_cached(unsigned long long gauge_bytes) { return gauge_bytes <= (128ull << 20); }
 
 ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* out,
-                const double2* x, const double2* dv, int rs) {
+                const double2* x, const double2* dv) {
   const Geom& g = ctx->g;
   static const bool forced = std::getenv("II_HOP_ORDER") != nullptr;
   if (forced && h.nrhs == 1 && !ctx->hop_tuned && !h.no_tune) II_CHECK(tune_hop(ctx));
-  SpF64 sin{in, g.stride, rs};
-  StF64 so{out, g.stride};
-  SpF64 sx{x ? x : in, g.stride, rs};
-  SpF64 sd{dv ? dv : in, g.stride, h.dv_shared ? -1 : rs};
+  SpF64 sin{in, g.stride, h.rs_in};
+  StF64 so{out, g.stride, h.rs_out};
+  SpF64 sx{x ? x : in, g.stride, x ? h.rs_x : h.rs_in};
+  SpF64 sd{dv ? dv : in, g.stride, h.dv_shared ? -1 : dv ? h.rs_dv : h.rs_in};
   const unsigned long long gb = (unsigned long long)72 * g.stride * sizeof(double2);
   if (h.nrhs == 1 && links_cached(gb))
     return dispatch_hop(ctx, sin, GaugeF64Flat<0>{ctx->gauge64, g.stride}, so, sx, sd, h);

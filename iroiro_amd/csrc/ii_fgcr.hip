@@ -400,7 +400,7 @@ __global__ void k_g_coef(int m, GScal* __restrict__ gs) {
 // written for it)
 __global__ void __launch_bounds__(kGThreads)
 k_g_fold(Geom g, const float2* __restrict__ Z, size_t slot, int mm, double2* __restrict__ y,
-         const GScal* __restrict__ gs) {
+         size_t yrs, const GScal* __restrict__ gs) {
   const int rhs = blockIdx.y;
   const GScal& S = gs[rhs];
   if (S.done) return;
@@ -415,7 +415,7 @@ k_g_fold(Geom g, const float2* __restrict__ Z, size_t slot, int mm, double2* __r
     gi[i] = i < m ? S.gamma[i][1] : 0.0;
   }
   for (int c = 0; c < 12; ++c) {
-    double2 v = y[rhs * he + (size_t)c * g.stride + hs];
+    double2 v = y[rhs * yrs + (size_t)c * g.stride + hs];
 #pragma unroll
     for (int i = 0; i < kMaxK; ++i)
       if (i < m) {
@@ -423,7 +423,7 @@ k_g_fold(Geom g, const float2* __restrict__ Z, size_t slot, int mm, double2* __r
         v.x += gr[i] * a.x - gi[i] * a.y;
         v.y += gr[i] * a.y + gi[i] * a.x;
       }
-    y[rhs * he + (size_t)c * g.stride + hs] = v;
+    y[rhs * yrs + (size_t)c * g.stride + hs] = v;
   }
 }
 
@@ -504,7 +504,7 @@ struct Buf {
   size_t n = 0;
 };
 struct FGState {
-  Buf Z, W, R, Rb, T, y, be, bo, bh, rho, t64, part, gs, aux;
+  Buf Z, W, R, Rb, T, bh, rho, t64, part, gs, aux;
   GScal* host = nullptr;
   int host_n = 0;
 };
@@ -525,7 +525,7 @@ ii_status grow(ii_context* ctx, Buf& b, size_t bytes) {
 void fgcr_release(void* p) {
   FGState* s = static_cast<FGState*>(p);
   if (!s) return;
-  for (Buf* b : {&s->Z, &s->W, &s->R, &s->Rb, &s->T, &s->y, &s->be, &s->bo, &s->bh, &s->rho, &s->t64,
+  for (Buf* b : {&s->Z, &s->W, &s->R, &s->Rb, &s->T, &s->bh, &s->rho, &s->t64,
                  &s->part, &s->gs, &s->aux})
     if (b->p) (void)hipFree(b->p);
   if (s->host) (void)hipHostFree(s->host);
@@ -554,7 +554,7 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   II_CHECK(grow(ctx, S.R, slot * sizeof(float2)));
   if (use_net) II_CHECK(grow(ctx, S.Rb, (size_t)nr * g.stride * 12 * sizeof(uint32_t)));
   II_CHECK(grow(ctx, S.T, slot * sizeof(float2)));
-  for (Buf* b : {&S.y, &S.be, &S.bo, &S.bh, &S.rho, &S.t64})
+  for (Buf* b : {&S.bh, &S.rho, &S.t64})
     II_CHECK(grow(ctx, *b, nr * he * sizeof(double2)));
   const int nbs = blocks_for(g.Vh, kGThreads);
   const int nbh = hop_dot_parts(g, nr, II_PREC_DOUBLE);
@@ -574,11 +574,14 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   float2* R = (float2*)S.R.p;
   uint32_t* Rb = use_net ? (uint32_t*)S.Rb.p : nullptr;  // r as the network's bf16 input
   float2* T = (float2*)S.T.p;
-  double2 *y = (double2*)S.y.p, *be = (double2*)S.be.p, *bo = (double2*)S.bo.p,
-          *bh = (double2*)S.bh.p, *rho = (double2*)S.rho.p, *t64 = (double2*)S.t64.p;
+  // the sources' parities are read and the solution's written in place
+  const int prs = (int)(2 * he);  // elements between the rhs of one parity
+  const double2 *be = src->data, *bo = src->data + he;
+  double2 *y = sol->data, *xo = sol->data + he, *bh = (double2*)S.bh.p,
+          *rho = (double2*)S.rho.p, *t64 = (double2*)S.t64.p;
   double* part = (double*)S.part.p;
   GScal* gs = (GScal*)S.gs.p;
-  double* aux = (double*)S.aux.p;  // |b_e|^2, |b_o|^2, |bhat|^2, the scalar 1.0
+  double* aux = (double*)S.aux.p;  // |b|^2 by rhs and parity, |bhat|^2, the scalar 1.0
   double* one = aux + 3 * nr;
   const dim3 sgrid(nbs, nr);
 
@@ -588,26 +591,23 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   if (ctx->mrhs_nrhs[II_PREC_DOUBLE] != nr) II_CHECK(tune_mrhs(ctx, II_PREC_DOUBLE, nr));
   II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   // bhat = b_e + kappa H_eo b_o (eoUtils.cpp:54-57), |b|^2 of the full sources
-  for (int k = 0; k < nr; ++k) {
-    const double2* base = src->data + (size_t)k * 2 * he;
-    II_CHECK(copy64(ctx, be + k * he, base));
-    II_CHECK(copy64(ctx, bo + k * he, base + he));
-  }
-  II_CHECK(dot64(ctx, be, be, aux, nr));
-  II_CHECK(dot64(ctx, bo, bo, aux + nr, nr));
+  II_CHECK(dot64(ctx, be, be, aux, 2 * nr));
   HopSpec h;
   h.out_par = 0;
   h.a = kappa;
   h.xpay = true;
   h.nrhs = nr;
+  h.rs_in = h.rs_x = prs;
+  h.epi = kEpiNorm;
+  h.partials = part;
   II_CHECK(hop64(ctx, h, bo, bh, be, nullptr));
-  II_CHECK(dot64(ctx, bh, bh, aux + 2 * nr, nr));
+  II_CHECK(finalize_sums(ctx, part, nbh, aux + 2 * nr, nr));
   {
     std::vector<double> hb(3 * nr + 1);
     II_HIP(ctx, hipMemcpyAsync(hb.data(), aux, 3 * nr * sizeof(double), hipMemcpyDeviceToHost,
                                ctx->stream));
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    for (int k = 0; k < nr; ++k) hb[k] += hb[nr + k];
+    for (int k = 0; k < nr; ++k) hb[k] = hb[2 * k] + hb[2 * k + 1];
     hb[3 * nr] = 1.0;
     II_HIP(ctx, hipMemcpyAsync(aux, hb.data(), nr * sizeof(double), hipMemcpyHostToDevice,
                                ctx->stream));
@@ -616,7 +616,7 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   }
   hipLaunchKernelGGL(k_g_init, dim3((nr + 63) / 64), dim3(64), 0, ctx->stream, aux, aux + 2 * nr,
                      tol, nr, gs);
-  II_CHECK(zero64(ctx, y, nr));
+  II_CHECK(zero64(ctx, y, nr, prs));
   hipLaunchKernelGGL(k_g_to32, sgrid, dim3(kGThreads), 0, ctx->stream, g, bh, R, Rb, gs);
   II_HIP(ctx, hipGetLastError());
 
@@ -668,13 +668,15 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
       II_HIP(ctx, hipGetLastError());
     }
     hipLaunchKernelGGL(k_g_coef, dim3(nr), dim3(64), 0, ctx->stream, m, gs);
-    hipLaunchKernelGGL(k_g_fold, sgrid, dim3(kGThreads), 0, ctx->stream, g, Z, slot, m, y, gs);
+    hipLaunchKernelGGL(k_g_fold, sgrid, dim3(kGThreads), 0, ctx->stream, g, Z, slot, m, y,
+                       (size_t)prs, gs);
     // rho = bhat - Dhat y (FP64) with |rho|^2 in the second hop's epilogue
     HopSpec b;
     b.nrhs = nr;
     b.skip = donef;
     b.skip_stride = kGInts;
     b.out_par = 1;
+    b.rs_in = prs;
     II_CHECK(hop64(ctx, b, y, t64, nullptr, nullptr));
     b.out_par = 0;
     b.a = -kappa * kappa;
@@ -683,6 +685,8 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
     b.coef = one;
     b.coef_stride = 0;
     b.partials = part;
+    b.rs_in = 0;
+    b.rs_x = prs;
     II_CHECK(hop64(ctx, b, t64, rho, y, bh));
     hipLaunchKernelGGL(k_g_rho, dim3(nr), dim3(1024), 0, ctx->stream, part, nbh, gs);
     hipLaunchKernelGGL(k_g_to32, sgrid, dim3(kGThreads), 0, ctx->stream, g, rho, R, Rb, gs);
@@ -768,7 +772,7 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
     II_CHECK(propagator(ctx, kappa, &fp, &tmp_src, &tmp_sol, fo.data()));
     for (int k = 0; k < nr; ++k)
       if (!S.host[k].done) {
-        II_CHECK(axpby64(ctx, 1.0, tmp_sol.data + (size_t)k * 2 * he, 1.0, y + k * he));
+        II_CHECK(axpby64(ctx, 1.0, tmp_sol.data + (size_t)k * 2 * he, 1.0, y + (size_t)k * prs));
         fb_its = std::max(fb_its, fo[k].iterations);
       }
     (void)stalled;
@@ -779,12 +783,8 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   h.a = kappa;
   h.xpay = true;
   h.nrhs = nr;
-  II_CHECK(hop64(ctx, h, y, t64, bo, nullptr));
-  for (int k = 0; k < nr; ++k) {
-    double2* base = sol->data + (size_t)k * 2 * he;
-    II_CHECK(copy64(ctx, base, y + k * he));
-    II_CHECK(copy64(ctx, base + he, t64 + k * he));
-  }
+  h.rs_in = h.rs_out = h.rs_x = prs;
+  II_CHECK(hop64(ctx, h, y, xo, bo, nullptr));
   II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
   II_HIP(ctx, hipMemcpyAsync(S.host, gs, sizeof(GScal) * nr, hipMemcpyDeviceToHost, ctx->stream));
   II_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -61,6 +61,9 @@ struct HopSpec {
   const void* p = nullptr;
   const float* p_nrm = nullptr;
   bool dv_shared = false;        // FP64: one dv for every rhs
+  // FP64: elements between the rhs of in, out, x and dv (0: back to back, 12 *
+  // stride; 24 * stride addresses one parity of full fields)
+  int rs_in = 0, rs_out = 0, rs_x = 0, rs_dv = 0;
   int nrhs = 1;
   double* partials = nullptr;
   // optional per-rhs skip flags: rhs r is skipped when skip[r * skip_stride] != 0
@@ -82,10 +85,8 @@ struct LoField {
   float* nrm = nullptr;
 };
 
-// rs: elements between the rhs of in, x and dv (0: back to back, 12 * stride;
-// 24 * stride addresses one parity of full fields); out is back to back
 ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* out,
-                const double2* x, const double2* dv, int rs = 0);
+                const double2* x, const double2* dv);
 ii_status hop32(ii_context* ctx, const HopSpec& h, const float2* in, float2* out,
                 const float2* x, const float2* dv);
 ii_status hop_half(ii_context* ctx, const HopSpec& h, const LoField& in, const LoField& out,
@@ -122,7 +123,8 @@ ii_status ddagd64(ii_context* ctx, double kappa, const double2* f, double2* out,
 ii_status dot64(ii_context* ctx, const double2* a, const double2* b, double* dst, int nrhs = 1);
 ii_status finalize_sums(ii_context* ctx, const double* partials, int nblk, double* dst, int nrhs);
 ii_status copy64(ii_context* ctx, double2* dst, const double2* src, int nrhs = 1);
-ii_status zero64(ii_context* ctx, double2* dst, int nrhs = 1);
+// rs: elements between the rhs (0: back to back)
+ii_status zero64(ii_context* ctx, double2* dst, int nrhs = 1, int rs = 0);
 // y = a*x + b*y with host scalars
 ii_status axpby64(ii_context* ctx, double a, const double2* x, double b, double2* y, int nrhs = 1);
 ii_status gamma5_64(ii_context* ctx, const double2* in, double2* out, int nrhs = 1);

@@ -113,18 +113,20 @@ __global__ void k_fin_rr(const double* __restrict__ partials, int nb, RUScal* __
 }
 
 // ============================================================ generic site BLAS
-// Accessor construction from an any-precision field.
+// Accessor construction from an any-precision field.  rs: FP64 fields only,
+// elements between the rhs (0: back to back).
 struct SF {
   void* v = nullptr;
   float* nrm = nullptr;
+  int rs = 0;
 };
 
 template <int P> struct Acc;
 template <> struct Acc<II_PREC_DOUBLE> {
   using Sp = SpF64;
   using St = StF64;
-  static Sp sp(const SF& f, int stride) { return Sp{(const double2*)f.v, stride}; }
-  static St st(const SF& f, int stride) { return St{(double2*)f.v, stride}; }
+  static Sp sp(const SF& f, int stride) { return Sp{(const double2*)f.v, stride, f.rs}; }
+  static St st(const SF& f, int stride) { return St{(double2*)f.v, stride, f.rs}; }
 };
 template <> struct Acc<II_PREC_SINGLE> {
   using Sp = SpF32;
@@ -244,7 +246,8 @@ struct DeferredDirs {
 template <typename SpP, typename SpY, typename StY>
 __global__ void __launch_bounds__(kBlock)
 k_cg_flush(Geom g, DeferredDirs<SpP> d, const double* __restrict__ ahist, int astride, SpY yr,
-           StY yw, double2* __restrict__ y64, const int* __restrict__ skip, int skip_stride) {
+           StY yw, double2* __restrict__ y64, size_t y64_rs, const int* __restrict__ skip,
+           int skip_stride) {
   const int rhs = blockIdx.y;
   const int hs = blockIdx.x * blockDim.x + threadIdx.x;
   if (hs >= g.Vh) return;
@@ -264,7 +267,7 @@ k_cg_flush(Geom g, DeferredDirs<SpP> d, const double* __restrict__ ahist, int as
     }
   }
   if (fold) {
-    double2* y = y64 + (size_t)rhs * 12 * g.stride;
+    double2* y = y64 + (size_t)rhs * y64_rs;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
       double2 o = y[(size_t)k * g.stride + hs];
@@ -378,9 +381,15 @@ __global__ void k_fin_ru(const double* __restrict__ partials, int nb, RUScal* __
 ii_status hopP(ii_context* ctx, int P, const HopSpec& h, const SF& in, const SF& out,
                const SF* x, const SF* dv) {
   switch (P) {
-    case II_PREC_DOUBLE:
-      return hop64(ctx, h, (const double2*)in.v, (double2*)out.v,
+    case II_PREC_DOUBLE: {
+      HopSpec k = h;
+      k.rs_in = in.rs;
+      k.rs_out = out.rs;
+      k.rs_x = x ? x->rs : 0;
+      k.rs_dv = dv ? dv->rs : 0;
+      return hop64(ctx, k, (const double2*)in.v, (double2*)out.v,
                    x ? (const double2*)x->v : nullptr, dv ? (const double2*)dv->v : nullptr);
+    }
     case II_PREC_SINGLE:
       return hop32(ctx, h, (const float2*)in.v, (float2*)out.v,
                    x ? (const float2*)x->v : nullptr, dv ? (const float2*)dv->v : nullptr);
@@ -476,6 +485,11 @@ ii_status ddagd_cg_fused(ii_context* ctx, int P, double kappa, const SF& p, cons
   return hopP(ctx, P, h, t, r, &q, &r);  // r -= alpha Dhat^dag q, |r|^2
 }
 
+// elements between the rhs of the FP64 field a flush folds into
+size_t fold_stride(const Geom& g, const SF* y) {
+  return y && y->rs ? (size_t)y->rs : (size_t)12 * g.stride;
+}
+
 // y += alpha p; r -= alpha s; |r|^2 partials, FP64
 ii_status cg_blas64(ii_context* ctx, const SF& p, const SF& s, const SF& r, const SF& y,
                     RUScal* sc, int nrhs, double* partials, int nb) {
@@ -508,7 +522,7 @@ ii_status cg_p_update(ii_context* ctx, const SF& r, const SF& p, const SF& pout,
 // y64, also fold into y64 (rhs not masked by skip)
 template <int P>
 ii_status cg_flush(ii_context* ctx, const SF* ring, const int* slots, int n, const double* ahist,
-                   int astride, const SF& y, int nrhs, double2* y64, const int* skip,
+                   int astride, const SF& y, int nrhs, const SF* y64, const int* skip,
                    int skip_stride) {
   const Geom& g = ctx->g;
   using A = Acc<P>;
@@ -522,7 +536,7 @@ ii_status cg_flush(ii_context* ctx, const SF* ring, const int* slots, int n, con
   hipLaunchKernelGGL((k_cg_flush<typename A::Sp, SpF32, StF32>), dim3(blocks_for(g.Vh), nrhs),
                      dim3(kBlock), 0, ctx->stream, g, d, ahist, astride,
                      Acc<II_PREC_SINGLE>::sp(y, g.stride), Acc<II_PREC_SINGLE>::st(y, g.stride),
-                     y64, skip, skip_stride);
+                     y64 ? (double2*)y64->v : nullptr, fold_stride(g, y64), skip, skip_stride);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
 }
@@ -580,7 +594,7 @@ ii_status cg_p_P(ii_context* ctx, int P, const SF& r, const SF& p, const SF& pou
 }
 ii_status cg_flush_P(ii_context* ctx, int P, const SF* ring, const int* slots, int n,
                      const double* ahist, int astride, const SF& y, int nrhs,
-                     double2* y64 = nullptr, const int* skip = nullptr, int skip_stride = 0) {
+                     const SF* y64 = nullptr, const int* skip = nullptr, int skip_stride = 0) {
   switch (P) {
     case 1: return cg_flush<1>(ctx, ring, slots, n, ahist, astride, y, nrhs, y64, skip, skip_stride);
     case 2: return cg_flush<2>(ctx, ring, slots, n, ahist, astride, y, nrhs, y64, skip, skip_stride);
@@ -1388,7 +1402,8 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   double* rr0 = sig + nrhs;
   double* bb = rr0 + nrhs;
   double* one = bb + nrhs;  // the device scalar 1.0 (alpha of rho = b - (A + sigma) x)
-  SF t64, u64, rho, ps, rs, ss_, qs, ts, ys;
+  SF t64, u64, rho, rs, ss_, qs, ts, ys;
+  const SF xf{x64};
   II_CHECK(fieldP(ctx, 39, 0, nrhs, &t64));  // Dhat x, intermediate
   II_CHECK(fieldP(ctx, 41, 0, nrhs, &u64));  // odd temporary
   II_CHECK(fieldP(ctx, 40, 0, nrhs, &rho));
@@ -1425,7 +1440,6 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
     h.out_par = 0;
     h.a = -kappa * kappa;
     h.xpay = true;
-    const SF xf{x64};
     II_CHECK(hopP(ctx, 0, h, u64, t64, &xf, nullptr));  // Dhat x
     h.out_par = 1;
     h.a = 1.0;
@@ -1472,7 +1486,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   auto flush = [&](bool fold, const int* skip) -> ii_status {
     if (!fold && pend.empty()) return II_OK;
     II_CHECK(cg_flush_P(ctx, P, ring.data(), pend.data(), (int)pend.size(), ahist, nring, ys, nrhs,
-                        fold ? x64 : nullptr, skip, ss));
+                        fold ? &xf : nullptr, skip, ss));
     pend.clear();
     return II_OK;
   };
@@ -1558,6 +1572,11 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   return II_OK;
 }
 
+// parity `par` of the rhs from r0 on of a full field, in place
+SF parity_of(const ii_field* f, int r0, int par, size_t he) {
+  return SF{f->data + ((size_t)2 * r0 + par) * he, nullptr, (int)(2 * he)};
+}
+
 // ============================================================ propagator
 // Work slots 40..63 belong to the propagator solver.
 ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
@@ -1585,16 +1604,14 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
   const int* skip_it = &sc[0].done;
   const int* skip_ru = &sc[0].skip_ru;
   void* auxp = nullptr;
-  // aux: |b_e|^2 [0, batch), |b_o|^2 [batch, 2 batch), |c|^2 [2 batch, 3 batch)
+  // aux: |b|^2 of each rhs and parity [0, 2 batch), |c|^2 [2 batch, 3 batch)
   II_CHECK(workspace(ctx, 40, sizeof(double) * 3 * batch + 64, &auxp));
   double* aux = (double*)auxp;
   double* one = aux + 3 * batch;  // the device scalar 1.0 (alpha of rho = bhat - Dhat y)
-  // FP64 fields
-  SF be, bo, bh, y, r64, q64, t64, rho;
-  II_CHECK(fieldP(ctx, 41, 0, batch, &be));
-  II_CHECK(fieldP(ctx, 42, 0, batch, &bo));
+  // FP64 fields; the sources' parities are read and the solution's written in
+  // place (y is the even part of sol)
+  SF be, bo, bh, y, xo, r64, q64, t64, rho;
   II_CHECK(fieldP(ctx, 43, 0, batch, &bh));
-  II_CHECK(fieldP(ctx, 44, 0, batch, &y));
   II_CHECK(fieldP(ctx, 45, 0, batch, &r64));
   II_CHECK(fieldP(ctx, 46, 0, batch, &q64));
   II_CHECK(fieldP(ctx, 47, 0, batch, &t64));
@@ -1614,7 +1631,6 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     II_CHECK(fieldP(ctx, 52, 0, batch, &ss_));
     qs = q64;
     ts = t64;
-    ys = y;
   }
   // Deferred solution update (sloppy precisions): the search directions of
   // up to kDefer iterations stay in a ring of kDefer + 1 fields, their
@@ -1635,26 +1651,24 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     const int nr = std::min(batch, nrhs_all - r0);
     auto t0 = std::chrono::steady_clock::now();
     II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    // gather even/odd parts of the sources
-    for (int k = 0; k < nr; ++k) {
-      const double2* base = src->data + (size_t)(r0 + k) * 2 * he;
-      II_CHECK(copy64(ctx, (double2*)be.v + k * he, base));
-      II_CHECK(copy64(ctx, (double2*)bo.v + k * he, base + he));
-    }
+    be = parity_of(src, r0, 0, he);
+    bo = parity_of(src, r0, 1, he);
+    y = parity_of(sol, r0, 0, he);
+    xo = parity_of(sol, r0, 1, he);
+    if (!lo) ys = y;
     // |b|^2 of the full sources
-    II_CHECK(dot64(ctx, (double2*)be.v, (double2*)be.v, aux, nr));
-    II_CHECK(dot64(ctx, (double2*)bo.v, (double2*)bo.v, aux + batch, nr));
+    II_CHECK(dot64(ctx, (double2*)be.v, (double2*)be.v, aux, 2 * nr));
     // bhat = b_e - mult_eo(b_o) = b_e + kappa H_eo b_o   (eoUtils.cpp:54-57)
     h = HopSpec();
     h.out_par = 0;
     h.a = kappa;
     h.xpay = true;
     h.nrhs = nr;
-    II_CHECK(hop64(ctx, h, (double2*)bo.v, (double2*)bh.v, (double2*)be.v, nullptr));
+    II_CHECK(hopP(ctx, 0, h, bo, bh, &be, nullptr));
     // c = Dhat^dag bhat  -> r64 ; y = 0
     II_CHECK(dhat_dag64(ctx, kappa, (double2*)bh.v, (double2*)r64.v, (double2*)t64.v, nullptr,
                         nullptr, nr));
-    II_CHECK(zero64(ctx, (double2*)y.v, nr));
+    II_CHECK(zero64(ctx, (double2*)y.v, nr, y.rs));
     // rr = |c|^2 into aux[2*batch ...]
     II_CHECK(dot64(ctx, (double2*)r64.v, (double2*)r64.v, aux + 2 * batch, nr));
     // b2 = |b_e|^2 + |b_o|^2 -> aux[0..nr)
@@ -1663,7 +1677,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
       II_HIP(ctx, hipMemcpyAsync(hb.data(), aux, 2 * batch * sizeof(double),
                                  hipMemcpyDeviceToHost, ctx->stream));
       II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-      for (int k = 0; k < nr; ++k) hb[k] += hb[batch + k];
+      for (int k = 0; k < nr; ++k) hb[k] = hb[2 * k] + hb[2 * k + 1];
       II_HIP(ctx, hipMemcpyAsync(aux, hb.data(), nr * sizeof(double), hipMemcpyHostToDevice,
                                  ctx->stream));
       const double unit = 1.0;
@@ -1718,7 +1732,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     // masked by skip), ys restarted at 0
     auto flush_fold = [&](const int* skip) -> ii_status {
       II_CHECK(cg_flush_P(ctx, P, ring.data(), pend.data(), (int)pend.size(), ahist, nring, ys,
-                          nr, (double2*)y.v, skip, ss));
+                          nr, &y, skip, ss));
       pend.clear();
       return II_OK;
     };
@@ -1783,7 +1797,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
         h.skip_stride = ss;
         h.out_par = 1;
         h.a = 1.0;
-        II_CHECK(hop64(ctx, h, (double2*)y.v, (double2*)t64.v, nullptr, nullptr));
+        II_CHECK(hopP(ctx, 0, h, y, t64, nullptr, nullptr));
         // rho = bhat - (y - kappa^2 H_eo t) and |rho|^2 in the hop's epilogue
         h.out_par = 0;
         h.a = -kappa * kappa;
@@ -1792,8 +1806,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
         h.coef = one;
         h.coef_stride = 0;
         h.partials = part;
-        II_CHECK(hop64(ctx, h, (double2*)t64.v, (double2*)rho.v, (double2*)y.v,
-                       (const double2*)bh.v));
+        II_CHECK(hopP(ctx, 0, h, t64, rho, &y, &bh));
         hipLaunchKernelGGL(k_fin_rho, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part,
                            hop_dot_parts(g, nr, II_PREC_DOUBLE), sc);
         // new CG residual r = Dhat^dag rho and |r|^2.  The true residual rho
@@ -1846,12 +1859,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     h.a = kappa;
     h.xpay = true;
     h.nrhs = nr;
-    II_CHECK(hop64(ctx, h, (double2*)y.v, (double2*)t64.v, (double2*)bo.v, nullptr));
-    for (int k = 0; k < nr; ++k) {
-      double2* base = sol->data + (size_t)(r0 + k) * 2 * he;
-      II_CHECK(copy64(ctx, base, (double2*)y.v + k * he));
-      II_CHECK(copy64(ctx, base + he, (double2*)t64.v + k * he));
-    }
+    II_CHECK(hopP(ctx, 0, h, y, xo, &bo, nullptr));
     II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     II_CHECK(read_scalars(ctx, nr));
     float ms = 0.f;
@@ -2092,7 +2100,8 @@ struct BiDirs {
 template <typename SpP, typename SpY, typename StY>
 __global__ void __launch_bounds__(kBlock)
 k_bi_flush(Geom g, BiDirs<SpP> d, const double* __restrict__ ahist, int astride, SpY yr, StY yw,
-           double2* __restrict__ y64, const int* __restrict__ skip, int skip_stride) {
+           double2* __restrict__ y64, size_t y64_rs, const int* __restrict__ skip,
+           int skip_stride) {
   const int rhs = blockIdx.y;
   const int hs = blockIdx.x * blockDim.x + threadIdx.x;
   if (hs >= g.Vh) return;
@@ -2124,7 +2133,7 @@ k_bi_flush(Geom g, BiDirs<SpP> d, const double* __restrict__ ahist, int astride,
     }
   }
   if (fold) {
-    double2* y = y64 + (size_t)rhs * 12 * g.stride;
+    double2* y = y64 + (size_t)rhs * y64_rs;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
       double2 o = y[(size_t)k * g.stride + hs];
@@ -2214,7 +2223,7 @@ struct BiBlas {
     return II_OK;
   }
   static ii_status flush(ii_context* ctx, const SF* rp, const SF* rs, const int* slots, int n,
-                         const double* ahist, int astride, const SF& y, int nrhs, double2* y64,
+                         const double* ahist, int astride, const SF& y, int nrhs, const SF* y64,
                          const int* skip, int ss) {
     const Geom& g = ctx->g;
     using Y = Acc<II_PREC_SINGLE>;
@@ -2228,7 +2237,8 @@ struct BiBlas {
     }
     hipLaunchKernelGGL((k_bi_flush<typename A::Sp, typename Y::Sp, typename Y::St>),
                        dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g, d, ahist,
-                       astride, Y::sp(y, g.stride), Y::st(y, g.stride), y64, skip, ss);
+                       astride, Y::sp(y, g.stride), Y::st(y, g.stride),
+                       y64 ? (double2*)y64->v : nullptr, fold_stride(g, y64), skip, ss);
     II_HIP(ctx, hipGetLastError());
     return II_OK;
   }
@@ -2287,11 +2297,8 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
   double* one = aux + 3 * batch;
   II_CHECK(workspace(ctx, 63, sizeof(BiCoef) * batch, &v));
   BiCoef* bc = (BiCoef*)v;
-  SF be, bo, bh, y, q64, t64;
-  II_CHECK(fieldP(ctx, 41, 0, batch, &be));
-  II_CHECK(fieldP(ctx, 42, 0, batch, &bo));
+  SF be, bo, bh, y, xo, q64, t64;  // be, bo: parities of src; y, xo: of sol
   II_CHECK(fieldP(ctx, 43, 0, batch, &bh));
-  II_CHECK(fieldP(ctx, 44, 0, batch, &y));
   II_CHECK(fieldP(ctx, 46, 0, batch, &q64));
   II_CHECK(fieldP(ctx, 47, 0, batch, &t64));
   SF r, r0, vv, w, t, ys;
@@ -2316,28 +2323,28 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
     const int nr = std::min(batch, nrhs_all - rb0);
     const size_t plh = (size_t)nr * nh, plb = (size_t)nr * nb;
     II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    for (int k = 0; k < nr; ++k) {
-      const double2* base = src->data + (size_t)(rb0 + k) * 2 * he;
-      II_CHECK(copy64(ctx, (double2*)be.v + k * he, base));
-      II_CHECK(copy64(ctx, (double2*)bo.v + k * he, base + he));
-    }
-    II_CHECK(dot64(ctx, (double2*)be.v, (double2*)be.v, aux, nr));
-    II_CHECK(dot64(ctx, (double2*)bo.v, (double2*)bo.v, aux + batch, nr));
+    be = parity_of(src, rb0, 0, he);
+    bo = parity_of(src, rb0, 1, he);
+    y = parity_of(sol, rb0, 0, he);
+    xo = parity_of(sol, rb0, 1, he);
+    II_CHECK(dot64(ctx, (double2*)be.v, (double2*)be.v, aux, 2 * nr));
     // bhat = b_e + kappa H_eo b_o   (eoUtils.cpp:54-57)
     h = HopSpec();
     h.out_par = 0;
     h.a = kappa;
     h.xpay = true;
     h.nrhs = nr;
-    II_CHECK(hop64(ctx, h, (double2*)bo.v, (double2*)bh.v, (double2*)be.v, nullptr));
-    II_CHECK(zero64(ctx, (double2*)y.v, nr));
-    II_CHECK(dot64(ctx, (double2*)bh.v, (double2*)bh.v, aux + 2 * batch, nr));
+    h.epi = kEpiNorm;
+    h.partials = part;
+    II_CHECK(hopP(ctx, 0, h, bo, bh, &be, nullptr));
+    II_CHECK(finalize_sums(ctx, part, hop_dot_parts(g, nr, II_PREC_DOUBLE), aux + 2 * batch, nr));
+    II_CHECK(zero64(ctx, (double2*)y.v, nr, y.rs));
     {
       std::vector<double> hb(2 * batch);
       II_HIP(ctx, hipMemcpyAsync(hb.data(), aux, 2 * batch * sizeof(double),
                                  hipMemcpyDeviceToHost, ctx->stream));
       II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-      for (int k = 0; k < nr; ++k) hb[k] += hb[batch + k];
+      for (int k = 0; k < nr; ++k) hb[k] = hb[2 * k] + hb[2 * k + 1];
       II_HIP(ctx, hipMemcpyAsync(aux, hb.data(), nr * sizeof(double), hipMemcpyHostToDevice,
                                  ctx->stream));
       const double unit = 1.0;
@@ -2355,7 +2362,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
     II_CHECK(convertP(ctx, 0, II_PREC_SINGLE, y, ys, nr));  // zeros
     int pos = 0;            // ring slot of this iteration's p and s
     std::vector<int> pend;  // slots whose alpha p + omega s is not yet in ys
-    auto flush = [&](double2* y64, const int* skip) -> ii_status {
+    auto flush = [&](const SF* y64, const int* skip) -> ii_status {
       if (pend.empty() && !y64) return II_OK;
       II_CHECK(BB::flush(ctx, rp, rsr, pend.empty() ? &pos : pend.data(), (int)pend.size(), ahist,
                          nring, ys, nr, y64, skip, ss));
@@ -2428,7 +2435,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       chunk = 1;
       II_CHECK(join_updates(ctx, nr));
       // reliable update for the flagged rhs: y64 += ys + pending, ys = 0
-      II_CHECK(flush((double2*)y.v, skip_ru));
+      II_CHECK(flush(&y, skip_ru));
       // rho_true = bhat - Dhat y (FP64) and |rho_true|^2
       h = HopSpec();
       h.nrhs = nr;
@@ -2436,7 +2443,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       h.skip_stride = ss;
       h.out_par = 1;
       h.a = 1.0;
-      II_CHECK(hop64(ctx, h, (double2*)y.v, (double2*)t64.v, nullptr, nullptr));
+      II_CHECK(hopP(ctx, 0, h, y, t64, nullptr, nullptr));
       h.out_par = 0;
       h.a = -kappa * kappa;
       h.xpay = true;
@@ -2444,8 +2451,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       h.coef = one;
       h.coef_stride = 0;
       h.partials = part;
-      II_CHECK(hop64(ctx, h, (double2*)t64.v, (double2*)q64.v, (double2*)y.v,
-                     (const double2*)bh.v));
+      II_CHECK(hopP(ctx, 0, h, t64, q64, &y, &bh));
       hipLaunchKernelGGL(k_fin_rho, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part, nhd, sc);
       // r = rho_true in the sloppy precision; rho = <r0, r>; restart if broken
       II_CHECK(convertP(ctx, 0, P, q64, r, nr, skip_ru, ss));
@@ -2455,19 +2461,14 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       II_CHECK(convertP(ctx, P, P, r, r0, nr, &sc[0].keep_p, ss));
       II_CHECK(convertP(ctx, P, P, r, rp[pos], nr, &sc[0].keep_p, ss));
     }
-    II_CHECK(flush((double2*)y.v, nullptr));
+    II_CHECK(flush(&y, nullptr));
     // x_o = b_o + kappa H_oe y   (eoUtils.cpp:67)
     h = HopSpec();
     h.out_par = 1;
     h.a = kappa;
     h.xpay = true;
     h.nrhs = nr;
-    II_CHECK(hop64(ctx, h, (double2*)y.v, (double2*)t64.v, (double2*)bo.v, nullptr));
-    for (int k = 0; k < nr; ++k) {
-      double2* base = sol->data + (size_t)(rb0 + k) * 2 * he;
-      II_CHECK(copy64(ctx, base, (double2*)y.v + k * he));
-      II_CHECK(copy64(ctx, base + he, (double2*)t64.v + k * he));
-    }
+    II_CHECK(hopP(ctx, 0, h, y, xo, &bo, nullptr));
     II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     II_CHECK(read_scalars(ctx, nr));
     float ms = 0.f;
@@ -2536,8 +2537,9 @@ ii_status full_residual(ii_context* ctx, double kappa, const ii_field* src, cons
     h.coef = d + 4 * n;
     h.partials = ctx->partials;
     h.nrhs = n;
+    h.rs_in = h.rs_x = h.rs_dv = (int)(2 * he);
     II_CHECK(hop64(ctx, h, sol->data + (1 - par) * he, w, sol->data + par * he,
-                   src->data + par * he, (int)(2 * he)));
+                   src->data + par * he));
     II_CHECK(finalize_sums(ctx, ctx->partials, nblk, d + par * n, n));
   }
   // |b|^2 of every half field of the sources in one call
@@ -2779,6 +2781,13 @@ ii_status ii_propagator_solve(ii_context* ctx, double kappa, const ii_prop_param
     return set_error(ctx, II_ERR_BAD_ARG, "propagator fields must be full and of equal nrhs");
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
+  // the solution is built in place while the source is still read
+  ii_field own;
+  if (src->data == sol->data) {
+    II_CHECK(temp_field(ctx, 0, II_FULL, src->nrhs, &own));
+    II_CHECK(copy64(ctx, own.data, src->data, 2 * src->nrhs));
+    src = &own;
+  }
   // the multi-rhs hops' launch shapes for this batch, before any iteration
   // is captured in a graph (a capture keeps the shape it records)
   if (p->batched && src->nrhs > 1) {

@@ -108,6 +108,7 @@ struct StF64 {
   using C = double2;
   double2* __restrict__ p;
   int stride;
+  int rs = 0;  // elements between rhs (0: 12 * stride, back to back)
   __device__ __forceinline__ void st(int site, const C v[12]) const {
 #pragma unroll
     for (int k = 0; k < 12; ++k) st_at<double2, kNT>(p, (uint32_t)(k * stride), (uint32_t)site, v[k]);
@@ -115,7 +116,9 @@ struct StF64 {
   __device__ __forceinline__ void st1(int site, int comp, C v) const {
     st_at<double2, kNT>(p, (uint32_t)(comp * stride), (uint32_t)site, v);
   }
-  __device__ __forceinline__ StF64 rhs(int r) const { return StF64{p + (size_t)r * 12 * stride, stride}; }
+  __device__ __forceinline__ StF64 rhs(int r) const {
+    return StF64{p + (size_t)r * (rs ? rs : 12 * stride), stride, rs};
+  }
 };
 
 // FP32 half spinor, [12][stride] float2.
