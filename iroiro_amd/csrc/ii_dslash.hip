@@ -20,14 +20,27 @@
 
 namespace ii {
 
+// one component's share of the sums of kEpiGram: d, o, p
+template <typename C>
+__device__ __forceinline__ void gram_add(const C d, const C o, const C p, double* ds) {
+  const double dx = d.x, dy = d.y, ox = o.x, oy = o.y, px = p.x, py = p.y;
+  ds[0] = fma(dx, ox, fma(dy, oy, ds[0]));
+  ds[1] = fma(dx, oy, fma(-dy, ox, ds[1]));
+  ds[2] = fma(ox, ox, fma(oy, oy, ds[2]));
+  ds[3] = fma(ox, px, fma(oy, py, ds[3]));
+  ds[4] = fma(ox, py, fma(-oy, px, ds[4]));
+  ds[5] = fma(dx, px, fma(dy, py, ds[5]));
+  ds[6] = fma(dx, py, fma(-dy, px, ds[6]));
+}
+
 // The epilogue (HopEpilogue) of one site's output o of rhs-offset accessors
-// dr (the dv field) and outr; the site's partial sums go to ds[0..2].  xs
+// dr (the dv field) and outr; the site's partial sums go to ds.  xs
 // holds the XPAY term the kernel added (kEpiTS).  16- and 32-bit fields: the
 // 24-term site sums in FP32, the sums over sites in FP64.
 template <int EPI, typename R, typename C, typename SpX, typename StOut>
 __device__ __forceinline__ void hop_epilogue(C o[12], const C* xs, int hs, const SpX& dr,
                                              const StOut& outr, double alpha, double shift,
-                                             const SpX& pr, double ds[3]) {
+                                             const SpX& pr, double* ds) {
   constexpr bool kF64 = std::is_same<R, double>::value;
   if constexpr (EPI == kEpiDot) {
     if constexpr (kF64) {
@@ -103,6 +116,9 @@ __device__ __forceinline__ void hop_epilogue(C o[12], const C* xs, int hs, const
     ds[0] = (double)re;
     ds[1] = (double)im;
     ds[2] = (double)nn;
+  } else if constexpr (EPI == kEpiGram) {
+#pragma unroll
+    for (int k = 0; k < 12; ++k) gram_add<C>(dr.ld(hs, k), o[k], pr.ld(hs, k), ds);
   }
   outr.st(hs, o);
 }
@@ -121,7 +137,7 @@ k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
   const int hs = base + threadIdx.x;
   const int rhs = blockIdx.y;
   if (skip && skip[rhs * skip_stride]) return;  // uniform per block
-  double dsum[3] = {0.0, 0.0, 0.0};
+  double dsum[epi_sums(EPI) + 1] = {};
   if (hs < g.Vh) {
     const SpIn inr = in.rhs(rhs);
     C acc[4][3];
@@ -166,7 +182,7 @@ k_hop(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
 template <int EPI, typename C, typename SpX>
 __device__ __forceinline__ void hop_epilogue_spin(C o[3], const C xs[3], int hs, int spin,
                                                   const SpX& dr, double alpha, double shift,
-                                                  const SpX& p, double ds[3]) {
+                                                  const SpX& p, double* ds) {
   if constexpr (EPI == kEpiStore) return;
   using R = decltype(C::x);
 #pragma unroll
@@ -196,6 +212,7 @@ __device__ __forceinline__ void hop_epilogue_spin(C o[3], const C xs[3], int hs,
       ds[1] = fma(ox, xy, fma(-oy, xx, ds[1]));
       ds[2] = fma(ox, ox, fma(oy, oy, ds[2]));
     }
+    if constexpr (EPI == kEpiGram) gram_add<C>(dr.ld(hs, 3 * spin + c), o[c], p.ld(hs, 3 * spin + c), ds);
   }
 }
 
@@ -284,7 +301,7 @@ k_hop_split(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
       if (sig) shift = sig[0];
     }
   }
-  double dsum[3] = {0.0, 0.0, 0.0};
+  double dsum[epi_sums(EPI) + 1] = {};
   if (valid) {
     C o[3], xsv[3];
 #pragma unroll
@@ -390,7 +407,7 @@ k_hop_mrhs(Geom g, SpIn in, Gauge gauge, StOut out, SpX x, SpX dv, int out_par,
   static_assert(TS == 64, "one wavefront per rhs row");
   const int rhs = __builtin_amdgcn_readfirstlane(blockIdx.y * blockDim.y + ty);
   const bool live = rhs < nrhs && !(skip && skip[rhs * skip_stride]);
-  double dsum[3] = {0.0, 0.0, 0.0};
+  double dsum[epi_sums(EPI) + 1] = {};
   if (live && hs < g.Vh) {
     const SpIn inr = in.rhs(rhs);
     C acc[4][3];
@@ -503,8 +520,8 @@ ii_status launch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, const 
                      const SpX& x, const SpX& dv, typename SpIn::R a, const HopSpec& h) {
   const Geom& g = ctx->g;
   bool flip = ctx->tbc_sign < 0;
-  SpX px = dv;  // the shift term's field
-  if (h.sig) {
+  SpX px = dv;  // the shift term's or kEpiGram's field
+  if (h.p) {
     px.p = (decltype(px.p))h.p;
     if constexpr (SpIn::kScaled) px.nrm = h.p_nrm;
     if constexpr (std::is_same<SpX, SpF64>::value) px.rs = 0;
@@ -547,7 +564,7 @@ ii_status dispatch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, cons
                        const SpX& x, const SpX& dv, const HopSpec& h) {
   using R = typename SpIn::R;
   const R a = (R)h.a;
-  if (h.epi < kEpiStore || h.epi > kEpiTS)
+  if (h.epi < kEpiStore || h.epi > kEpiGram)
     return set_error(ctx, II_ERR_BAD_ARG, "unknown hop epilogue");
   if (h.epi == kEpiTS && !h.xpay)
     return set_error(ctx, II_ERR_BAD_ARG, "kEpiTS needs the XPAY term");
@@ -559,6 +576,15 @@ ii_status dispatch_hop(ii_context* ctx, const SpIn& in, const Gauge& gauge, cons
     return set_error(ctx, II_ERR_BAD_ARG, "bad shift term of a residual update");
   if (h.epi == kEpiRUpd && !h.coef && !h.ru.den)
     return set_error(ctx, II_ERR_BAD_ARG, "residual-update hop without its scalars");
+  if (h.epi == kEpiGram) {
+    if constexpr (std::is_same<SpX, SpF32>::value) {
+      if (!h.p || !h.xpay || h.g5in || h.g5out)
+        return set_error(ctx, II_ERR_BAD_ARG, "bad hop with inner products");
+      return launch_hop<false, false, true, kEpiGram>(ctx, in, gauge, out, x, dv, a, h);
+    } else {
+      return set_error(ctx, II_ERR_BAD_ARG, "the inner-product hop takes 32-bit fields");
+    }
+  }
   const int sel = (h.g5in ? 32 : 0) | (h.g5out ? 16 : 0) | (h.xpay ? 8 : 0) | h.epi;
 #define II_CASE(A, B, CC, E)                                                                 \
   case ((A) ? 32 : 0) | ((B) ? 16 : 0) | ((CC) ? 8 : 0) | (E):                               \

@@ -21,10 +21,14 @@ namespace ii {
 //              (re, im)                             (BiCGStab <r0, A p>)
 //   kEpiTS     XPAY only: store o; partial sums of the complex <o, x> and of
 //              |o|^2 from the x it adds             (BiCGStab omega = <t, s>/|t|^2)
+//   kEpiGram   32-bit fields, XPAY only: store o; the seven real sums of <dv, o>,
+//              |o|^2, <o, p> and <dv, p> (re, im; p: HopSpec::p), FP64 from the
+//              stored values on                     (flexible GCR, window 1)
 // Several sums are stored as planes: sum j of (rhs, block) at
 // partials[j * plane + rhs * nblocks + block], plane = nrhs * nblocks.
 enum HopEpilogue {
-  kEpiStore = 0, kEpiDot = 1, kEpiNorm = 2, kEpiRUpd = 3, kEpiCDot = 4, kEpiTS = 5
+  kEpiStore = 0, kEpiDot = 1, kEpiNorm = 2, kEpiRUpd = 3, kEpiCDot = 4, kEpiTS = 5,
+  kEpiGram = 6
 };
 // Single-rhs FP64 / FP32 hops also take kEpiRUpd with the scalar and a shift
 // folded in (HopSpec::ru):
@@ -42,7 +46,9 @@ struct RUpdFold {
   double* alpha = nullptr;
   const void* p = nullptr;       // the field of the shift term, in the hop's precision
 };
-constexpr int epi_sums(int epi) { return epi == kEpiStore ? 0 : epi == kEpiCDot ? 2 : epi == kEpiTS ? 3 : 1; }
+constexpr int epi_sums(int epi) {
+  return epi == kEpiStore ? 0 : epi == kEpiCDot ? 2 : epi == kEpiTS ? 3 : epi == kEpiGram ? 7 : 1;
+}
 
 struct HopSpec {
   int out_par = 0;
