@@ -1385,7 +1385,18 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   const Geom& g = ctx->g;
   if (P != II_PREC_DOUBLE && !ctx->gauge_lp[P]) II_CHECK(build_lowprec_gauge(ctx, P));
   const bool lo = P != II_PREC_DOUBLE;
-  const double delta = lo ? 0.1 : 0.0;
+  // A reliable update costs four FP64 hops of every rhs it takes, twice an
+  // iteration's time in FP16, and two decades between updates stay above the
+  // rounding of FP32 and FP16 directions (2^-11): 10 shifts at kappa 0.1265,
+  // delta 0.1 / 0.05 / 0.03 / 0.01 / 0.003: 54.2 / 51.5 / 50.7 / 47.3 / 48.1 ms
+  // (FP16, 24^3x48), 65.5 / 62.9 / 61.9 / 58.6 / 58.1 ms (FP32).  BF16
+  // (2^-8) keeps one decade.  The queued iterations may pass the trigger by
+  // far more than delta, until the recursion's r is mostly rounding: an update
+  // that finds |rho|^2 above 1.5 |r|^2 (1.0002 while it is sound) restarts the
+  // direction.  With the propagator's factor 16 a shift at 2.1 kept its
+  // direction and diverged (FP16, delta 0.003).
+  const double delta = !lo ? 0.0 : P == II_PREC_BF16 ? 0.1 : 0.01;
+  const double restart = lo ? 1.5 : 16.0;
   const int nb = hop_blocks(g), nh = hop_dot_parts(g, nrhs, P);
   const int nhd = hop_dot_parts(g, nrhs, II_PREC_DOUBLE);
   const size_t np = (size_t)std::max(std::max(nb, nh), nhd) * nrhs;
@@ -1479,7 +1490,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   II_CHECK(residual(nullptr, 0));
   II_CHECK(finalize_sums(ctx, part, nhd, rr0, nrhs));
   hipLaunchKernelGGL(k_scal_init, dim3(nrhs), dim3(64), 0, ctx->stream, sc, rr0, bb, 0.0, tol,
-                     delta, 1);
+                     delta, 1, restart);
   II_HIP(ctx, hipGetLastError());
   int pos = 0;            // ring slot of the current search directions
   std::vector<int> pend;  // ring slots whose alpha p is not yet in ys
