@@ -25,12 +25,14 @@ namespace {
 
 constexpr int kPipeThreads = 2;
 constexpr size_t kPieceMax = (size_t)4 << 20;    // bytes of a slot
-constexpr size_t kPieceMin = (size_t)128 << 10;
 constexpr size_t kThreadBytes = (size_t)4 << 20; // a second thread from twice that: it takes
                                                  // about 50 us to start
-// Smaller copies are the runtime's: it writes them through its own staging
-// without a second engine (one Dhat at 4^3x8, 49 KB each way: 48 against 61 us).
-constexpr size_t kDirect = (size_t)64 << 10;
+// Smaller copies are the runtime's: its own staging has less latency than a
+// slot and its event.  One Dhat on host arrays, us, through the runtime /
+// through the slots, by the bytes each way: 72 KB 52 / 63, 243 KB 65 / 100,
+// 768 KB 106 / 130, 1152 KB 165 / 152, 2.6 MB 287 / 260, 8.2 MB 632 / 620 (823
+// before).
+constexpr size_t kDirect = (size_t)1 << 20;
 
 }  // namespace
 
@@ -89,7 +91,7 @@ static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
   const int want = (int)std::max<size_t>(1, bytes / kThreadBytes);
   const int nthr = std::min(kPipeThreads, want);
   size_t piece = (bytes + 2 * nthr - 1) / (2 * nthr);
-  piece = std::min(kPieceMax, std::max(kPieceMin, (piece + 4095) / 4096 * 4096));
+  piece = std::min(kPieceMax, (piece + 4095) / 4096 * 4096);
   const size_t n = (bytes + piece - 1) / piece;
   std::atomic<size_t> next{0};
   std::atomic<int> err{hipSuccess};
