@@ -39,8 +39,10 @@ constexpr size_t kDirect = (size_t)1 << 20;
 // The pinned slots of a device, 16 MiB, shared by its contexts (pinning them
 // takes about 10 ms, which every context would pay): allocated at the first
 // copy that needs them, freed with the last context that used them.  A copy
-// holds `mu` throughout; a slot whose piece is still on its way to the device,
-// on whichever context's stream, is waited for through its event.
+// holds `mu` throughout.  An upload returns with its last pieces still on their
+// way from the slots, on its context's stream: the next user of a slot waits
+// for the slot's event, an upload on the host before it fills the slot, a
+// download on its stream before the device does.
 struct HostPipe {
   std::mutex mu;
   char* pin = nullptr;
@@ -83,9 +85,9 @@ static ii_status host_pipe(ii_context* ctx, HostPipe* H) {
   return II_OK;
 }
 
-// Runs piece(thread, slot, first, bytes) over [0, bytes); the pieces of one
-// thread come in order and alternate between its two slots.  done(slot) waits
-// for a slot whose device side is pending.
+// Runs work(t, take, e) on each thread t: take(&first, &bytes) hands out the
+// pieces of [0, bytes) in order until none is left or a thread has failed, e is
+// the thread's error.  After a failure nothing of the copy is left in flight.
 template <typename Piece>
 static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
   const int want = (int)std::max<size_t>(1, bytes / kThreadBytes);
@@ -114,9 +116,11 @@ static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
   }
   run(0);
   for (auto& h : helpers) h.join();
-  if (err != hipSuccess)
+  if (err != hipSuccess) {
+    (void)hipStreamSynchronize(ctx->stream);
     return set_error(ctx, II_ERR_DEVICE,
                      std::string("host copy: ") + hipGetErrorString((hipError_t)err.load()));
+  }
   return II_OK;
 }
 
@@ -154,12 +158,15 @@ ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes
   II_CHECK(host_pipe(ctx, H));
   return run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first[2] = {0, 0}, len[2] = {0, 0};
+    bool used[2] = {false, false};  // by this call, whose pieces the stream keeps in order
     auto request = [&](int b) {
       const int slot = 2 * t + b;
       len[b] = 0;
       size_t f = 0, l = 0;
       if (!take(&f, &l)) return;
       first[b] = f;
+      if (!used[b] && (e = hipStreamWaitEvent(ctx->stream, H->ev[slot], 0)) != hipSuccess) return;
+      used[b] = true;
       if ((e = hipMemcpyAsync(H->pin + slot * kPieceMax, (const char*)src + f, l,
                               hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess)
         return;

@@ -24,3 +24,32 @@ def test_field_and_gauge_round_trip(dims):
     ctx.upload_gauge(u)
     assert np.array_equal(ctx.download_gauge(), u)
     ctx.close()
+
+
+def test_two_contexts_of_a_device_copying_at_once():
+    """An upload of one context beside another context's download, each in a
+    thread of its own, byte for byte; the slots given up by both and taken
+    again."""
+    import threading
+    dims = (14, 10, 12, 18)  # 5.8 MB a field
+    for _ in range(2):
+        ctxs = [ii.Context(dims) for _ in range(2)]
+        bad = []
+
+        def work(k):
+            rng = np.random.default_rng(10 + k)
+            f = ii.DeviceField(ctxs[k], "full", 1)
+            for i in range(8):
+                a = rng.normal(size=f.size)
+                f.upload(0, a)
+                if not np.array_equal(f.download(0), a):
+                    bad.append((k, i))
+
+        ts = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        for c in ctxs:
+            c.close()
+        assert not bad
