@@ -15,6 +15,7 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -36,53 +37,107 @@ constexpr size_t kDirect = (size_t)1 << 20;
 
 }  // namespace
 
-// The pinned slots of a device, 16 MiB, shared by its contexts (pinning them
-// takes about 10 ms, which every context would pay): allocated at the first
-// copy that needs them, freed with the last context that used them.  A copy
-// holds `mu` throughout.  An upload returns with its last pieces still on their
-// way from the slots, on its context's stream: the next user of a slot waits
-// for the slot's event, an upload on the host before it fills the slot, a
-// download on its stream before the device does.
-struct HostPipe {
-  std::mutex mu;
+// A set of pinned slots, 16 MiB.  Pinning one takes about 10 ms, so the sets
+// belong to the device and not to a context: a copy takes the set its context
+// used last, else one with nothing in flight, else pins a new one.  So a copy
+// never waits for another context's kernels or copies, its own stream orders
+// the uses of a set in flight, and there are never more sets than contexts
+// that copy: programs that use their contexts one after the other pin one.
+struct HostSet {
   char* pin = nullptr;
   hipEvent_t ev[2 * kPipeThreads] = {};
-  int users = 0;
-  void free_slots() {
-    for (auto& e : ev) {
-      if (e) (void)hipEventDestroy(e);
-      e = nullptr;
-    }
-    if (pin) (void)hipHostFree(pin);
-    pin = nullptr;
+  ii_context* owner = nullptr;  // whose stream may have pieces in flight
+  bool busy = false;            // a copy is running on it
+  HostSet* next = nullptr;
+  bool create() {
+    bool ok = hipHostMalloc((void**)&pin, 2 * kPipeThreads * kPieceMax) == hipSuccess;
+    for (auto& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    return ok;
   }
+  bool complete() const {
+    for (auto& e : ev)
+      if (hipEventQuery(e) != hipSuccess) {
+        (void)hipGetLastError();  // not ready is no error of the caller's launches
+        return false;
+      }
+    return true;
+  }
+  ~HostSet() {
+    for (auto& e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (pin) (void)hipHostFree(pin);
+  }
+};
+struct HostPipe {
+  std::mutex mu;  // over the list, never held while a copy or a kernel runs
+  HostSet* sets = nullptr;
+  int nsets = 0, users = 0;  // users: contexts that have copied
 };
 constexpr int kPipeDevices = 64;  // as many as noalloc_setup lets a context be created on
 static HostPipe g_pipe[kPipeDevices];
 
+// frees the sets beyond the number of contexts that may use one (mu held)
+static void trim(HostPipe* H) {
+  for (HostSet** at = &H->sets; *at && H->nsets > H->users;) {
+    HostSet* s = *at;
+    if (s->busy || (s->owner && !s->complete())) {
+      at = &s->next;
+      continue;
+    }
+    *at = s->next;
+    --H->nsets;
+    delete s;
+  }
+}
+
+// The stream of a context that goes has been waited for.
 void host_pipe_release(ii_context* ctx) {
   HostPipe* H = static_cast<HostPipe*>(ctx->host_pipe);
   if (!H) return;
   std::lock_guard<std::mutex> lock(H->mu);
-  if (--H->users == 0) H->free_slots();
+  for (HostSet* s = H->sets; s; s = s->next)
+    if (s->owner == ctx) s->owner = nullptr;
+  --H->users;
+  trim(H);
   ctx->host_pipe = nullptr;
 }
 
-// the device's slots, H->mu held
-static ii_status host_pipe(ii_context* ctx, HostPipe* H) {
-  if (ctx->host_pipe) return II_OK;
-  if (!H->pin) {
-    bool ok = hipHostMalloc((void**)&H->pin, 2 * kPipeThreads * kPieceMax) == hipSuccess;
-    for (auto& e : H->ev)
-      ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-      H->free_slots();
-      return set_error(ctx, II_ERR_DEVICE, "pinned staging memory");
+// a set for one copy of ctx, null if none can be pinned
+static HostSet* take_set(ii_context* ctx) {
+  HostPipe* H = &g_pipe[ctx->device];
+  HostSet* s = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(H->mu);
+    if (!ctx->host_pipe) {
+      ++H->users;
+      ctx->host_pipe = H;
+    }
+    for (s = H->sets; s && (s->busy || s->owner != ctx);) s = s->next;
+    if (!s)
+      for (s = H->sets; s && (s->busy || !s->complete());) s = s->next;
+    if (s) {
+      s->owner = ctx;
+      s->busy = true;
+      return s;
     }
   }
-  ++H->users;
-  ctx->host_pipe = H;
-  return II_OK;
+  s = new (std::nothrow) HostSet();  // pinned outside the lock
+  if (!s || !s->create()) {
+    delete s;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  s->owner = ctx;
+  s->busy = true;
+  std::lock_guard<std::mutex> lock(H->mu);
+  s->next = H->sets;
+  H->sets = s;
+  ++H->nsets;
+  return s;
+}
+static void give_set(ii_context* ctx, HostSet* s) {
+  std::lock_guard<std::mutex> lock(static_cast<HostPipe*>(ctx->host_pipe)->mu);
+  s->busy = false;
 }
 
 // Runs work(t, take, e) on each thread t: take(&first, &bytes) hands out the
@@ -129,10 +184,9 @@ ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t byt
     II_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return II_OK;
   }
-  HostPipe* H = &g_pipe[ctx->device];
-  std::lock_guard<std::mutex> lock(H->mu);
-  II_CHECK(host_pipe(ctx, H));
-  return run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
+  HostSet* H = take_set(ctx);
+  if (!H) return set_error(ctx, II_ERR_DEVICE, "pinned staging memory");
+  const ii_status st = run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first = 0, len = 0;
     for (int i = 0; take(&first, &len); ++i) {
       const int slot = 2 * t + (i & 1);
@@ -145,6 +199,8 @@ ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t byt
       if ((e = hipEventRecord(H->ev[slot], ctx->stream)) != hipSuccess) return;
     }
   });
+  give_set(ctx, H);
+  return st;
 }
 
 ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes) {
@@ -153,20 +209,16 @@ ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return II_OK;
   }
-  HostPipe* H = &g_pipe[ctx->device];
-  std::lock_guard<std::mutex> lock(H->mu);
-  II_CHECK(host_pipe(ctx, H));
-  return run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
+  HostSet* H = take_set(ctx);
+  if (!H) return set_error(ctx, II_ERR_DEVICE, "pinned staging memory");
+  const ii_status st = run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first[2] = {0, 0}, len[2] = {0, 0};
-    bool used[2] = {false, false};  // by this call, whose pieces the stream keeps in order
     auto request = [&](int b) {
       const int slot = 2 * t + b;
       len[b] = 0;
       size_t f = 0, l = 0;
       if (!take(&f, &l)) return;
       first[b] = f;
-      if (!used[b] && (e = hipStreamWaitEvent(ctx->stream, H->ev[slot], 0)) != hipSuccess) return;
-      used[b] = true;
       if ((e = hipMemcpyAsync(H->pin + slot * kPieceMax, (const char*)src + f, l,
                               hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess)
         return;
@@ -180,6 +232,8 @@ ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes
       std::memcpy((char*)dst + first[b], H->pin + slot * kPieceMax, len[b]);
     }
   });
+  give_set(ctx, H);
+  return st;
 }
 
 }  // namespace ii

@@ -101,7 +101,7 @@ struct ii_context {
   int nscal = 0;
   void* host_pin = nullptr;       // pinned host block of the multishift scalars
   size_t host_pin_len = 0;
-  void* host_pipe = nullptr;      // the device's pinned slots, once used (ii_hostcopy.hip)
+  void* host_pipe = nullptr;      // the device's pinned slots, once copied with (ii_hostcopy.hip)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // autotuned launch shapes
   ii::HopOrder hop_order;

@@ -258,6 +258,63 @@ void threads() {
   for (auto& t : th) t.join();
 }
 
+// While A's stream is held by a kernel, with an upload queued behind it or a
+// download waiting for it, B's copies run: none waits for another's kernels.
+void no_waiting() {
+  const size_t n = 12 << 20;
+  for (int down = 0; down < 2; ++down) {
+    Ctx a, b;
+    sim::Mark gate, done;
+    std::vector<char> src = pattern(n, 7), da(n), ha(n), db(n), hb(n);
+    upload(b, db, src);
+    upload(a, da, src);  // both have copied before
+    a.s.push([&] { gate.wait(); });
+    std::thread ta([&] {
+      if (down) download(a, ha, da);
+      else upload(a, da, src);
+    });
+    std::this_thread::sleep_for(std::chrono::milliseconds(20));
+    std::thread tb([&] {
+      upload(b, db, src);
+      download(b, hb, db);
+      done.set();
+    });
+    bool ok = false;
+    {
+      std::unique_lock<std::mutex> l(done.mu);
+      ok = done.cv.wait_for(l, std::chrono::seconds(20), [&] { return done.done; });
+    }
+    CHECK(ok, "a context waits for another one's kernel (%s)", down ? "its download" : "its upload");
+    CHECK(hb == src, "copies beside a held stream");
+    gate.set();
+    ta.join();
+    tb.join();
+  }
+}
+
+// as many sets of slots as contexts with copies in flight, and one for
+// contexts used in turn
+void set_count() {
+  const int before = sim::pin_calls;
+  {
+    Ctx a, b, c;
+    std::vector<char> src = pattern(12 << 20, 8), dev(src.size()), dst(src.size());
+    for (int i = 0; i < 3; ++i)
+      for (Ctx* x : {&a, &b, &c}) {
+        upload(*x, dev, src);
+        download(*x, dst, dev);
+      }
+    CHECK(sim::pin_calls == before + 1, "contexts in turn pinned %d sets", sim::pin_calls - before);
+    for (Ctx* x : {&a, &b, &c}) {
+      x->kernel(30);
+      upload(*x, dev, src);
+    }
+    for (Ctx* x : {&a, &b, &c}) x->s.sync();
+    CHECK(sim::pins <= 3, "three contexts pinned %d sets", (int)sim::pins);
+  }
+  CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
+}
+
 // a copy that fails leaves nothing of its own in flight, and the next is right
 void failures() {
   Ctx a, b;
@@ -283,6 +340,8 @@ int main() {
   round_trips();
   other_context();
   threads();
+  no_waiting();
+  set_count();
   failures();
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
   round_trips();  // the slots come back after the last context gave them up
