@@ -95,6 +95,7 @@ struct Event {
 };
 
 std::atomic<int> pins{0}, pin_calls{0}, fail_copy{-1}, copies{0};
+const char *pinned_lo = nullptr, *pinned_hi = nullptr;  // the caller's pinned memory
 
 Stream* of(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
 Event* of(hipEvent_t e) { return reinterpret_cast<Event*>(e); }
@@ -153,6 +154,11 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
   if (sim::fail_copy >= 0 && sim::fail_copy-- == 0) return hipErrorUnknown;
   ++sim::copies;
   sim::of(st)->push([=] { std::memcpy(d, s, n); });
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  if (p < sim::pinned_lo || p >= sim::pinned_hi) return hipErrorInvalidValue;
+  a->type = hipMemoryTypeHost;
   return hipSuccess;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
@@ -292,6 +298,24 @@ void no_waiting() {
   }
 }
 
+// a caller's pinned memory: one copy each way, between it and the device
+void pinned_memory() {
+  Ctx a;
+  for (size_t n : kSizes) {
+    std::vector<char> src = pattern(n, 9), keep = src, dev(n);
+    sim::pinned_lo = src.data();
+    sim::pinned_hi = src.data() + n;
+    a.kernel(2);
+    const int before = sim::copies;
+    upload(a, dev, src);
+    std::fill(src.begin(), src.end(), 0);
+    download(a, src, dev);
+    CHECK(src == keep, "pinned round trip of %zu bytes", n);
+    CHECK(sim::copies == before + 2, "%d copies of pinned memory", sim::copies - before);
+    sim::pinned_lo = sim::pinned_hi = nullptr;
+  }
+}
+
 // as many sets of slots as contexts with copies in flight, and one for
 // contexts used in turn
 void set_count() {
@@ -341,6 +365,7 @@ int main() {
   other_context();
   threads();
   no_waiting();
+  pinned_memory();
   set_count();
   failures();
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
