@@ -14,17 +14,16 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace ii {
 
 namespace {
 
-constexpr int kPipeThreads = 2;
+constexpr int kPipeThreads = 2;                  // this one and a helper
 constexpr size_t kPieceMax = (size_t)4 << 20;    // bytes of a slot
 constexpr size_t kThreadBytes = (size_t)4 << 20; // a second thread from twice that: it takes
                                                  // about 50 us to start
@@ -102,7 +101,8 @@ void host_pipe_release(ii_context* ctx) {
   ctx->host_pipe = nullptr;
 }
 
-// a set for one copy of ctx, null if none can be pinned
+// a set for one copy of ctx; null if none can be pinned (the copy is the
+// runtime's then)
 static HostSet* take_set(ii_context* ctx) {
   HostPipe* H = &g_pipe[ctx->device];
   HostSet* s = nullptr;
@@ -163,14 +163,14 @@ static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
     }, e);
     if (e != hipSuccess) err = e;
   };
-  std::vector<std::thread> helpers;
-  try {
-    for (int t = 1; t < nthr; ++t) helpers.emplace_back(run, t);
-  } catch (const std::system_error&) {
-    // no more threads: those that started, and this one, share the pieces
-  }
+  std::thread helper;
+  if (nthr > 1) try {
+      helper = std::thread(run, 1);
+    } catch (const std::exception&) {
+      // no thread to be had: this one takes all the pieces
+    }
   run(0);
-  for (auto& h : helpers) h.join();
+  if (helper.joinable()) helper.join();
   if (err != hipSuccess) {
     (void)hipStreamSynchronize(ctx->stream);
     return set_error(ctx, II_ERR_DEVICE,
@@ -190,13 +190,12 @@ static bool pageable(const void* p) {
 }
 
 ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t bytes) {
-  if (bytes < kDirect || !pageable(src)) {
+  HostSet* H = bytes < kDirect || !pageable(src) ? nullptr : take_set(ctx);
+  if (!H) {
     II_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     if (bytes >= kDirect) II_HIP(ctx, hipStreamSynchronize(ctx->stream));  // src has been read
     return II_OK;
   }
-  HostSet* H = take_set(ctx);
-  if (!H) return set_error(ctx, II_ERR_DEVICE, "pinned staging memory");
   const ii_status st = run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first = 0, len = 0;
     for (int i = 0; take(&first, &len); ++i) {
@@ -215,13 +214,12 @@ ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t byt
 }
 
 ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes) {
-  if (bytes < kDirect || !pageable(dst)) {
+  HostSet* H = bytes < kDirect || !pageable(dst) ? nullptr : take_set(ctx);
+  if (!H) {
     II_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return II_OK;
   }
-  HostSet* H = take_set(ctx);
-  if (!H) return set_error(ctx, II_ERR_DEVICE, "pinned staging memory");
   const ii_status st = run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first[2] = {0, 0}, len[2] = {0, 0};
     auto request = [&](int b) {

@@ -13,6 +13,7 @@
 #include <deque>
 #include <functional>
 #include <memory>
+#include <vector>
 
 #define CHECK(c, ...)                                        \
   do {                                                       \
@@ -95,6 +96,7 @@ struct Event {
 };
 
 std::atomic<int> pins{0}, pin_calls{0}, fail_copy{-1}, copies{0};
+std::atomic<bool> no_pins{false};
 const char *pinned_lo = nullptr, *pinned_hi = nullptr;  // the caller's pinned memory
 
 Stream* of(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
@@ -105,6 +107,7 @@ Event* of(hipEvent_t e) { return reinterpret_cast<Event*>(e); }
 extern "C" {
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (sim::no_pins) return hipErrorOutOfMemory;
   ++sim::pin_calls;
   *p = std::malloc(n);
   ++sim::pins;
@@ -366,6 +369,10 @@ int main() {
   threads();
   no_waiting();
   pinned_memory();
+  sim::no_pins = true;  // copies without slots are the runtime's
+  round_trips();
+  other_context();
+  sim::no_pins = false;
   set_count();
   failures();
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
