@@ -82,15 +82,28 @@ ii_status copy64(ii_context* ctx, double2* dst, const double2* src, int nrhs) {
 }
 
 __global__ void __launch_bounds__(kBlock)
-k_zero64(double2* __restrict__ dst, size_t n, size_t rs) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[blockIdx.y * rs + i] = make_double2(0.0, 0.0);
+k_zero64(double2* __restrict__ y, size_t n) {
+  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i] = make_double2(0.0, 0.0);
 }
 
-ii_status zero64(ii_context* ctx, double2* dst, int nrhs, int rs) {
+ii_status zero64(ii_context* ctx, double2* dst, int nrhs) {
+  size_t n = half_elems(ctx->g) * nrhs;
+  hipLaunchKernelGGL(k_zero64, dim3(blocks_for((long)n)), dim3(kBlock), 0, ctx->stream, dst, n);
+  II_HIP(ctx, hipGetLastError());
+  return II_OK;
+}
+
+__global__ void __launch_bounds__(kBlock)
+k_copy_rhs64(double2* __restrict__ dst, size_t rs, const double2* __restrict__ src, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[blockIdx.y * rs + i] = src[blockIdx.y * n + i];
+}
+
+ii_status copy_rhs64(ii_context* ctx, double2* dst, size_t rs, const double2* src, int nrhs) {
   const size_t n = half_elems(ctx->g);
-  hipLaunchKernelGGL(k_zero64, dim3(blocks_for((long)n), nrhs), dim3(kBlock), 0, ctx->stream, dst,
-                     n, rs ? (size_t)rs : n);
+  hipLaunchKernelGGL(k_copy_rhs64, dim3(blocks_for((long)n), nrhs), dim3(kBlock), 0, ctx->stream,
+                     dst, rs, src, n);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
 }

@@ -380,7 +380,7 @@ __global__ void k_g_coef(int m, GScal* __restrict__ gs) {
 // written for it)
 __global__ void __launch_bounds__(kGThreads)
 k_g_fold(Geom g, const float2* __restrict__ Z, size_t slot, int mm, double2* __restrict__ y,
-         size_t yrs, const GScal* __restrict__ gs) {
+         const GScal* __restrict__ gs) {
   const int rhs = blockIdx.y;
   const GScal& S = gs[rhs];
   if (S.done) return;
@@ -395,7 +395,7 @@ k_g_fold(Geom g, const float2* __restrict__ Z, size_t slot, int mm, double2* __r
     gi[i] = i < m ? S.gamma[i][1] : 0.0;
   }
   for (int c = 0; c < 12; ++c) {
-    double2 v = y[rhs * yrs + (size_t)c * g.stride + hs];
+    double2 v = y[rhs * he + (size_t)c * g.stride + hs];
 #pragma unroll
     for (int i = 0; i < kMaxK; ++i)
       if (i < m) {
@@ -403,7 +403,7 @@ k_g_fold(Geom g, const float2* __restrict__ Z, size_t slot, int mm, double2* __r
         v.x += gr[i] * a.x - gi[i] * a.y;
         v.y += gr[i] * a.y + gi[i] * a.x;
       }
-    y[rhs * yrs + (size_t)c * g.stride + hs] = v;
+    y[rhs * he + (size_t)c * g.stride + hs] = v;
   }
 }
 
@@ -484,7 +484,7 @@ struct Buf {
   size_t n = 0;
 };
 struct FGState {
-  Buf Z, W, R, Rb, T, bh, rho, t64, part, gs, aux;
+  Buf Z, W, R, Rb, T, y, bh, rho, t64, part, gs, aux;
   GScal* host = nullptr;
   int host_n = 0;
 };
@@ -505,7 +505,7 @@ ii_status grow(ii_context* ctx, Buf& b, size_t bytes) {
 void fgcr_release(void* p) {
   FGState* s = static_cast<FGState*>(p);
   if (!s) return;
-  for (Buf* b : {&s->Z, &s->W, &s->R, &s->Rb, &s->T, &s->bh, &s->rho, &s->t64,
+  for (Buf* b : {&s->Z, &s->W, &s->R, &s->Rb, &s->T, &s->y, &s->bh, &s->rho, &s->t64,
                  &s->part, &s->gs, &s->aux})
     if (b->p) (void)hipFree(b->p);
   if (s->host) (void)hipHostFree(s->host);
@@ -534,7 +534,7 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   II_CHECK(grow(ctx, S.R, slot * sizeof(float2)));
   if (use_net) II_CHECK(grow(ctx, S.Rb, (size_t)nr * g.stride * 12 * sizeof(uint32_t)));
   II_CHECK(grow(ctx, S.T, slot * sizeof(float2)));
-  for (Buf* b : {&S.bh, &S.rho, &S.t64})
+  for (Buf* b : {&S.y, &S.bh, &S.rho, &S.t64})
     II_CHECK(grow(ctx, *b, nr * he * sizeof(double2)));
   const int nbs = blocks_for(g.Vh, kGThreads);
   const int nbh = hop_dot_parts(g, nr, II_PREC_DOUBLE);
@@ -556,10 +556,12 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   float2* R = (float2*)S.R.p;
   uint32_t* Rb = use_net ? (uint32_t*)S.Rb.p : nullptr;  // r as the network's bf16 input
   float2* T = (float2*)S.T.p;
-  // the sources' parities are read and the solution's written in place
+  // the sources' parities are read in place; the even solution y is formed
+  // beside sol, which is written when the solve has ended (a solve that fails
+  // leaves it as it was)
   const int prs = (int)(2 * he);  // elements between the rhs of one parity
   const double2 *be = src->data, *bo = src->data + he;
-  double2 *y = sol->data, *xo = sol->data + he, *bh = (double2*)S.bh.p,
+  double2 *y = (double2*)S.y.p, *bh = (double2*)S.bh.p,
           *rho = (double2*)S.rho.p, *t64 = (double2*)S.t64.p;
   double* part = (double*)S.part.p;
   GScal* gs = (GScal*)S.gs.p;
@@ -598,7 +600,7 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   }
   hipLaunchKernelGGL(k_g_init, dim3((nr + 63) / 64), dim3(64), 0, ctx->stream, aux, aux + 2 * nr,
                      tol, nr, gs);
-  II_CHECK(zero64(ctx, y, nr, prs));
+  II_CHECK(zero64(ctx, y, nr));
   hipLaunchKernelGGL(k_g_to32, sgrid, dim3(kGThreads), 0, ctx->stream, g, bh, R, Rb, gs);
   II_HIP(ctx, hipGetLastError());
 
@@ -653,15 +655,13 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
       II_HIP(ctx, hipGetLastError());
     }
     hipLaunchKernelGGL(k_g_coef, dim3(nr), dim3(64), 0, ctx->stream, m, gs);
-    hipLaunchKernelGGL(k_g_fold, sgrid, dim3(kGThreads), 0, ctx->stream, g, Z, slot, m, y,
-                       (size_t)prs, gs);
+    hipLaunchKernelGGL(k_g_fold, sgrid, dim3(kGThreads), 0, ctx->stream, g, Z, slot, m, y, gs);
     // rho = bhat - Dhat y (FP64) with |rho|^2 in the second hop's epilogue
     HopSpec b;
     b.nrhs = nr;
     b.skip = donef;
     b.skip_stride = kGInts;
     b.out_par = 1;
-    b.rs_in = prs;
     II_CHECK(hop64(ctx, b, y, t64, nullptr, nullptr));
     b.out_par = 0;
     b.a = -kappa * kappa;
@@ -670,8 +670,6 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
     b.coef = one;
     b.coef_stride = 0;
     b.partials = part;
-    b.rs_in = 0;
-    b.rs_x = prs;
     II_CHECK(hop64(ctx, b, t64, rho, y, bh));
     hipLaunchKernelGGL(k_g_rho, dim3(nr), dim3(1024), 0, ctx->stream, part, nbh, gs);
     hipLaunchKernelGGL(k_g_to32, sgrid, dim3(kGThreads), 0, ctx->stream, g, rho, R, Rb, gs);
@@ -757,7 +755,7 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
     II_CHECK(propagator(ctx, kappa, &fp, &tmp_src, &tmp_sol, fo.data()));
     for (int k = 0; k < nr; ++k)
       if (!S.host[k].done) {
-        II_CHECK(axpby64(ctx, 1.0, tmp_sol.data + (size_t)k * 2 * he, 1.0, y + (size_t)k * prs));
+        II_CHECK(axpby64(ctx, 1.0, tmp_sol.data + (size_t)k * 2 * he, 1.0, y + k * he));
         fb_its = std::max(fb_its, fo[k].iterations);
       }
     (void)stalled;
@@ -768,8 +766,9 @@ ii_status fgcr_batched(ii_context* ctx, void** state, double kappa, const ii_pro
   h.a = kappa;
   h.xpay = true;
   h.nrhs = nr;
-  h.rs_in = h.rs_out = h.rs_x = prs;
-  II_CHECK(hop64(ctx, h, y, xo, bo, nullptr));
+  h.rs_out = h.rs_x = prs;
+  II_CHECK(hop64(ctx, h, y, sol->data + he, bo, nullptr));
+  II_CHECK(copy_rhs64(ctx, sol->data, prs, y, nr));
   II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
   II_HIP(ctx, hipMemcpyAsync(S.host, gs, sizeof(GScal) * nr, hipMemcpyDeviceToHost, ctx->stream));
   II_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -129,8 +129,9 @@ ii_status ddagd64(ii_context* ctx, double kappa, const double2* f, double2* out,
 ii_status dot64(ii_context* ctx, const double2* a, const double2* b, double* dst, int nrhs = 1);
 ii_status finalize_sums(ii_context* ctx, const double* partials, int nblk, double* dst, int nrhs);
 ii_status copy64(ii_context* ctx, double2* dst, const double2* src, int nrhs = 1);
-// rs: elements between the rhs (0: back to back)
-ii_status zero64(ii_context* ctx, double2* dst, int nrhs = 1, int rs = 0);
+ii_status zero64(ii_context* ctx, double2* dst, int nrhs = 1);
+// nrhs half fields back to back into dst, rs elements between its rhs
+ii_status copy_rhs64(ii_context* ctx, double2* dst, size_t rs, const double2* src, int nrhs);
 // y = a*x + b*y with host scalars
 ii_status axpby64(ii_context* ctx, double a, const double2* x, double b, double2* y, int nrhs = 1);
 ii_status gamma5_64(ii_context* ctx, const double2* in, double2* out, int nrhs = 1);

@@ -246,8 +246,7 @@ struct DeferredDirs {
 template <typename SpP, typename SpY, typename StY>
 __global__ void __launch_bounds__(kBlock)
 k_cg_flush(Geom g, DeferredDirs<SpP> d, const double* __restrict__ ahist, int astride, SpY yr,
-           StY yw, double2* __restrict__ y64, size_t y64_rs, const int* __restrict__ skip,
-           int skip_stride) {
+           StY yw, double2* __restrict__ y64, const int* __restrict__ skip, int skip_stride) {
   const int rhs = blockIdx.y;
   const int hs = blockIdx.x * blockDim.x + threadIdx.x;
   if (hs >= g.Vh) return;
@@ -267,7 +266,7 @@ k_cg_flush(Geom g, DeferredDirs<SpP> d, const double* __restrict__ ahist, int as
     }
   }
   if (fold) {
-    double2* y = y64 + (size_t)rhs * y64_rs;
+    double2* y = y64 + (size_t)rhs * 12 * g.stride;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
       double2 o = y[(size_t)k * g.stride + hs];
@@ -485,11 +484,6 @@ ii_status ddagd_cg_fused(ii_context* ctx, int P, double kappa, const SF& p, cons
   return hopP(ctx, P, h, t, r, &q, &r);  // r -= alpha Dhat^dag q, |r|^2
 }
 
-// elements between the rhs of the FP64 field a flush folds into
-size_t fold_stride(const Geom& g, const SF* y) {
-  return y && y->rs ? (size_t)y->rs : (size_t)12 * g.stride;
-}
-
 // y += alpha p; r -= alpha s; |r|^2 partials, FP64
 ii_status cg_blas64(ii_context* ctx, const SF& p, const SF& s, const SF& r, const SF& y,
                     RUScal* sc, int nrhs, double* partials, int nb) {
@@ -522,7 +516,7 @@ ii_status cg_p_update(ii_context* ctx, const SF& r, const SF& p, const SF& pout,
 // y64, also fold into y64 (rhs not masked by skip)
 template <int P>
 ii_status cg_flush(ii_context* ctx, const SF* ring, const int* slots, int n, const double* ahist,
-                   int astride, const SF& y, int nrhs, const SF* y64, const int* skip,
+                   int astride, const SF& y, int nrhs, double2* y64, const int* skip,
                    int skip_stride) {
   const Geom& g = ctx->g;
   using A = Acc<P>;
@@ -536,7 +530,7 @@ ii_status cg_flush(ii_context* ctx, const SF* ring, const int* slots, int n, con
   hipLaunchKernelGGL((k_cg_flush<typename A::Sp, SpF32, StF32>), dim3(blocks_for(g.Vh), nrhs),
                      dim3(kBlock), 0, ctx->stream, g, d, ahist, astride,
                      Acc<II_PREC_SINGLE>::sp(y, g.stride), Acc<II_PREC_SINGLE>::st(y, g.stride),
-                     y64 ? (double2*)y64->v : nullptr, fold_stride(g, y64), skip, skip_stride);
+                     y64, skip, skip_stride);
   II_HIP(ctx, hipGetLastError());
   return II_OK;
 }
@@ -594,7 +588,7 @@ ii_status cg_p_P(ii_context* ctx, int P, const SF& r, const SF& p, const SF& pou
 }
 ii_status cg_flush_P(ii_context* ctx, int P, const SF* ring, const int* slots, int n,
                      const double* ahist, int astride, const SF& y, int nrhs,
-                     const SF* y64 = nullptr, const int* skip = nullptr, int skip_stride = 0) {
+                     double2* y64 = nullptr, const int* skip = nullptr, int skip_stride = 0) {
   switch (P) {
     case 1: return cg_flush<1>(ctx, ring, slots, n, ahist, astride, y, nrhs, y64, skip, skip_stride);
     case 2: return cg_flush<2>(ctx, ring, slots, n, ahist, astride, y, nrhs, y64, skip, skip_stride);
@@ -1497,7 +1491,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   auto flush = [&](bool fold, const int* skip) -> ii_status {
     if (!fold && pend.empty()) return II_OK;
     II_CHECK(cg_flush_P(ctx, P, ring.data(), pend.data(), (int)pend.size(), ahist, nring, ys, nrhs,
-                        fold ? &xf : nullptr, skip, ss));
+                        fold ? x64 : nullptr, skip, ss));
     pend.clear();
     return II_OK;
   };
@@ -1587,6 +1581,11 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
 SF parity_of(const ii_field* f, int r0, int par, size_t he) {
   return SF{f->data + ((size_t)2 * r0 + par) * he, nullptr, (int)(2 * he)};
 }
+// the even part of nrhs rhs of f from r0 on
+ii_status copy_even64(ii_context* ctx, ii_field* f, int r0, const SF& y, int nrhs) {
+  const size_t he = half_elems(ctx->g);
+  return copy_rhs64(ctx, f->data + (size_t)2 * r0 * he, 2 * he, (const double2*)y.v, nrhs);
+}
 
 // ============================================================ propagator
 // Work slots 40..63 belong to the propagator solver.
@@ -1619,10 +1618,12 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
   II_CHECK(workspace(ctx, 40, sizeof(double) * 3 * batch + 64, &auxp));
   double* aux = (double*)auxp;
   double* one = aux + 3 * batch;  // the device scalar 1.0 (alpha of rho = bhat - Dhat y)
-  // FP64 fields; the sources' parities are read and the solution's written in
-  // place (y is the even part of sol)
-  SF be, bo, bh, y, xo, r64, q64, t64, rho;
+  // FP64 fields; the sources' parities are read in place.  The even solution y
+  // is formed beside sol, which is written when the solve has ended: a solve
+  // that fails leaves it as it was.
+  SF be, bo, bh, y, r64, q64, t64, rho;
   II_CHECK(fieldP(ctx, 43, 0, batch, &bh));
+  II_CHECK(fieldP(ctx, 44, 0, batch, &y));
   II_CHECK(fieldP(ctx, 45, 0, batch, &r64));
   II_CHECK(fieldP(ctx, 46, 0, batch, &q64));
   II_CHECK(fieldP(ctx, 47, 0, batch, &t64));
@@ -1642,6 +1643,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     II_CHECK(fieldP(ctx, 52, 0, batch, &ss_));
     qs = q64;
     ts = t64;
+    ys = y;
   }
   // Deferred solution update (sloppy precisions): the search directions of
   // up to kDefer iterations stay in a ring of kDefer + 1 fields, their
@@ -1664,9 +1666,6 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     be = parity_of(src, r0, 0, he);
     bo = parity_of(src, r0, 1, he);
-    y = parity_of(sol, r0, 0, he);
-    xo = parity_of(sol, r0, 1, he);
-    if (!lo) ys = y;
     // |b|^2 of the full sources
     II_CHECK(dot64(ctx, (double2*)be.v, (double2*)be.v, aux, 2 * nr));
     // bhat = b_e - mult_eo(b_o) = b_e + kappa H_eo b_o   (eoUtils.cpp:54-57)
@@ -1679,7 +1678,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     // c = Dhat^dag bhat  -> r64 ; y = 0
     II_CHECK(dhat_dag64(ctx, kappa, (double2*)bh.v, (double2*)r64.v, (double2*)t64.v, nullptr,
                         nullptr, nr));
-    II_CHECK(zero64(ctx, (double2*)y.v, nr, y.rs));
+    II_CHECK(zero64(ctx, (double2*)y.v, nr));
     // rr = |c|^2 into aux[2*batch ...]
     II_CHECK(dot64(ctx, (double2*)r64.v, (double2*)r64.v, aux + 2 * batch, nr));
     // b2 = |b_e|^2 + |b_o|^2 -> aux[0..nr)
@@ -1743,7 +1742,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     // masked by skip), ys restarted at 0
     auto flush_fold = [&](const int* skip) -> ii_status {
       II_CHECK(cg_flush_P(ctx, P, ring.data(), pend.data(), (int)pend.size(), ahist, nring, ys,
-                          nr, &y, skip, ss));
+                          nr, (double2*)y.v, skip, ss));
       pend.clear();
       return II_OK;
     };
@@ -1870,7 +1869,8 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
     h.a = kappa;
     h.xpay = true;
     h.nrhs = nr;
-    II_CHECK(hopP(ctx, 0, h, y, xo, &bo, nullptr));
+    II_CHECK(hopP(ctx, 0, h, y, parity_of(sol, r0, 1, he), &bo, nullptr));
+    II_CHECK(copy_even64(ctx, sol, r0, y, nr));
     II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     II_CHECK(read_scalars(ctx, nr));
     float ms = 0.f;
@@ -2111,8 +2111,7 @@ struct BiDirs {
 template <typename SpP, typename SpY, typename StY>
 __global__ void __launch_bounds__(kBlock)
 k_bi_flush(Geom g, BiDirs<SpP> d, const double* __restrict__ ahist, int astride, SpY yr, StY yw,
-           double2* __restrict__ y64, size_t y64_rs, const int* __restrict__ skip,
-           int skip_stride) {
+           double2* __restrict__ y64, const int* __restrict__ skip, int skip_stride) {
   const int rhs = blockIdx.y;
   const int hs = blockIdx.x * blockDim.x + threadIdx.x;
   if (hs >= g.Vh) return;
@@ -2144,7 +2143,7 @@ k_bi_flush(Geom g, BiDirs<SpP> d, const double* __restrict__ ahist, int astride,
     }
   }
   if (fold) {
-    double2* y = y64 + (size_t)rhs * y64_rs;
+    double2* y = y64 + (size_t)rhs * 12 * g.stride;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
       double2 o = y[(size_t)k * g.stride + hs];
@@ -2234,7 +2233,7 @@ struct BiBlas {
     return II_OK;
   }
   static ii_status flush(ii_context* ctx, const SF* rp, const SF* rs, const int* slots, int n,
-                         const double* ahist, int astride, const SF& y, int nrhs, const SF* y64,
+                         const double* ahist, int astride, const SF& y, int nrhs, double2* y64,
                          const int* skip, int ss) {
     const Geom& g = ctx->g;
     using Y = Acc<II_PREC_SINGLE>;
@@ -2248,8 +2247,7 @@ struct BiBlas {
     }
     hipLaunchKernelGGL((k_bi_flush<typename A::Sp, typename Y::Sp, typename Y::St>),
                        dim3(blocks_for(g.Vh), nrhs), dim3(kBlock), 0, ctx->stream, g, d, ahist,
-                       astride, Y::sp(y, g.stride), Y::st(y, g.stride),
-                       y64 ? (double2*)y64->v : nullptr, fold_stride(g, y64), skip, ss);
+                       astride, Y::sp(y, g.stride), Y::st(y, g.stride), y64, skip, ss);
     II_HIP(ctx, hipGetLastError());
     return II_OK;
   }
@@ -2308,8 +2306,9 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
   double* one = aux + 3 * batch;
   II_CHECK(workspace(ctx, 63, sizeof(BiCoef) * batch, &v));
   BiCoef* bc = (BiCoef*)v;
-  SF be, bo, bh, y, xo, q64, t64;  // be, bo: parities of src; y, xo: of sol
+  SF be, bo, bh, y, q64, t64;  // be, bo: parities of src
   II_CHECK(fieldP(ctx, 43, 0, batch, &bh));
+  II_CHECK(fieldP(ctx, 44, 0, batch, &y));  // the even solution, until the solve has ended
   II_CHECK(fieldP(ctx, 46, 0, batch, &q64));
   II_CHECK(fieldP(ctx, 47, 0, batch, &t64));
   SF r, r0, vv, w, t, ys;
@@ -2336,8 +2335,6 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
     II_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     be = parity_of(src, rb0, 0, he);
     bo = parity_of(src, rb0, 1, he);
-    y = parity_of(sol, rb0, 0, he);
-    xo = parity_of(sol, rb0, 1, he);
     II_CHECK(dot64(ctx, (double2*)be.v, (double2*)be.v, aux, 2 * nr));
     // bhat = b_e + kappa H_eo b_o   (eoUtils.cpp:54-57)
     h = HopSpec();
@@ -2349,7 +2346,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
     h.partials = part;
     II_CHECK(hopP(ctx, 0, h, bo, bh, &be, nullptr));
     II_CHECK(finalize_sums(ctx, part, hop_dot_parts(g, nr, II_PREC_DOUBLE), aux + 2 * batch, nr));
-    II_CHECK(zero64(ctx, (double2*)y.v, nr, y.rs));
+    II_CHECK(zero64(ctx, (double2*)y.v, nr));
     {
       std::vector<double> hb(2 * batch);
       II_HIP(ctx, hipMemcpyAsync(hb.data(), aux, 2 * batch * sizeof(double),
@@ -2373,7 +2370,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
     II_CHECK(convertP(ctx, 0, II_PREC_SINGLE, y, ys, nr));  // zeros
     int pos = 0;            // ring slot of this iteration's p and s
     std::vector<int> pend;  // slots whose alpha p + omega s is not yet in ys
-    auto flush = [&](const SF* y64, const int* skip) -> ii_status {
+    auto flush = [&](double2* y64, const int* skip) -> ii_status {
       if (pend.empty() && !y64) return II_OK;
       II_CHECK(BB::flush(ctx, rp, rsr, pend.empty() ? &pos : pend.data(), (int)pend.size(), ahist,
                          nring, ys, nr, y64, skip, ss));
@@ -2446,7 +2443,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       chunk = 1;
       II_CHECK(join_updates(ctx, nr));
       // reliable update for the flagged rhs: y64 += ys + pending, ys = 0
-      II_CHECK(flush(&y, skip_ru));
+      II_CHECK(flush((double2*)y.v, skip_ru));
       // rho_true = bhat - Dhat y (FP64) and |rho_true|^2
       h = HopSpec();
       h.nrhs = nr;
@@ -2472,14 +2469,15 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       II_CHECK(convertP(ctx, P, P, r, r0, nr, &sc[0].keep_p, ss));
       II_CHECK(convertP(ctx, P, P, r, rp[pos], nr, &sc[0].keep_p, ss));
     }
-    II_CHECK(flush(&y, nullptr));
+    II_CHECK(flush((double2*)y.v, nullptr));
     // x_o = b_o + kappa H_oe y   (eoUtils.cpp:67)
     h = HopSpec();
     h.out_par = 1;
     h.a = kappa;
     h.xpay = true;
     h.nrhs = nr;
-    II_CHECK(hopP(ctx, 0, h, y, xo, &bo, nullptr));
+    II_CHECK(hopP(ctx, 0, h, y, parity_of(sol, rb0, 1, he), &bo, nullptr));
+    II_CHECK(copy_even64(ctx, sol, rb0, y, nr));
     II_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     II_CHECK(read_scalars(ctx, nr));
     float ms = 0.f;
@@ -2792,7 +2790,7 @@ ii_status ii_propagator_solve(ii_context* ctx, double kappa, const ii_prop_param
     return set_error(ctx, II_ERR_BAD_ARG, "propagator fields must be full and of equal nrhs");
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
-  // the solution is built in place while the source is still read
+  // the true residual below needs the source once the solution is written
   ii_field own;
   if (src->data == sol->data) {
     II_CHECK(temp_field(ctx, 0, II_FULL, src->nrhs, &own));

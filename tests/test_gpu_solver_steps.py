@@ -144,3 +144,33 @@ def test_propagator_parities_in_place(method, precision, nrhs):
             assert lat.true_residual_full(u, kappa, f.download(k), bs[k]) <= 1e-10, k
             assert f is src or np.array_equal(src.download(k), bs[k])
     ctx.close()
+
+
+@pytest.mark.parametrize("method,precision,size", [("cg", "double", 1e200), ("cg", "half", 1e50),
+                                                   ("bicgstab", "single", 1e50),
+                                                   ("fgcr", "single", 1e50)])
+@pytest.mark.parametrize("same", [False, True])
+def test_failed_propagator_solve_leaves_the_solution(method, precision, size, same):
+    """A source beyond the range of the solver's scalars ends the solve with an
+    error: the solution field, and a source that is the solution field too, are
+    left as they were."""
+    dims = (6, 4, 2, 10)
+    lat = orc.Lattice(dims)
+    ctx = ii.Context(dims)
+    ctx.upload_gauge(lat.apbc(lat.gauge_expH(0.3, 23)))
+    rng = np.random.default_rng(1)
+    b = rng.normal(size=(3, lat.full_size))
+    b[1] *= size
+    old = b if same else rng.normal(size=(3, lat.full_size))
+    sol = ii.DeviceField(ctx, "full", 3)
+    src = sol if same else ii.DeviceField(ctx, "full", 3)
+    for k in range(3):
+        sol.upload(k, old[k])
+        src.upload(k, b[k])
+    with pytest.raises(ii.IIError) as e:
+        ii.PropagatorSolver(ctx, 0.12, precision=precision, batched=True, method=method,
+                            maxiter=200).solve(src, sol)
+    assert not isinstance(e.value, ii.ConvergenceErr)
+    for k in range(3):
+        assert np.array_equal(sol.download(k), old[k]), k
+    ctx.close()
