@@ -118,6 +118,17 @@ ii_status temp_field(ii_context* ctx, int slot, int subset, int nrhs, ii_field* 
   return II_OK;
 }
 
+TempFields::~TempFields() {
+  size_t held = 0;
+  for (int i = kSlotFields; i < ii_context::kSlots; ++i) held += ctx->work[i].bytes;
+  if (held <= kKeepFields) return;
+  (void)hipStreamSynchronize(ctx->stream);
+  for (int i = kSlotFields; i < ii_context::kSlots; ++i) {
+    if (ctx->work[i].ptr) (void)hipFree(ctx->work[i].ptr);
+    ctx->work[i] = Buffer();
+  }
+}
+
 // FP64 half-field workspaces: slots 2.. (nrhs = 1).
 ii_status half64(ii_context* ctx, int k, double2** p) {
   void* v = nullptr;

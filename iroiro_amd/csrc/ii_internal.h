@@ -165,10 +165,16 @@ ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t byt
 ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes);
 void host_pipe_release(ii_context* ctx);
 // A field of nrhs rhs in workspace slots (kSlotFields ...), for the solvers'
-// inputs and results on host arrays: kept between calls, where a field of its
-// own took an allocation, a clear and a free each.
+// inputs and results on host arrays: kept between calls up to kKeepFields bytes
+// in all, where a field of its own took an allocation, a clear and a free each.
+// Every function that takes one holds a TempFields, which gives back more.
 constexpr int kSlotFields = 96;
+constexpr size_t kKeepFields = (size_t)4 << 30;  // 1.4% of the card
 ii_status temp_field(ii_context* ctx, int slot, int subset, int nrhs, ii_field* f);
+struct TempFields {
+  ii_context* ctx;
+  ~TempFields();
+};
 ii_status require_gauge(ii_context* ctx);
 // Entry of every API call on a context: selects its device and clears a
 // stale HIP error left by an earlier, already reported failure.

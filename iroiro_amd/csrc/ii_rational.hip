@@ -105,6 +105,7 @@ ii_status ii_rational_solve(ii_context* ctx, double kappa, double* sol, const do
   auto t0 = std::chrono::steady_clock::now();
   ii_field fb_, fx_, fs_;
   ii_field *fb = &fb_, *fx = &fx_, *fs = &fs_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
   II_CHECK(temp_field(ctx, 1, II_EVEN, npoles, fx));
   II_CHECK(temp_field(ctx, 2, II_EVEN, 1, fs));
@@ -142,6 +143,7 @@ ii_status ii_action_nf_md_force(ii_context* ctx, double kappa, const double* phi
   const size_t he = half_elems(g);
   ii_field fphi_, fx_, fz_;
   ii_field *fphi = &fphi_, *fx = &fx_, *fz = &fz_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_EVEN, npf, fphi));
   II_CHECK(temp_field(ctx, 1, II_EVEN, npoles, fx));
   II_CHECK(temp_field(ctx, 2, II_EVEN, 2, fz));  // zeta and an odd temporary

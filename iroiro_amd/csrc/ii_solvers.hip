@@ -1412,7 +1412,14 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   II_CHECK(fieldP(ctx, 39, 0, nrhs, &t64));  // Dhat x, intermediate
   II_CHECK(fieldP(ctx, 41, 0, nrhs, &u64));  // odd temporary
   II_CHECK(fieldP(ctx, 40, 0, nrhs, &rho));
-  const int nring = lo ? kDefer + 1 : 1;
+  // Directions kept for the deferred solution update: kDefer + 1 sets while
+  // they take at most 8 GiB, else 4 FP32 or 6 16-bit sets, which with the other
+  // fields here are the memory of a solver that keeps one set, A p and (A) y.
+  const size_t set = field_bytes(g, P) * nrhs;
+  const int nring = !lo                                               ? 1
+                    : set * (kDefer + 1) <= ((size_t)8 << 30) ? kDefer + 1
+                    : P == II_PREC_SINGLE                             ? 4
+                                                                      : 6;
   std::vector<SF> ring(nring);
   double* ahist = nullptr;
   if (lo) {
@@ -1516,7 +1523,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
         pend.push_back(pos);
         pos = (pos + 1) % nring;
         II_CHECK(cg_p_P(ctx, P, rs, p, ring[pos], sc, nrhs, pnorm));
-        if ((int)pend.size() == kDefer) II_CHECK(flush(false, nullptr));
+        if ((int)pend.size() == nring - 1) II_CHECK(flush(false, nullptr));
       } else {
         II_CHECK(ddagdP(ctx, P, kappa, p, ss_, qs, ts, nullptr, nullptr, nrhs, skip_it, ss));
         II_CHECK(sp_shift64(ctx, p, ss_, sig, sc, nrhs, part));
@@ -2614,6 +2621,7 @@ ii_status ii_solver_cg(ii_context* ctx, double kappa, double* x, const double* b
   const Geom& g = ctx->g;
   ii_field fb_, fx_;
   ii_field *fb = &fb_, *fx = &fx_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
   II_CHECK(temp_field(ctx, 1, II_EVEN, 1, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
@@ -2635,6 +2643,7 @@ ii_status ii_multishift_cg(ii_context* ctx, double kappa, double* x, const doubl
   const Geom& g = ctx->g;
   ii_field fb_, fx_;
   ii_field *fb = &fb_, *fx = &fx_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
   II_CHECK(temp_field(ctx, 1, II_EVEN, nshift, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
@@ -2658,6 +2667,7 @@ ii_status ii_multishift_mixed(ii_context* ctx, double kappa, double* x, const do
   const Geom& g = ctx->g;
   ii_field fb_, fx_;
   ii_field *fb = &fb_, *fx = &fx_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_EVEN, 1, fb));
   II_CHECK(temp_field(ctx, 1, II_EVEN, nshift, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
@@ -2679,6 +2689,7 @@ ii_status ii_multishift_cg_full(ii_context* ctx, double kappa, double* x, const 
   const Geom& g = ctx->g;
   ii_field fb_, fx_;
   ii_field *fb = &fb_, *fx = &fx_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_FULL, 1, fb));
   II_CHECK(temp_field(ctx, 1, II_FULL, nshift, fx));
   II_CHECK(ii_field_upload(fb, 0, b));
@@ -2748,6 +2759,7 @@ ii_status ii_eo_invert(ii_context* ctx, double kappa, double* sol, const double*
   const size_t he = half_elems(g);
   ii_field fs_, fx_, fb_, fy_;
   ii_field *fs = &fs_, *fx = &fx_, *fb = &fb_, *fy = &fy_;
+  TempFields temps{ctx};
   II_CHECK(temp_field(ctx, 0, II_FULL, 1, fs));
   II_CHECK(temp_field(ctx, 1, II_FULL, 1, fx));
   II_CHECK(temp_field(ctx, 2, II_EVEN, 1, fb));
@@ -2791,6 +2803,7 @@ ii_status ii_propagator_solve(ii_context* ctx, double kappa, const ii_prop_param
   II_CHECK(require_gauge(ctx));
   II_CHECK(enter(ctx));
   // the true residual below needs the source once the solution is written
+  TempFields temps{ctx};
   ii_field own;
   if (src->data == sol->data) {
     II_CHECK(temp_field(ctx, 0, II_FULL, src->nrhs, &own));

@@ -174,3 +174,37 @@ def test_failed_propagator_solve_leaves_the_solution(method, precision, size, sa
     for k in range(3):
         assert np.array_equal(sol.download(k), old[k]), k
     ctx.close()
+
+
+def test_many_shifts_on_a_large_lattice_hold_no_more_memory():
+    """64 shifts at 24^3x52: one FP64 set of half fields takes 4.4 GB.  The mixed
+    solve keeps four FP32 directions a shift there and gives its input and result
+    fields back: five FP64-set equivalents of FP32 fields (4 directions, r, q, t,
+    the solution, stage 1's p and x), three FP64 sets and the hop tuner's two."""
+    import ctypes
+    hip = ctypes.CDLL(ii._lib.LIB_PATH)  # the library's own HIP runtime
+
+    def free():
+        v = [ctypes.c_size_t(), ctypes.c_size_t()]
+        assert hip.hipMemGetInfo(ctypes.byref(v[0]), ctypes.byref(v[1])) == 0
+        return v[0].value
+
+    dims, n = (24, 24, 24, 52), 64
+    ctx = ii.Context(dims)
+    u = np.zeros((4, ctx.V, 3, 3, 2))
+    u[..., [0, 1, 2], [0, 1, 2], 0] = 1.0
+    D = ii.Dirac_Wilson_EvenOdd(1.0 / (2 * 0.11) - 4.0, u.ravel(), ctx)
+    del u
+    A = ii.Fopr_DdagD(D)
+    b = np.random.default_rng(8).normal(size=D.fsize())
+    A.mult(b)
+    shifts = np.geomspace(1e-2, 10.0, n)
+    x = list(np.empty((n, D.fsize())))
+    free0 = free()
+    outs = ii.MultiShiftSolver_Mixed(A, tol=1e-10, precision="single").solve(x, b, shifts)
+    used = free0 - free()
+    for i in (0, 17, 63):
+        r = np.linalg.norm(A.mult(x[i]) + shifts[i] * x[i] - b) / np.linalg.norm(b)
+        assert r <= 1.001e-10 and abs(outs[i].true_residual - r) < 1e-3 * r + 1e-14
+    ctx.close()
+    assert used < 10.3 * 8 * D.fsize() * n, used / (8 * D.fsize() * n)
