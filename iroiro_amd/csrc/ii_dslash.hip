@@ -626,7 +626,8 @@ int hop_dot_parts(const Geom& g, int nrhs, int precision) {
 // Runs when ii_autotune asks for it, never inside a stream capture: the
 // contiguous order that a context starts with is within 2% of the best strip
 // everywhere (us, contiguous / best strip: 17.8 / 17.5 at 16^3x32, 139.0 /
-// 139.3 at 32^4, 262.8 / 262.0 at 32^3x64).  II_HOP_ORDER=0 or II_HOP_ORDER=1:W forces an order.
+// 139.3 at 32^4, 262.8 / 262.0 at 32^3x64).  II_HOP_ORDER=0 or
+// II_HOP_ORDER=1:W, read at a context's first such hop, forces an order.
 ii_status tune_hop(ii_context* ctx) {
   ctx->hop_tuned = true;
   const Geom& g = ctx->g;
@@ -802,8 +803,10 @@ static bool links_cached(unsigned long long gauge_bytes) { return gauge_bytes <=
 ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* out,
                 const double2* x, const double2* dv) {
   const Geom& g = ctx->g;
-  static const bool forced = std::getenv("II_HOP_ORDER") != nullptr;
-  if (forced && h.nrhs == 1 && !ctx->hop_tuned && !h.no_tune) II_CHECK(tune_hop(ctx));
+  if (h.nrhs == 1 && !ctx->hop_env_read && !h.no_tune) {
+    ctx->hop_env_read = true;
+    if (!ctx->hop_tuned && std::getenv("II_HOP_ORDER")) II_CHECK(tune_hop(ctx));
+  }
   SpF64 sin{in, g.stride, h.rs_in};
   StF64 so{out, g.stride, h.rs_out};
   SpF64 sx{x ? x : in, g.stride, x ? h.rs_x : h.rs_in};

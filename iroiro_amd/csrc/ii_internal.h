@@ -114,6 +114,7 @@ struct ii_context {
   ii::HopOrder mrhs_ord[4];
   std::string mrhs_report[4];
   bool hop_tuned = false;
+  bool hop_env_read = false;  // II_HOP_ORDER has been looked for
   std::string tune_report;
   // learned preconditioner state (owned by ii_learned.hip) and the batched
   // network and flexible solver workspaces (owned by ii_bnet.hip)

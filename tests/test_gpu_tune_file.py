@@ -46,3 +46,31 @@ def test_tune_file_round_trip(tmp_path):
             other.tune_load(files[0])
     finally:
         other.close()
+
+
+def hop_line(ctx, path):
+    ctx.tune_save(path)
+    return [v for v in path.read_text().splitlines() if v.startswith("hop ")]
+
+
+def test_forced_hop_order_is_read_by_each_context(tmp_path, monkeypatch):
+    """II_HOP_ORDER set after a context of the process has run its hops holds
+    for the next context, and no longer once it is unset; the order changes no
+    bit of the result."""
+    dims = (16, 16, 4, 16)
+    lat = orc.Lattice(dims)
+    u = lat.apbc(lat.gauge_expH(0.4, 92))
+    f = np.random.default_rng(6).normal(size=lat.half_size)
+    res, lines = [], []
+    for env in (None, "1:2", None):
+        if env:
+            monkeypatch.setenv("II_HOP_ORDER", env)
+        else:
+            monkeypatch.delenv("II_HOP_ORDER", raising=False)
+        ctx = ii.Context(dims)
+        res.append(ii.Dirac_Wilson_EvenOdd(0.1, u, ctx).mult(f))
+        lines.append(hop_line(ctx, tmp_path / "t.tune"))
+        ctx.close()
+    assert lines[1][0].startswith("hop 1 2 ")
+    assert not any(v.startswith("hop 1") for v in lines[0] + lines[2])
+    assert np.array_equal(res[0], res[1]) and np.array_equal(res[0], res[2])
