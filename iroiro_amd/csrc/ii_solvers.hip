@@ -2860,7 +2860,8 @@ ii_status ii_autotune(ii_context* ctx, char* report, size_t len) {
 // Tuning file: one line per choice, for one lattice.
 //   iroiro-hip tuning 1
 //   lattice Lx Ly Lz Lt
-//   hop mode W bpp bs                      (the single-rhs FP64 hop's order)
+//   hop mode W bpp bs                      (the single-rhs FP64 hop's order, once
+//                                           chosen; bs is not read)
 //   mrhs P nrhs rb mode W bpp bs           (each tuned multi-rhs precision P)
 //   net nrhs rg0..rg3 by0..by3 bz0..bz3    (the network stages)
 ii_status ii_tune_save(ii_context* ctx, const char* path) {
@@ -2869,8 +2870,10 @@ ii_status ii_tune_save(ii_context* ctx, const char* path) {
   std::FILE* f = std::fopen(path, "w");
   if (!f) return set_error(ctx, II_ERR_BAD_ARG, std::string("cannot create tuning file ") + path);
   std::fprintf(f, "iroiro-hip tuning 1\nlattice %d %d %d %d\n", g.L[0], g.L[1], g.L[2], g.L[3]);
-  const HopOrder& h = ctx->hop_order;
-  std::fprintf(f, "hop %d %d %d %d\n", h.mode, h.W, h.bpp, h.bs);
+  if (ctx->hop_tuned) {
+    const HopOrder& o = ctx->hop_order;
+    std::fprintf(f, "hop %d %d %d %d\n", o.mode, o.W, o.bpp, o.bs);
+  }
   for (int P = 0; P < 4; ++P)
     if (ctx->mrhs_nrhs[P] > 0) {
       const HopOrder& o = ctx->mrhs_ord[P];

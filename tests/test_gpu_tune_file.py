@@ -74,3 +74,25 @@ def test_forced_hop_order_is_read_by_each_context(tmp_path, monkeypatch):
     assert lines[1][0].startswith("hop 1 2 ")
     assert not any(v.startswith("hop 1") for v in lines[0] + lines[2])
     assert np.array_equal(res[0], res[1]) and np.array_equal(res[0], res[2])
+
+
+def test_file_of_an_untuned_context_leaves_the_hop_order(tmp_path, monkeypatch):
+    """A context that has chosen no hop order writes none, and its file does not
+    replace the order another context has."""
+    dims = (16, 16, 4, 16)
+    lat = orc.Lattice(dims)
+    u = lat.apbc(lat.gauge_expH(0.4, 93))
+    f = np.random.default_rng(7).normal(size=lat.half_size)
+    plain, tuned = tmp_path / "plain.tune", tmp_path / "tuned.tune"
+    monkeypatch.delenv("II_HOP_ORDER", raising=False)
+    a = ii.Context(dims)
+    ii.Dirac_Wilson_EvenOdd(0.1, u, a).mult(f)
+    assert hop_line(a, plain) == []
+    monkeypatch.setenv("II_HOP_ORDER", "1:2")
+    b = ii.Context(dims)
+    ii.Dirac_Wilson_EvenOdd(0.1, u, b).mult(f)
+    want = hop_line(b, tuned)
+    b.tune_load(plain)
+    assert hop_line(b, tuned) == want and want[0].startswith("hop 1 2 ")
+    a.close()
+    b.close()
