@@ -216,9 +216,11 @@ def as_f64(a, n=None):
 
 def result_f64(a, n):
     """Where a solver writes n doubles for the caller's array `a`: `a` itself
-    if it is such an array in memory, else a new one (to be copied into `a`)."""
-    if (isinstance(a, np.ndarray) and a.dtype == np.float64 and a.size == n and
-            a.flags.c_contiguous and a.flags.writeable):
+    if it is a plain array of n doubles in memory, else a new one, to be copied
+    by `a[...] =`, which is what other shapes, types and subclasses (masks,
+    memory maps) take or refuse."""
+    if (type(a) is np.ndarray and a.dtype == np.float64 and a.shape == (n,) and
+            a.flags.c_contiguous and a.flags.writeable and a.flags.aligned):
         return a
     return np.empty(n)
 

@@ -1,0 +1,46 @@
+"""Which arrays of the caller a solver writes in place, and that the others
+take or refuse the result as an assignment does."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from iroiro_amd import _lib
+
+
+def deliver(a, x):
+    """What the solver classes do with a result x for the caller's array a."""
+    y = _lib.result_f64(a, x.size)
+    ctypes.memmove(y.ctypes.data, x.ctypes.data, x.nbytes)  # the library's write
+    if y is not a:
+        a[...] = y
+
+
+def test_plain_arrays_in_place():
+    a = np.zeros(6)
+    assert _lib.result_f64(a, 6) is a
+    deliver(a, np.arange(6.0))
+    assert np.array_equal(a, np.arange(6.0))
+
+
+@pytest.mark.parametrize("a", [np.zeros(6, np.float32), np.zeros(12)[::2], np.zeros((1, 6)),
+                               np.zeros(6, ">f8"), np.zeros((6, 1)).T,
+                               np.frombuffer(bytearray(49), np.float64, 6, 1)])
+def test_other_arrays_by_assignment(a):
+    assert _lib.result_f64(a, 6) is not a
+    deliver(a, np.arange(6.0))
+    assert np.array_equal(np.ravel(a), np.arange(6.0))
+
+
+def test_masked_arrays_take_the_values_as_an_assignment():
+    a = np.ma.array(np.zeros(6), mask=[True] * 6)
+    deliver(a, np.arange(6.0))
+    assert not a.mask.any() and np.array_equal(a.data, np.arange(6.0))
+
+
+@pytest.mark.parametrize("shape", [(2, 3), (6, 1), (3, 2, 1), (5,)])
+def test_shapes_that_an_assignment_refuses(shape):
+    a = np.zeros(shape)
+    with pytest.raises(ValueError):
+        deliver(a, np.arange(6.0))
+    assert not a.any()
