@@ -1010,7 +1010,7 @@ class LearnedPreconditioner:
         """Loss sum_k |M b_k - y_k|^2/|y_k|^2 and its gradient per layer."""
         nh = 24 * self.ctx.V // 2
         bs, ys = [np.ravel(v) for v in bs], [np.ravel(v) for v in ys]
-        if len(bs) != len(ys) or any(v.size != nh for v in bs + ys):
+        if not bs or len(bs) != len(ys) or any(v.size != nh for v in bs + ys):
             bs = _lib.as_f64(np.concatenate(bs), nh * len(bs)).reshape(-1, nh)
             ys = _lib.as_f64(np.concatenate(ys), nh * len(bs)).reshape(-1, nh)
         sizes = [int(np.prod(self.shape(l))) for l in range(_lib.NET_LAYERS)]

@@ -1,10 +1,13 @@
 """Which arrays of the caller a solver writes in place, and that the others
-take or refuse the result as an assignment does."""
+take or refuse the result as an assignment does; arguments refused before the
+library is called."""
 import ctypes
+import types
 
 import numpy as np
 import pytest
 
+import iroiro_amd as ii
 from iroiro_amd import _lib
 
 
@@ -44,3 +47,13 @@ def test_shapes_that_an_assignment_refuses(shape):
     with pytest.raises(ValueError):
         deliver(a, np.arange(6.0))
     assert not a.any()
+
+
+@pytest.mark.parametrize("bs,ys", [([], []), ([np.zeros(192)], []),
+                                   ([np.zeros(192)], [np.zeros(180)])])
+def test_loss_grad_refuses_pairs_that_do_not_match(bs, ys):
+    """Before anything reaches the device: no pairs, pairs of different number
+    or size are a ValueError."""
+    ctx = types.SimpleNamespace(V=16, handle=None)
+    with pytest.raises(ValueError):
+        ii.LearnedPreconditioner(ctx).loss_grad(bs, ys)
