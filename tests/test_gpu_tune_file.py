@@ -96,3 +96,20 @@ def test_file_of_an_untuned_context_leaves_the_hop_order(tmp_path, monkeypatch):
     assert hop_line(b, tuned) == want and want[0].startswith("hop 1 2 ")
     a.close()
     b.close()
+
+
+def test_multi_rhs_shapes_timed_where_blocks_are_few(tmp_path):
+    """On a small lattice, and for fewer rhs than fill a block, the tuner times
+    every number of rhs per block: 64 tiles x 1 block of 12 rhs would leave most
+    of the chip idle."""
+    dims = (8, 8, 8, 16)
+    ctx = ii.Context(dims)
+    lat = orc.Lattice(dims)
+    ctx.upload_gauge(lat.apbc(lat.gauge_expH(0.4, 94)))
+    parts = ctx.autotune().split(";")
+    mrhs = [p for p in parts if "multi-rhs hop" in p]
+    assert len(mrhs) == 4
+    for p in mrhs:
+        for rb in (12, 6, 4, 3, 2):
+            assert " %d/contig=" % rb in p
+    ctx.close()
