@@ -84,12 +84,9 @@ __global__ void k_fin_pap(const double* __restrict__ partials, int nb, RUScal* _
   }
 }
 
-// rr_new -> beta, and the stopping / reliable-update decisions.
-// mode 0: reference CG test rr*snorm < prec (solver_CG.cpp:57-60)
-// mode 1: reliable-update CG: flag an update when |r|^2 < delta2*rmax2 or
-//         |r|^2 < target2.
-__global__ void k_fin_rr(const double* __restrict__ partials, int nb, RUScal* __restrict__ sc,
-                         int mode) {
+// rr_new -> beta; flags a reliable update when |r|^2 < delta2*rmax2 or
+// |r|^2 < target2.
+__global__ void k_fin_rr(const double* __restrict__ partials, int nb, RUScal* __restrict__ sc) {
   RUScal& S = sc[blockIdx.x];
   if (S.done) return;
   const double* p = partials + (size_t)blockIdx.x * nb;
@@ -103,12 +100,8 @@ __global__ void k_fin_rr(const double* __restrict__ partials, int nb, RUScal* __
     S.count += 1;
     S.keep_p = 1;
     if (!finite(s) || !finite(S.beta)) { S.nan = 1; S.done = 1; S.skip_ru = 1; return; }
-    if (mode == 0) {
-      if (s * S.snorm < S.prec) { S.done = 1; S.iter = S.count - 1; }
-    } else {
-      bool upd = (s < S.delta2 * S.rmax2) || (s < S.target2);
-      S.skip_ru = upd ? 0 : 1;
-    }
+    bool upd = (s < S.delta2 * S.rmax2) || (s < S.target2);
+    S.skip_ru = upd ? 0 : 1;
   }
 }
 
@@ -654,7 +647,7 @@ ii_status join_updates(ii_context* ctx, int n) {
 }
 
 __global__ void k_scal_init(RUScal* sc, const double* __restrict__ rr, const double* __restrict__ bb,
-                            double prec, double tol, double delta, int mode,
+                            double prec, double tol, double delta,
                             double restart = 16.0) {
   RUScal& S = sc[blockIdx.x];
   if (threadIdx.x != 0) return;
@@ -673,7 +666,6 @@ __global__ void k_scal_init(RUScal* sc, const double* __restrict__ rr, const dou
   z.skip_ru = 1;
   z.keep_p = 1;
   if (!(z.rr > 0.0)) { z.done = 1; }
-  if (mode == 0) z.skip_ru = 1;
   S = z;
 }
 
@@ -815,7 +807,7 @@ ii_status cg_reference(ii_context* ctx, double kappa, double2* x, const double2*
   II_CHECK(dot64(ctx, (double2*)fr.v, (double2*)fr.v, tmp2));
   II_CHECK(dot64(ctx, b, b, tmp2 + 1));
   hipLaunchKernelGGL(k_scal_init, dim3(1), dim3(64), 0, ctx->stream, sc, tmp2, tmp2 + 1, prec,
-                     0.0, 0.0, 0);
+                     0.0, 0.0);
   II_HIP(ctx, hipGetLastError());
   const size_t n = half_elems(g);
   const int xpblk = std::min(blocks_for((long)n, 2 * kBlock), 2048);
@@ -1491,7 +1483,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
   II_CHECK(residual(nullptr, 0));
   II_CHECK(finalize_sums(ctx, part, nhd, rr0, nrhs));
   hipLaunchKernelGGL(k_scal_init, dim3(nrhs), dim3(64), 0, ctx->stream, sc, rr0, bb, 0.0, tol,
-                     delta, 1, restart);
+                     delta, restart);
   II_HIP(ctx, hipGetLastError());
   int pos = 0;            // ring slot of the current search directions
   std::vector<int> pend;  // ring slots whose alpha p is not yet in ys
@@ -1518,8 +1510,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
       if (lo) {
         II_CHECK(ddagd_cg_fused(ctx, P, kappa, p, rs, qs, ts, sc, part, nrhs, skip_it, ss, ahist,
                                 pos, nring, sig, pnorm));
-        hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kFinThreads), 0, ctx->stream, part, nh, sc,
-                           1);
+        hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kFinThreads), 0, ctx->stream, part, nh, sc);
         pend.push_back(pos);
         pos = (pos + 1) % nring;
         II_CHECK(cg_p_P(ctx, P, rs, p, ring[pos], sc, nrhs, pnorm));
@@ -1530,7 +1521,7 @@ ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, in
         hipLaunchKernelGGL(k_fin_pap, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc,
                            nullptr, 0, 0);
         II_CHECK(cg_blas64(ctx, p, ss_, rs, ys, sc, nrhs, part, nb));
-        hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc, 1);
+        hipLaunchKernelGGL(k_fin_rr, dim3(nrhs), dim3(kBlock), 0, ctx->stream, part, nb, sc);
         II_CHECK(cg_p_P(ctx, P, rs, p, p, sc, nrhs));
       }
     }
@@ -1702,7 +1693,7 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
       II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
     hipLaunchKernelGGL(k_scal_init, dim3(nr), dim3(64), 0, ctx->stream, sc, aux + 2 * batch, aux,
-                       0.0, tol, delta, 1, prm->restart_factor > 0 ? prm->restart_factor : 16.0);
+                       0.0, tol, delta, prm->restart_factor > 0 ? prm->restart_factor : 16.0);
     II_HIP(ctx, hipGetLastError());
     if (lo) {
       II_CHECK(convertP(ctx, 0, P, r64, rs, nr));
@@ -1728,13 +1719,13 @@ ii_status propagator(ii_context* ctx, double kappa, const ii_prop_params* prm,
         II_CHECK(ddagd_cg_fused(ctx, P, kappa, p, rs, qs, ts, sc, part, nr, skip_it, ss, ahist,
                                 cur, nring));
         hipLaunchKernelGGL(k_fin_rr, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part,
-                           hop_dot_parts(g, nr, P), sc, 1);
+                           hop_dot_parts(g, nr, P), sc);
       } else {
         II_CHECK(ddagdP(ctx, P, kappa, p, ss_, qs, ts, &p, part, nr, skip_it, ss));
         hipLaunchKernelGGL(k_fin_pap, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part,
                            hop_dot_parts(g, nr, P), sc, nullptr, 0, 0);
         II_CHECK(cg_blas64(ctx, p, ss_, rs, ys, sc, nr, part, nb));
-        hipLaunchKernelGGL(k_fin_rr, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part, nb, sc, 1);
+        hipLaunchKernelGGL(k_fin_rr, dim3(nr), dim3(kFinThreads), 0, ctx->stream, part, nb, sc);
       }
       return cg_p_P(ctx, P, rs, p, ring[(cur + 1) % nring], sc, nr);
     };
@@ -2367,7 +2358,7 @@ ii_status propagator_bicgstab_t(ii_context* ctx, double kappa, const ii_prop_par
       II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
     hipLaunchKernelGGL(k_scal_init, dim3(nr), dim3(64), 0, ctx->stream, sc, aux + 2 * batch, aux,
-                       0.0, tol, delta, 1, prm->restart_factor > 0 ? prm->restart_factor : 16.0);
+                       0.0, tol, delta, prm->restart_factor > 0 ? prm->restart_factor : 16.0);
     hipLaunchKernelGGL(k_bi_init, dim3(nr), dim3(64), 0, ctx->stream, sc, bc);
     II_HIP(ctx, hipGetLastError());
     // r = r0 = p = bhat (x0 = 0), ys = 0

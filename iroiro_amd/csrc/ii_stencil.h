@@ -329,7 +329,6 @@ struct GaugeLoR12 {
 // sunk to the final store), and the memory clobber keeps the next
 // direction's loads after it.  Without this the compiler keeps all eight
 // directions' spinors and links live at once (about 500 registers in FP64,
-// one wave per SIMD).
 template <typename C>
 __device__ __forceinline__ void pin_acc(C acc[4][3]) {
 #pragma unroll
@@ -710,24 +709,21 @@ __device__ __forceinline__ void wilson_hop_site(typename SpIn::C acc[4][3], cons
   const int op = 1 - out_par;
   const bool tf_fw = tbc_flip && sc.t == g.L[3] - 1;
   const bool tf_bw = tbc_flip && sc.t == 0;
-  // directions between register barriers: FP64 keeps four directions'
-  // loads in flight (256 VGPRs, 0.293 -> 0.281 ms at 32^3x64); the 32- and
-  // 16-bit hops pin every direction
-  constexpr int kDirGroup = std::is_same<R, double>::value ? 4 : 1;
+  // a register barrier after every direction (the 16-bit hop, its one caller)
   hop_dir<0, true, G5IN>(acc, in, gauge, neighbour(g, sc, hs, 0, true), out_par, hs, false);
-  if constexpr (1 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   { int nb = neighbour(g, sc, hs, 0, false); hop_dir<0, false, G5IN>(acc, in, gauge, nb, op, nb, false); }
-  if constexpr (2 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   hop_dir<1, true, G5IN>(acc, in, gauge, neighbour(g, sc, hs, 1, true), out_par, hs, false);
-  if constexpr (3 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   { int nb = neighbour(g, sc, hs, 1, false); hop_dir<1, false, G5IN>(acc, in, gauge, nb, op, nb, false); }
-  if constexpr (4 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   hop_dir<2, true, G5IN>(acc, in, gauge, neighbour(g, sc, hs, 2, true), out_par, hs, false);
-  if constexpr (5 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   { int nb = neighbour(g, sc, hs, 2, false); hop_dir<2, false, G5IN>(acc, in, gauge, nb, op, nb, false); }
-  if constexpr (6 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   hop_dir<3, true, G5IN>(acc, in, gauge, neighbour(g, sc, hs, 3, true), out_par, hs, tf_fw);
-  if constexpr (7 % kDirGroup == 0) II_DIR_BARRIER();
+  II_DIR_BARRIER();
   { int nb = neighbour(g, sc, hs, 3, false); hop_dir<3, false, G5IN>(acc, in, gauge, nb, op, nb, tf_bw); }
 }
 
