@@ -328,7 +328,7 @@ struct GaugeLoR12 {
 // asm statement (so every product of this direction is computed here, not
 // sunk to the final store), and the memory clobber keeps the next
 // direction's loads after it.  Without this the compiler keeps all eight
-// directions' spinors and links live at once (about 500 registers in FP64,
+// directions' spinors and links live at once.
 template <typename C>
 __device__ __forceinline__ void pin_acc(C acc[4][3]) {
 #pragma unroll

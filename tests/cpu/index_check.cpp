@@ -6,9 +6,9 @@
 //     one lattice step away in direction mu, and the backward neighbour of
 //     the forward neighbour is the site itself; the batched network's
 //     branch-free nb_of() gives the same site;
-//   * every site traversal the hop autotuner may pick (contiguous with 256
-//     or 128 threads per block, the XCD time-strip orders) and the 64-site
-//     tiles of the multi-rhs hop cover [0, V/2) exactly once;
+//   * every site traversal of the hops (contiguous in blocks of 256, 128 and
+//     64 sites, the XCD time-strip orders in blocks of 256 and of 64, on planes
+//     that 64 divides but 256 does not too) covers [0, V/2) exactly once;
 //   * the batched network's stage kernels take every (16-site tile, rhs)
 //     item once (ii_sweep.h: per-XCD slabs, t-fastest fronts, rhs groups),
 //     in the static order and in the dynamic order over the live rhs.
@@ -66,7 +66,8 @@ static void check_cover(const Geom& g, const HopOrder& o, int bs, const char* wh
 int main() {
   const int lats[][4] = {{2, 2, 2, 2},   {4, 4, 4, 4},   {6, 2, 2, 6},     {6, 4, 4, 6},
                          {4, 6, 2, 4},   {8, 8, 8, 16},  {16, 16, 16, 32}, {24, 24, 24, 48},
-                         {32, 32, 32, 64}, {12, 10, 6, 8},  {8, 8, 32, 32}};
+                         {32, 32, 32, 64}, {12, 10, 6, 8},  {8, 8, 32, 32},
+                         {16, 8, 2, 8},  {16, 24, 4, 16}, {12, 10, 14, 18}};
   for (const auto& L : lats) {
     const Geom g = make_geom(L);
     // neighbours
@@ -104,6 +105,10 @@ int main() {
     if (P % kBlock == 0 && g.L[3] % 8 == 0)
       for (int W : {1, 2, 4, 8, 16})
         if ((g.L[3] / 8) % W == 0) check_cover(g, HopOrder{1, W, P / kBlock}, kBlock, "strip");
+    // 64-site blocks (the split single-rhs hop) and tiles (the multi-rhs hop)
+    if (P % 64 == 0 && g.L[3] % 8 == 0)
+      for (int W : {1, 2, 4, 8, 16})
+        if ((g.L[3] / 8) % W == 0) check_cover(g, HopOrder{1, W, P / 64}, 64, "64-site strip");
     check_cover(g, HopOrder(), 64, "multi-rhs tiles");
     // batched network: every (tile, rhs) item exactly once for each stage's
     // block size, rhs count and grouping, on a 256-CU and a 38-CU device
