@@ -703,14 +703,16 @@ ii_status tune_hop(ii_context* ctx) {
 // give more, smaller blocks) and the tile order (contiguous per XCD, or
 // strips of W time slices, as for the single-rhs hop).  Timed with the
 // plain hop (no epilogue) of this precision on scratch fields of nrhs rhs,
-// one warm-up and 3 timed launches per candidate.  Candidates are 12, 6, 4, 3
-// and 2 rhs per block; with 12 rhs and more on 512 tiles and more only 12 and
-// 6, where the blocks fill the chip and the others lost in every precision.
-// us for 12 rhs, 12 / 6 / 4 / 3 / 2 per block:
-//   8^3x16 (64 tiles)    FP64 14.3 / 10.7 / 10.0 / 10.2 / 11.6, FP16 10.3 / 9.3 / 8.5 / 8.7 / 10.2
-//   12^3x24 (324)        FP64 39.1 / 35.4 / 38.1 / 43.2 / 52.0, FP16 15.5 / 14.7 / 14.0 / 19.8 / 22.9
-//   16^4 (512)           FP64 50.6 / 55.7 / 65.5 / 64.7 / 76.3, FP16 15.8 / 20.2 / 20.5 / 24.4 / 34.5
-//   32^3x64 (16384)      FP64 1860 / 1790 / 1840 / 2030 / 2530, FP16 480 / 560 / 580 / 740 / 1070
+// one warm-up and 3 timed launches per candidate.  Candidates are 12 (or all)
+// and 6 rhs per block, and 4, 3 and 2 below 512 tiles: with 2 to 24 rhs at 16^4
+// (512 tiles), 16^3x32 and 24^3x48 these won nowhere by more than 1%, on fewer
+// tiles by up to 13%, as more, smaller blocks reach more of the chip (timing
+// them at 24^3x48 with 10 rhs takes 10 ms).  us, 12 / 6 / 4 / 3 / 2 per block,
+// 12 rhs:
+//   8^3x16 (64 tiles)  FP64 13.5 / 9.8 / 8.9 / 9.1 / 10.4, FP16 9.5 / 8.8 / 7.7 / 8.3 / 9.8
+//   12^3x24 (324)      FP64 39.1 / 35.4 / 38.1 / 43.2 / 52.0, FP16 14.3 / 13.6 / 12.8 / 18.8 / 21.9
+//   16^4 (512)         FP64 50.6 / 55.7 / 65.5 / 64.7 / 76.3, FP16 15.8 / 20.2 / 20.5 / 24.4 / 34.5
+//   32^3x64 (16384)    FP64 1860 / 1790 / 1840 / 2030 / 2530, FP16 480 / 560 / 580 / 740 / 1070
 ii_status tune_mrhs(ii_context* ctx, int P, int nrhs) {
   if (P < 0 || P > 3 || nrhs < 2) return II_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -720,7 +722,7 @@ ii_status tune_mrhs(ii_context* ctx, int P, int nrhs) {
   const Geom& g = ctx->g;
   constexpr int TS = 64, RBMAX = 768 / 64;
   std::vector<int> rbs;
-  const bool few = (g.Vh + TS - 1) / TS < 512 || nrhs < RBMAX;
+  const bool few = (g.Vh + TS - 1) / TS < 512;
   for (int rb : {RBMAX, 6, 4, 3, 2})
     if ((rb >= 6 || few) && rb <= std::min(nrhs, RBMAX) && std::find(rbs.begin(), rbs.end(), rb) == rbs.end())
       rbs.push_back(rb);

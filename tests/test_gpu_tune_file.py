@@ -99,9 +99,8 @@ def test_file_of_an_untuned_context_leaves_the_hop_order(tmp_path, monkeypatch):
 
 
 def test_multi_rhs_shapes_timed_where_blocks_are_few(tmp_path):
-    """On a small lattice, and for fewer rhs than fill a block, the tuner times
-    every number of rhs per block: 64 tiles x 1 block of 12 rhs would leave most
-    of the chip idle."""
+    """On a small lattice the tuner times every number of rhs per block: 64 tiles
+    x 1 block of 12 rhs would leave most of the chip idle."""
     dims = (8, 8, 8, 16)
     ctx = ii.Context(dims)
     lat = orc.Lattice(dims)
