@@ -495,7 +495,7 @@ def main():
         "bound": "hbm", "achieved": hop_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": hop_gbs / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_src,
         "algorithmic_bytes": FP64_HOP_BYTES_PER_SITE * Vh,
-        "kernel": "k_hop FP64 even/odd Wilson hop, V/2 = %d sites/launch, 1536 B/site "
+        "kernel": "k_hop_split FP64 even/odd Wilson hop, V/2 = %d sites/launch, 1536 B/site "
                   "algorithmic" % Vh,
         "avg_ms": hop_ms, "gflops": HOP_FLOPS_PER_SITE * Vh / (hop_ms * 1e-3) / 1e9,
         "copy_kernel_gbs": copy_gbs}

@@ -351,7 +351,9 @@ enum { II_METHOD_CG = 0, II_METHOD_BICGSTAB = 1, II_METHOD_FGCR = 2 };
  * Schur system (Inverter_WilsonLike::invert, eoUtils.cpp:43-80) with a
  * device CG on Dhat^dag Dhat or (p->method) BiCGStab on Dhat; stops on the
  * FP64 true full-D residual.
- * Sources and solutions stay on the device.  out: one entry per rhs. */
+ * Sources and solutions stay on the device.  out: one entry per rhs.  sol is
+ * written when the solve (rhs by rhs: of each rhs) has ended, converged or not;
+ * another error leaves it, and a src that is the same field, as it was. */
 ii_status ii_propagator_solve(ii_context* ctx, double kappa, const ii_prop_params* p,
                               const ii_field* src, ii_field* sol, ii_solver_output* out);
 

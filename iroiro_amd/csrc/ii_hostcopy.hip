@@ -1,7 +1,7 @@
 // Copies between a caller's pageable arrays and the device.
 //
-// The runtime moves pageable memory at 15 (1.6 MB) to 30 GB/s up and 14 to 17
-// GB/s down; the link takes 56 GB/s from pinned memory in pieces of some MiB
+// The runtime moves pageable memory at 15 (1.6 MB) to 29 GB/s (127 MB) up and
+// 14 to 17 GB/s down; the link takes 56 GB/s from pinned memory in pieces of some MiB
 // (21 GB/s in pieces of 512 KiB, 30 in 1 MiB).  Here the bytes go through
 // pinned slots: a thread moves one piece between the caller's array and a slot
 // while its other slot is on the link.  One thread copies 28

@@ -19,9 +19,11 @@
 // path, pre-arranged per lane (8 bf16 = 16 bytes) and staged in LDS once per
 // block.  C rows are (out channel, spin, re/im), accumulated in FP32 over
 // the 9 paths, the next path's loads requested before a path's products (8x8
-// at 16^3x32 158 -> 144 us, 1x8 83 -> 69 us; the FP32 transports' VALU work, 400
-// instructions a path and lane, is 70% of the time that is left).  The adjoint layer is the same kernel with the paths
-// mirrored and W -> W^dag (channel-transposed): T_{+mu}^dag = T_{-mu}.
+// at 16^3x32 158 -> 144 us, 1x8 83 -> 69 us; of the 144, the issue of the FP32
+// transports, about 400 VALU instructions a path and wave, is 48: 8192 tiles x
+// 9 paths on 1024 SIMDs at 4 cycles each).  The adjoint layer is the same
+// kernel with the paths mirrored and W -> W^dag (channel-transposed):
+// T_{+mu}^dag = T_{-mu}.
 //
 // Weight gradient: FP32 matrix cores, gw[d][o][i] = sum_{x,c} g[o](x)
 // conj(T_d in[i](x)), per-block partials in FP32 then a fixed-order FP64 sum.
@@ -350,8 +352,8 @@ __global__ void __launch_bounds__(kLayerThreads, 2) k_net_layer(LayerArgs a) {
 // registers for all paths, and the next path's spinors and links are requested
 // before a path's products.  Two blocks per CU (registers).  One pair's
 // gradients at 16^3x32 (two 8x8 layers, one 1x8, one 8x1): 0.89 ms, where FP32
-// products on the VALU took 2.0 ms; with the reduction below, net_loss_grad of
-// 4 pairs 44.7 -> 18.9 ms on host arrays.  8x8 is bound by the FP32 matrix rate
+// products on the VALU took 2.0 ms (368 us a layer with 8x8 channels, 86 us with
+// one).  8x8 is bound by the FP32 matrix rate
 // (221 kFLOP per site), the others by the transports' loads.  Error against 64
 // bits on Gaussian fields, 1x8 / 8x8 / 8x1: 1.4 / 3.6 / 1.4e-7 on the VALU,
 // 1.2 / 2.5 / 1.2e-7 here (one-channel sums go over 8 accumulators for that).

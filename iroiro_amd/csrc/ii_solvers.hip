@@ -436,6 +436,10 @@ ii_status ddagdP(ii_context* ctx, int P, double kappa, const SF& f, const SF& ou
 // partials (hop_dot_parts per rhs).  With sig (one shift per rhs) the operator
 // is A + sig: <p, (A + sig) p> = |q|^2 + sig |p|^2 (pnorm: hop_blocks partial
 // sums of |p|^2 per rhs) and r -= alpha (Dhat^dag q + sig p).
+// The arithmetic is the inner precision's: in FP32 and 16 bits the 24-term site
+// sums of |q|^2 and |r|^2 and the residual update, alpha and sig rounded with it,
+// run in FP32 (hop_epilogue), the sums over sites, the scalars and y += alpha p
+// in FP64; single-rhs FP32 hops form theirs in FP64 (hop_epilogue_spin).
 static_assert(sizeof(RUScal) % sizeof(double) == 0, "RUScal is read as a double array");
 ii_status ddagd_cg_fused(ii_context* ctx, int P, double kappa, const SF& p, const SF& r,
                          const SF& q, const SF& t, RUScal* sc, double* partials, int nrhs,
@@ -1365,6 +1369,9 @@ ii_status multishift_sloppy(ii_context* ctx, double kappa, float2* x32, const do
 // take the propagator's fused steps with the shift in their scalars and
 // epilogues (ddagd_cg_fused), its deferred solution update and its joined
 // reliable updates; the FP64 residual of an update is its last hop's epilogue.
+// What the inner precision rounds (ddagd_cg_fused) changes the iterations only:
+// a shift is done when its FP64 residual, formed from the FP64 solution every
+// two decades (one in BF16) and at the end, is below tol |b|.
 ii_status shifted_refine(ii_context* ctx, double kappa, const double* shifts, int nrhs,
                          const double2* b64, double2* x64, double tol, int P, int maxiter,
                          ii_solver_output* outs) {

@@ -121,10 +121,10 @@ def test_mixed_multishift_true_residuals(precision, nshift):
 @pytest.mark.parametrize("method,precision", [("cg", "double"), ("cg", "half"),
                                               ("bicgstab", "single"), ("fgcr", "single")])
 def test_propagator_parities_in_place(method, precision, nrhs):
-    """The solvers read the sources' parities and build the solution where they
-    lie: the sources are left as they were, every rhs reaches the true residual
-    1e-10 by the oracle's operator, and a field that is source and solution at
-    once is solved too."""
+    """The solvers read the sources' parities where they lie and write the
+    solution's: the sources are left as they were, every rhs reaches the true
+    residual 1e-10 by the oracle's operator, and a field that is source and
+    solution at once is solved too."""
     dims = (6, 4, 2, 10)
     kappa = 0.12
     lat = orc.Lattice(dims)
