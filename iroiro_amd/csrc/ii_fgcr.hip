@@ -232,9 +232,9 @@ k_g_rupd(Geom g, const float2* __restrict__ W, size_t slot, int k, float2* __res
 // k >= 1: every scalar the direction needs comes from the epilogue of the hop
 // that forms w_k (kEpiGram with dv = w_{k-1}, p = r, while w_k is in
 // registers), then one pass for the update.  Against a pass of its own for
-// the sums this saves one read of w_k: 12 rhs at 32^3x64, hop + pass +
-// scalars 0.98 + 0.49 + 0.04 ms before, 1.36 + 0.02 ms with the epilogue (the
-// two added reads run at the HBM rate).
+// the sums this saves one read of w_k: 12 rhs at 32^3x64, part of them done,
+// hop + pass + scalars 0.98 + 0.49 + 0.04 ms before, 1.36 + 0.02 ms with the
+// epilogue; with all of them live the hop takes 1.59 ms, 1.14 without the sums.
 //
 // beta = <w_{k-1}, w_k> / |w_{k-1}|^2; for w' = w_k - beta w_{k-1}:
 // |w'|^2 = |w_k|^2 - |<w_{k-1}, w_k>|^2 / |w_{k-1}|^2 and
