@@ -425,6 +425,9 @@ ii_status ii_net_layer_wgrad(ii_context* ctx, int layer, const double* in,
  * gradient with respect to every layer's weights (concatenated). */
 ii_status ii_net_loss_grad(ii_context* ctx, int npairs, const double* b_even,
                            const double* y_even, double* loss, float* grads);
+/* The same for pairs in arrays of their own: b_even[k], y_even[k]. */
+ii_status ii_net_loss_grad_pairs(ii_context* ctx, int npairs, const double* const* b_even,
+                                 const double* const* y_even, double* loss, float* grads);
 /* z = M r on even half fields (esec order, 24*V/2 doubles). */
 ii_status ii_net_apply(ii_context* ctx, const double* r_even, double* z_even);
 /* z = M r for nrhs even half fields back to back, all rhs in one launch per

@@ -1013,22 +1013,20 @@ class LearnedPreconditioner:
         if not bs or len(bs) != len(ys) or any(v.size != nh for v in bs + ys):
             bs = _lib.as_f64(np.concatenate(bs), nh * len(bs)).reshape(-1, nh)
             ys = _lib.as_f64(np.concatenate(ys), nh * len(bs)).reshape(-1, nh)
+        bs, ys = [_lib.as_f64(v) for v in bs], [_lib.as_f64(v) for v in ys]
         sizes = [int(np.prod(self.shape(l))) for l in range(_lib.NET_LAYERS)]
-        total, loss, one = None, 0.0, ctypes.c_double()
-        for b, y in zip(bs, ys):  # one pair a call: no copy that joins them
-            b, y = _lib.as_f64(b), _lib.as_f64(y)
-            f = np.empty(2 * sum(sizes), np.float32)
-            self.ctx.check(self._L().ii_net_loss_grad(self.ctx.handle, 1, _lib.dptr(b),
-                                                      _lib.dptr(y), ctypes.byref(one),
-                                                      _lib.fptr(f)), "ii_net_loss_grad")
-            loss += one.value
-            total = f if total is None else total + f
-        c = total.view(np.complex64)
+        f = np.empty(2 * sum(sizes), np.float32)
+        loss = ctypes.c_double()
+        at = ctypes.POINTER(ctypes.c_double) * len(bs)
+        self.ctx.check(self._L().ii_net_loss_grad_pairs(
+            self.ctx.handle, len(bs), at(*map(_lib.dptr, bs)), at(*map(_lib.dptr, ys)),
+            ctypes.byref(loss), _lib.fptr(f)), "ii_net_loss_grad_pairs")
+        c = f.view(np.complex64)
         grads, off = [], 0
         for l, n in enumerate(sizes):
             grads.append(c[off:off + n].reshape(self.shape(l)))
             off += n
-        return loss, grads
+        return loss.value, grads
 
     def apply(self, r):
         r = _lib.as_f64(r, 24 * self.ctx.V // 2)

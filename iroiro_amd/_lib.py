@@ -33,7 +33,7 @@ EXPORTS = [
     "ii_multishift_mixed",
     "ii_qprop_multishift",
     "ii_net_init", "ii_net_set_weights", "ii_net_get_weights", "ii_net_layer_apply",
-    "ii_net_layer_wgrad", "ii_net_loss_grad", "ii_net_apply", "ii_net_apply_batched",
+    "ii_net_layer_wgrad", "ii_net_loss_grad", "ii_net_loss_grad_pairs", "ii_net_apply", "ii_net_apply_batched",
     "ii_net_train", "ii_net_save",
     "ii_net_load", "ii_net_bench", "ii_bench_net_batched", "ii_net_tune", "ii_fgcr_solve",
     "ii_autotune", "ii_tune_save", "ii_tune_load", "ii_bench_hop", "ii_bench_copy",
@@ -174,6 +174,7 @@ def load():
         "ii_net_layer_apply": [vp, ci, ci, dp, dp],
         "ii_net_layer_wgrad": [vp, ci, dp, dp, fp],
         "ii_net_loss_grad": [vp, ci, dp, dp, dp, fp],
+        "ii_net_loss_grad_pairs": [vp, ci, ctypes.POINTER(dp), ctypes.POINTER(dp), dp, fp],
         "ii_net_apply": [vp, dp, dp],
         "ii_net_apply_batched": [vp, ci, dp, dp],
         "ii_net_train": [vp, cd, ctypes.POINTER(TrainParamsC), ctypes.POINTER(TrainReportC)],

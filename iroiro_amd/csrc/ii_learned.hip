@@ -1236,6 +1236,57 @@ ii_status learned_propagator(ii_context* ctx, double kappa, const ii_prop_params
 
 using namespace ii;
 
+// b(k), y(k): the host arrays of pair k
+template <typename At>
+static ii_status loss_grad(ii_context* ctx, int npairs, const At& b, const At& y, double* loss,
+                           float* grads) {
+  II_CHECK(enter(ctx));
+  Net* N = nullptr;
+  II_CHECK(net_get(ctx, &N));
+  if (!N->init) return set_error(ctx, II_ERR_STATE, "network not initialised");
+  const Geom& g = ctx->g;
+  const size_t nh = (size_t)24 * g.Vh;
+  const size_t he = half_elems(g);
+  II_CHECK(stage(ctx, N, 2 * nh));
+  double2 *b64 = nullptr, *y64 = nullptr;
+  II_CHECK(dev_alloc(ctx, &N->fw[3], he));
+  II_CHECK(dev_alloc(ctx, &N->fw[4], he));
+  b64 = N->fw[3];
+  y64 = N->fw[4];
+  float2 *bfull = nullptr, *yhalf = nullptr;
+  II_CHECK(dev_alloc(ctx, &N->fw[5], he * 2));  // FP32 storage: full b (24*stride float2) + y
+  bfull = (float2*)N->fw[5];
+  yhalf = bfull + 24 * (size_t)g.stride;
+  II_CHECK(zero_grads(ctx, N));
+  double L = 0.0;
+  for (int k = 0; k < npairs; ++k) {
+    II_CHECK(copy_to_device(ctx, N->stage, b(k), nh * sizeof(double)));
+    II_CHECK(copy_to_device(ctx, N->stage + nh, y(k), nh * sizeof(double)));
+    II_CHECK(pack_half_spinor(ctx, N->stage, b64));
+    II_CHECK(pack_half_spinor(ctx, N->stage + nh, y64));
+    hipLaunchKernelGGL(k_net_to32, dim3(blocks_for(g.Vh)), dim3(kBlock), 0, ctx->stream, g, b64,
+                       bfull, 1);
+    hipLaunchKernelGGL(k_net_to32, dim3(blocks_for(g.Vh)), dim3(kBlock), 0, ctx->stream, g, y64,
+                       yhalf, 0);
+    II_HIP(ctx, hipGetLastError());
+    double yy[2];
+    II_CHECK(cdot(ctx, N, y64, y64, yy));
+    II_CHECK(pair_loss(ctx, N, bfull, yhalf, 1.0 / yy[0], 1.0f, &L));
+    II_CHECK(backward(ctx, N, 1.0f));
+  }
+  *loss = L;
+  if (grads) {
+    size_t off = 0;
+    for (int l = 0; l < kNL; ++l) {
+      II_HIP(ctx, hipMemcpyAsync(grads + 2 * off, N->L[l].gacc, N->L[l].nw * sizeof(float2),
+                                 hipMemcpyDeviceToHost, ctx->stream));
+      off += N->L[l].nw;
+    }
+  }
+  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  return II_OK;
+}
+
 extern "C" {
 
 ii_status ii_net_init(ii_context* ctx, double kappa, double noise, unsigned long long seed) {
@@ -1374,51 +1425,25 @@ ii_status ii_net_layer_wgrad(ii_context* ctx, int layer, const double* in, const
 ii_status ii_net_loss_grad(ii_context* ctx, int npairs, const double* b_even, const double* y_even,
                            double* loss, float* grads) {
   if (!ctx || npairs < 1 || !b_even || !y_even || !loss) return II_ERR_BAD_ARG;
-  II_CHECK(enter(ctx));
-  Net* N = nullptr;
-  II_CHECK(net_get(ctx, &N));
-  if (!N->init) return set_error(ctx, II_ERR_STATE, "network not initialised");
-  const Geom& g = ctx->g;
-  const size_t nh = (size_t)24 * g.Vh;
-  const size_t he = half_elems(g);
-  II_CHECK(stage(ctx, N, 2 * nh));
-  double2 *b64 = nullptr, *y64 = nullptr;
-  II_CHECK(dev_alloc(ctx, &N->fw[3], he));
-  II_CHECK(dev_alloc(ctx, &N->fw[4], he));
-  b64 = N->fw[3];
-  y64 = N->fw[4];
-  float2 *bfull = nullptr, *yhalf = nullptr;
-  II_CHECK(dev_alloc(ctx, &N->fw[5], he * 2));  // FP32 storage: full b (24*stride float2) + y
-  bfull = (float2*)N->fw[5];
-  yhalf = bfull + 24 * (size_t)g.stride;
-  II_CHECK(zero_grads(ctx, N));
-  double L = 0.0;
-  for (int k = 0; k < npairs; ++k) {
-    II_CHECK(copy_to_device(ctx, N->stage, b_even + k * nh, nh * sizeof(double)));
-    II_CHECK(copy_to_device(ctx, N->stage + nh, y_even + k * nh, nh * sizeof(double)));
-    II_CHECK(pack_half_spinor(ctx, N->stage, b64));
-    II_CHECK(pack_half_spinor(ctx, N->stage + nh, y64));
-    hipLaunchKernelGGL(k_net_to32, dim3(blocks_for(g.Vh)), dim3(kBlock), 0, ctx->stream, g, b64,
-                       bfull, 1);
-    hipLaunchKernelGGL(k_net_to32, dim3(blocks_for(g.Vh)), dim3(kBlock), 0, ctx->stream, g, y64,
-                       yhalf, 0);
-    II_HIP(ctx, hipGetLastError());
-    double yy[2];
-    II_CHECK(cdot(ctx, N, y64, y64, yy));
-    II_CHECK(pair_loss(ctx, N, bfull, yhalf, 1.0 / yy[0], 1.0f, &L));
-    II_CHECK(backward(ctx, N, 1.0f));
-  }
-  *loss = L;
-  if (grads) {
-    size_t off = 0;
-    for (int l = 0; l < kNL; ++l) {
-      II_HIP(ctx, hipMemcpyAsync(grads + 2 * off, N->L[l].gacc, N->L[l].nw * sizeof(float2),
-                                 hipMemcpyDeviceToHost, ctx->stream));
-      off += N->L[l].nw;
-    }
-  }
-  II_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return II_OK;
+  struct At {
+    const double* p;
+    size_t nh;
+    const double* operator()(int k) const { return p + k * nh; }
+  };
+  const size_t nh = (size_t)24 * ctx->g.Vh;
+  return loss_grad(ctx, npairs, At{b_even, nh}, At{y_even, nh}, loss, grads);
+}
+
+ii_status ii_net_loss_grad_pairs(ii_context* ctx, int npairs, const double* const* b_even,
+                                 const double* const* y_even, double* loss, float* grads) {
+  if (!ctx || npairs < 1 || !b_even || !y_even || !loss) return II_ERR_BAD_ARG;
+  for (int k = 0; k < npairs; ++k)
+    if (!b_even[k] || !y_even[k]) return II_ERR_BAD_ARG;
+  struct At {
+    const double* const* p;
+    const double* operator()(int k) const { return p[k]; }
+  };
+  return loss_grad(ctx, npairs, At{b_even}, At{y_even}, loss, grads);
 }
 
 ii_status ii_net_apply(ii_context* ctx, const double* r_even, double* z_even) {

@@ -398,3 +398,20 @@ def test_fgcr_graph_equals_eager_and_network_saves_directions():
         assert d_net < d_plain
     finally:
         ctx.close()
+
+
+def test_loss_grad_of_pairs_in_arrays_of_their_own(env):
+    """The same bits as the pairs back to back in one array."""
+    import ctypes
+    from iroiro_amd import _lib
+    lat, u, ctx, net = env
+    rng = np.random.default_rng(41)
+    bs, ys = rng.normal(size=(2, 3, lat.half_size))
+    loss, grads = net.loss_grad(list(bs), list(ys))
+    f = np.empty(2 * sum(g.size for g in grads), np.float32)
+    one = ctypes.c_double()
+    assert _lib.load().ii_net_loss_grad(ctx.handle, 3, _lib.dptr(bs.ravel()),
+                                        _lib.dptr(ys.ravel()), ctypes.byref(one),
+                                        _lib.fptr(f)) == _lib.II_OK
+    assert one.value == loss
+    assert np.array_equal(f.view(np.complex64), np.concatenate([g.ravel() for g in grads]))

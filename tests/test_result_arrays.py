@@ -57,3 +57,20 @@ def test_loss_grad_refuses_pairs_that_do_not_match(bs, ys):
     ctx = types.SimpleNamespace(V=16, handle=None)
     with pytest.raises(ValueError):
         ii.LearnedPreconditioner(ctx).loss_grad(bs, ys)
+
+
+def test_loss_grad_is_one_call_of_the_library():
+    """Several pairs, in arrays of their own: one call, that is one download and
+    one synchronisation, and no copy that joins them."""
+    calls = []
+
+    def record(handle, n, bs, ys, loss, grads):
+        calls.append([[ctypes.addressof(v[k].contents) for k in range(n)] for v in (bs, ys)])
+        return _lib.II_OK
+
+    ctx = types.SimpleNamespace(V=16, handle=None, check=lambda st, what: None)
+    net = ii.LearnedPreconditioner(ctx)
+    net._L = lambda: types.SimpleNamespace(ii_net_loss_grad_pairs=record)
+    bs, ys = list(np.zeros((3, 192))), [np.zeros(192) for _ in range(3)]
+    net.loss_grad(bs, ys)
+    assert calls == [[[v.ctypes.data for v in bs], [v.ctypes.data for v in ys]]]
