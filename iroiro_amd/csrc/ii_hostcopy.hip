@@ -5,14 +5,14 @@
 // (21 GB/s in pieces of 512 KiB, 30 in 1 MiB).  Here the bytes go through
 // pinned slots: a thread moves one piece between the caller's array and a slot
 // while its other slot is on the link.  One thread copies 28
-// GB/s, so a large copy takes two (three and four were no faster); the second
-// is started for the call and joined before it returns.  127 MB: 29 -> 43 GB/s
-// up, 17 -> 44 GB/s down; 25 MB: 32 -> 37 and 17 -> 32; 1.6 MB: 15 -> 18 and
-// 14 -> 17.
+// GB/s, so a large copy takes two (three and four were no faster).  127 MB: 29
+// -> 43 GB/s up, 17 -> 44 GB/s down; 25 MB: 32 -> 37 and 17 -> 32; 1.6 MB: 15 ->
+// 18 and 14 -> 17.
 #include "ii_internal.h"
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <exception>
 #include <mutex>
@@ -25,8 +25,8 @@ namespace {
 
 constexpr int kPipeThreads = 2;                  // this one and a helper
 constexpr size_t kPieceMax = (size_t)4 << 20;    // bytes of a slot
-constexpr size_t kThreadBytes = (size_t)4 << 20; // a second thread from twice that: it takes
-                                                 // about 50 us to start
+constexpr size_t kThreadBytes = (size_t)4 << 20; // the helper from twice that: it takes some
+                                                 // tens of us to wake
 // Smaller copies are the runtime's: its own staging has less latency than a
 // slot and its event.  One Dhat on host arrays, us, through the runtime /
 // through the slots, by the bytes each way: 72 KB 52 / 63, 243 KB 65 / 100,
@@ -42,12 +42,61 @@ constexpr size_t kDirect = (size_t)1 << 20;
 // never waits for another context's kernels or copies, its own stream orders
 // the uses of a set in flight, and there are never more sets than contexts
 // that copy: programs that use their contexts one after the other pin one.
+//
+// The helper thread belongs to the set and sleeps between copies.  It takes
+// pieces while there are any; a copy waits only for pieces that it has taken,
+// not for it to wake.  (A thread started and joined for each copy waited a time
+// slice of 4 ms for a core while the caller's BLAS threads spun between calls:
+// Dhat at 16^3x32 up to 3.9 ms, 0.9 alone.)
+struct HostJob {
+  virtual void run() = 0;
+};
 struct HostSet {
   char* pin = nullptr;
   hipEvent_t ev[2 * kPipeThreads] = {};
   ii_context* owner = nullptr;  // whose stream may have pieces in flight
   bool busy = false;            // a copy is running on it
   HostSet* next = nullptr;
+  std::mutex jmu;
+  std::condition_variable jcv;
+  std::thread helper;
+  bool tried = false, stop = false, active = false;
+  HostJob* job = nullptr;
+  // offers j to the helper
+  void post(HostJob* j) {
+    if (!tried) {
+      tried = true;
+      try {
+        helper = std::thread([this] { serve(); });
+      } catch (const std::exception&) {
+        // no thread to be had: the callers take all the pieces
+      }
+    }
+    std::lock_guard<std::mutex> l(jmu);
+    job = j;
+    jcv.notify_all();
+  }
+  // the job is not offered any more, and the helper is not in it
+  void retract() {
+    std::unique_lock<std::mutex> l(jmu);
+    job = nullptr;
+    jcv.wait(l, [&] { return !active; });
+  }
+  void serve() {
+    std::unique_lock<std::mutex> l(jmu);
+    for (;;) {
+      jcv.wait(l, [&] { return stop || job; });
+      if (stop) return;
+      HostJob* j = job;
+      job = nullptr;
+      active = true;
+      l.unlock();
+      j->run();
+      l.lock();
+      active = false;
+      jcv.notify_all();
+    }
+  }
   bool create() {
     bool ok = hipHostMalloc((void**)&pin, 2 * kPipeThreads * kPieceMax) == hipSuccess;
     for (auto& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
@@ -62,6 +111,12 @@ struct HostSet {
     return true;
   }
   ~HostSet() {
+    {
+      std::lock_guard<std::mutex> l(jmu);
+      stop = true;
+      jcv.notify_all();
+    }
+    if (helper.joinable()) helper.join();
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     if (pin) (void)hipHostFree(pin);
@@ -144,7 +199,7 @@ static void give_set(ii_context* ctx, HostSet* s) {
 // pieces of [0, bytes) in order until none is left or a thread has failed, e is
 // the thread's error.  After a failure nothing of the copy is left in flight.
 template <typename Piece>
-static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
+static ii_status run_pieces(ii_context* ctx, HostSet* H, size_t bytes, const Piece& work) {
   const int want = (int)std::max<size_t>(1, bytes / kThreadBytes);
   const int nthr = std::min(kPipeThreads, want);
   size_t piece = (bytes + 2 * nthr - 1) / (2 * nthr);
@@ -152,7 +207,7 @@ static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
   const size_t n = (bytes + piece - 1) / piece;
   std::atomic<size_t> next{0};
   std::atomic<int> err{hipSuccess};
-  auto run = [&](int t) {
+  auto pieces = [&](int t) {
     hipError_t e = t ? hipSetDevice(ctx->device) : hipSuccess;
     work(t, [&](size_t* first, size_t* len) {
       const size_t k = e == hipSuccess && err == hipSuccess ? next++ : n;
@@ -163,14 +218,14 @@ static ii_status run_pieces(ii_context* ctx, size_t bytes, const Piece& work) {
     }, e);
     if (e != hipSuccess) err = e;
   };
-  std::thread helper;
-  if (nthr > 1) try {
-      helper = std::thread(run, 1);
-    } catch (const std::exception&) {
-      // no thread to be had: this one takes all the pieces
-    }
-  run(0);
-  if (helper.joinable()) helper.join();
+  struct Job final : HostJob {
+    const decltype(pieces)& f;
+    explicit Job(const decltype(pieces)& f) : f(f) {}
+    void run() override { f(1); }
+  } job(pieces);
+  if (nthr > 1) H->post(&job);
+  pieces(0);
+  if (nthr > 1) H->retract();
   if (err != hipSuccess) {
     (void)hipStreamSynchronize(ctx->stream);
     return set_error(ctx, II_ERR_DEVICE,
@@ -196,7 +251,7 @@ ii_status copy_to_device(ii_context* ctx, void* dst, const void* src, size_t byt
     if (bytes >= kDirect) II_HIP(ctx, hipStreamSynchronize(ctx->stream));  // src has been read
     return II_OK;
   }
-  const ii_status st = run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
+  const ii_status st = run_pieces(ctx, H, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first = 0, len = 0;
     for (int i = 0; take(&first, &len); ++i) {
       const int slot = 2 * t + (i & 1);
@@ -220,7 +275,7 @@ ii_status copy_to_host(ii_context* ctx, void* dst, const void* src, size_t bytes
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return II_OK;
   }
-  const ii_status st = run_pieces(ctx, bytes, [&](int t, auto&& take, hipError_t& e) {
+  const ii_status st = run_pieces(ctx, H, bytes, [&](int t, auto&& take, hipError_t& e) {
     size_t first[2] = {0, 0}, len[2] = {0, 0};
     auto request = [&](int b) {
       const int slot = 2 * t + b;

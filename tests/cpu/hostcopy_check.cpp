@@ -6,6 +6,9 @@
 // Exits non-zero on the first violation.
 #include "../../iroiro_amd/csrc/ii_hostcopy.hip"
 
+#include <dlfcn.h>
+#include <pthread.h>
+
 #include <chrono>
 #include <condition_variable>
 #include <cstdio>
@@ -103,6 +106,28 @@ Stream* of(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
 Event* of(hipEvent_t e) { return reinterpret_cast<Event*>(e); }
 
 }  // namespace sim
+
+// threads started while `late` is set get no core for that many milliseconds
+namespace sim {
+std::atomic<int> late{0};
+struct Start {
+  void* (*f)(void*);
+  void* arg;
+  int ms;
+};
+void* late_start(void* v) {
+  Start s = *static_cast<Start*>(v);
+  delete static_cast<Start*>(v);
+  std::this_thread::sleep_for(std::chrono::milliseconds(s.ms));
+  return s.f(s.arg);
+}
+}  // namespace sim
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* arg) {
+  using Fn = int (*)(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*);
+  static Fn real = (Fn)dlsym(RTLD_NEXT, "pthread_create");
+  if (!sim::late) return real(t, a, f, arg);
+  return real(t, a, sim::late_start, new sim::Start{f, arg, sim::late});
+}
 
 extern "C" {
 hipError_t hipSetDevice(int) { return hipSuccess; }
@@ -319,6 +344,21 @@ void pinned_memory() {
   }
 }
 
+// a copy does not wait for its helper thread to get a core
+void late_helper() {
+  const size_t n = 37 << 20;
+  std::vector<char> src = pattern(n, 10), dev(n), dst(n);
+  Ctx a;
+  sim::late = 3000;
+  const auto t0 = std::chrono::steady_clock::now();
+  upload(a, dev, src);
+  download(a, dst, dev);
+  const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  sim::late = 0;
+  CHECK(dst == src, "copies without a helper");
+  CHECK(s < 1.5, "copies waited %.1f s for their helper", s);
+}
+
 // as many sets of slots as contexts with copies in flight, and one for
 // contexts used in turn
 void set_count() {
@@ -375,6 +415,7 @@ int main() {
   sim::no_pins = false;
   set_count();
   failures();
+  late_helper();
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
   round_trips();  // the slots come back after the last context gave them up
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
