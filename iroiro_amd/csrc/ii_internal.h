@@ -102,6 +102,7 @@ struct ii_context {
   void* host_pin = nullptr;       // pinned host block of the multishift scalars
   size_t host_pin_len = 0;
   void* host_pipe = nullptr;      // the device's pinned slots, once copied with (ii_hostcopy.hip)
+  size_t host_moved = 0;          // bytes it has copied without slots
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // autotuned launch shapes
   ii::HopOrder hop_order;

@@ -208,7 +208,10 @@ namespace {
 struct Ctx {
   sim::Stream s;
   ii_context c;
-  Ctx() { c.stream = reinterpret_cast<hipStream_t>(&s); }
+  explicit Ctx(bool fresh = false) {
+    c.stream = reinterpret_cast<hipStream_t>(&s);
+    if (!fresh) c.host_moved = kPinAfter;  // a context that has copied a lot
+  }
   // earlier work on the stream, ms long
   void kernel(int ms) {
     s.push([ms] { std::this_thread::sleep_for(std::chrono::milliseconds(ms)); });
@@ -344,6 +347,29 @@ void pinned_memory() {
   }
 }
 
+// a context pins nothing before it has copied a lot, unless a set is idle
+void short_lived() {
+  const size_t n = 37 << 20;
+  std::vector<char> src = pattern(n, 11), dev(n), dst(n);
+  const int before = sim::pin_calls;
+  {
+    Ctx a(true);
+    upload(a, dev, src);
+    download(a, dst, dev);
+    CHECK(dst == src && sim::pin_calls == before, "a short-lived context pinned a set");
+    upload(a, dev, src);
+    CHECK(sim::pin_calls == before, "pinned after 111 MiB");
+    upload(a, dev, src);
+    CHECK(sim::pin_calls == before + 1, "not pinned after 148 MiB");
+    Ctx b(true);
+    a.s.sync();
+    const int copies = sim::copies;
+    upload(b, dev, src);
+    CHECK(sim::copies > copies + 1 && sim::pin_calls == before + 1, "an idle set is taken");
+  }
+  CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
+}
+
 // a copy does not wait for its helper thread to get a core
 void late_helper() {
   const size_t n = 37 << 20;
@@ -416,6 +442,7 @@ int main() {
   set_count();
   failures();
   late_helper();
+  short_lived();
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);
   round_trips();  // the slots come back after the last context gave them up
   CHECK(sim::pins == 0, "%d pinned blocks left", (int)sim::pins);

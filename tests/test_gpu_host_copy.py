@@ -9,6 +9,18 @@ import iroiro_amd as ii
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def idle_slots():
+    """A context that has copied enough to have a set of pinned slots: the
+    contexts of a test take it from their first copy on."""
+    ctx = ii.Context((8, 8, 8, 16))
+    u = np.zeros(72 * ctx.V)
+    for _ in range(32):
+        ctx.upload_gauge(u)
+    yield
+    ctx.close()
+
+
 @pytest.mark.parametrize("dims", [(2, 2, 2, 2), (4, 4, 4, 8), (6, 4, 2, 10), (8, 8, 8, 16),
                                   (14, 10, 12, 18), (22, 14, 18, 26)])
 def test_field_and_gauge_round_trip(dims):
@@ -39,7 +51,7 @@ def test_two_contexts_of_a_device_copying_at_once():
         def work(k):
             rng = np.random.default_rng(10 + k)
             f = ii.DeviceField(ctxs[k], "full", 1)
-            for i in range(8):
+            for i in range(16):  # 186 MB: the second context pins slots of its own on the way
                 a = rng.normal(size=f.size)
                 f.upload(0, a)
                 if not np.array_equal(f.download(0), a):
