@@ -135,30 +135,36 @@ struct HostPipe {
 constexpr int kPipeDevices = 64;  // as many as noalloc_setup lets a context be created on
 static HostPipe g_pipe[kPipeDevices];
 
-// frees the sets beyond the number of contexts that may use one (mu held)
-static void trim(HostPipe* H) {
-  for (HostSet** at = &H->sets; *at && H->nsets > H->users;) {
-    HostSet* s = *at;
-    if (s->busy || (s->owner && !s->complete())) {
-      at = &s->next;
-      continue;
-    }
-    *at = s->next;
-    --H->nsets;
-    delete s;
-  }
-}
-
-// The stream of a context that goes has been waited for.
+// The stream of a context that goes has been waited for.  Sets beyond the number
+// of contexts that may use one are freed, outside the lock: freeing pinned
+// memory may wait for the device.
 void host_pipe_release(ii_context* ctx) {
   HostPipe* H = static_cast<HostPipe*>(ctx->host_pipe);
   if (!H) return;
-  std::lock_guard<std::mutex> lock(H->mu);
-  for (HostSet* s = H->sets; s; s = s->next)
-    if (s->owner == ctx) s->owner = nullptr;
-  --H->users;
-  trim(H);
   ctx->host_pipe = nullptr;
+  HostSet* gone = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(H->mu);
+    for (HostSet* s = H->sets; s; s = s->next)
+      if (s->owner == ctx) s->owner = nullptr;
+    --H->users;
+    for (HostSet** at = &H->sets; *at && H->nsets > H->users;) {
+      HostSet* s = *at;
+      if (s->busy || (s->owner && !s->complete())) {
+        at = &s->next;
+        continue;
+      }
+      *at = s->next;
+      --H->nsets;
+      s->next = gone;
+      gone = s;
+    }
+  }
+  while (gone) {
+    HostSet* s = gone;
+    gone = s->next;
+    delete s;
+  }
 }
 
 // a set for a copy of ctx of so many bytes; null if none is to be pinned for it

@@ -100,6 +100,7 @@ struct Event {
 
 std::atomic<int> pins{0}, pin_calls{0}, fail_copy{-1}, copies{0};
 std::atomic<bool> no_pins{false};
+Mark* free_gate = nullptr;  // pinned memory is freed when the device lets go
 const char *pinned_lo = nullptr, *pinned_hi = nullptr;  // the caller's pinned memory
 
 Stream* of(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
@@ -139,6 +140,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   return hipSuccess;
 }
 hipError_t hipHostFree(void* p) {
+  if (sim::free_gate) sim::free_gate->wait();
   std::free(p);
   --sim::pins;
   return hipSuccess;
@@ -329,6 +331,39 @@ void no_waiting() {
   }
 }
 
+// a context that goes, and waits for the device to give up its slots, holds up
+// no other one's copies
+void closing() {
+  const size_t n = 12 << 20;
+  std::vector<char> src = pattern(n, 12), da(n), db(n), hb(n);
+  sim::Mark gate, done;
+  Ctx b;
+  auto a = std::make_unique<Ctx>();
+  a->kernel(20);
+  upload(*a, da, src);
+  upload(b, db, src);  // a set of its own
+  b.s.sync();
+  sim::free_gate = &gate;
+  std::thread ta([&] { a.reset(); });
+  std::this_thread::sleep_for(std::chrono::milliseconds(100));
+  std::thread tb([&] {
+    upload(b, db, src);
+    download(b, hb, db);
+    done.set();
+  });
+  bool ok = false;
+  {
+    std::unique_lock<std::mutex> l(done.mu);
+    ok = done.cv.wait_for(l, std::chrono::seconds(20), [&] { return done.done; });
+  }
+  CHECK(ok, "a context waits for another one that goes");
+  CHECK(hb == src, "copies beside a context that goes");
+  gate.set();
+  ta.join();
+  tb.join();
+  sim::free_gate = nullptr;
+}
+
 // a caller's pinned memory: one copy each way, between it and the device
 void pinned_memory() {
   Ctx a;
@@ -434,6 +469,7 @@ int main() {
   other_context();
   threads();
   no_waiting();
+  closing();
   pinned_memory();
   sim::no_pins = true;  // copies without slots are the runtime's
   round_trips();
