@@ -328,6 +328,7 @@ void no_waiting() {
     gate.set();
     ta.join();
     tb.join();
+    a.s.sync();
   }
 }
 
@@ -433,9 +434,11 @@ void set_count() {
         download(*x, dst, dev);
       }
     CHECK(sim::pin_calls == before + 1, "contexts in turn pinned %d sets", sim::pin_calls - before);
+    std::vector<char> devs[3] = {dev, dev, dev};
+    int k = 0;
     for (Ctx* x : {&a, &b, &c}) {
       x->kernel(30);
-      upload(*x, dev, src);
+      upload(*x, devs[k++], src);
     }
     for (Ctx* x : {&a, &b, &c}) x->s.sync();
     CHECK(sim::pins <= 3, "three contexts pinned %d sets", (int)sim::pins);
@@ -457,6 +460,7 @@ void failures() {
         sim::fail_copy = -1;
         CHECK(st == II_OK || a.s.idle(), "copy of %zu bytes failed at its piece %d with work left",
               n, at);
+        a.s.sync();
         download(b, dst, src);
         CHECK(dst == src, "download of %zu bytes after another context's failure", n);
       }
