@@ -520,3 +520,20 @@ def test_graph_replayed_iterations_equal_eager(precision, batched):
             assert o2[k].true_residual <= 1e-10
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4, 8), (8, 4, 6, 10), (12, 10, 14, 18), (16, 16, 16, 32)])
+def test_gauge_field_written_right_after_its_context_is_created(dims):
+    """The clear of a new context's gauge memory is ordered before its first
+    kernels: every link of a unit field set at once, and of a heat-bath sweep
+    from it, is there."""
+    n = 60 if dims[3] < 18 else 10
+    for i in range(n):
+        ctx = ii.Context(dims)
+        ctx.unit_gauge()
+        u = ctx.download_gauge().reshape(-1, 3, 3, 2)
+        ctx.heatbath(6.0, i, 1)
+        h = ctx.download_gauge()
+        ctx.close()
+        assert np.array_equal(u[..., 0], np.broadcast_to(np.eye(3), u.shape[:3])), i
+        assert not u[..., 1].any() and np.isfinite(h).all(), i
