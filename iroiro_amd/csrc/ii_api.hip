@@ -37,6 +37,8 @@ ii_status ensure_partials(ii_context* ctx, size_t n) {
     if (ctx->partials) {
       II_HIP(ctx, hipStreamSynchronize(ctx->stream));
       II_HIP(ctx, hipFree(ctx->partials));
+      ctx->partials = nullptr;
+      ctx->partials_len = 0;
     }
     size_t len = n < 65536 ? 65536 : n;
     II_HIP(ctx, hipMalloc(&ctx->partials, len * sizeof(double)));
@@ -62,7 +64,10 @@ ii_status ensure_scalars(ii_context* ctx, int n) {
   if (ctx->nscal < n) {
     II_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (ctx->scal) II_HIP(ctx, hipFree(ctx->scal));
+    ctx->scal = nullptr;
+    ctx->nscal = 0;
     if (ctx->scal_host) II_HIP(ctx, hipHostFree(ctx->scal_host));
+    ctx->scal_host = nullptr;
     int len = n < 64 ? 64 : n;
     II_HIP(ctx, hipMalloc(&ctx->scal, len * sizeof(CGScalars)));
     II_HIP(ctx, hipHostMalloc(&ctx->scal_host, len * sizeof(CGScalars)));

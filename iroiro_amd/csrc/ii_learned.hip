@@ -841,6 +841,7 @@ ii_status launch_wgrad(ii_context* ctx, Net* N, const float2* T, const float2* L
   if (need > N->partial_len) {
     if (N->partial) dfree(N->partial);
     N->partial = nullptr;
+    N->partial_len = 0;
     II_CHECK(dev_alloc(ctx, &N->partial, need));
     N->partial_len = need;
   }
@@ -917,6 +918,7 @@ ii_status stage(ii_context* ctx, Net* N, size_t n) {
   if (n > N->stage_len) {
     if (N->stage) dfree(N->stage);
     N->stage = nullptr;
+    N->stage_len = 0;
     II_CHECK(dev_alloc(ctx, &N->stage, n));
     N->stage_len = n;
   }
@@ -1480,6 +1482,7 @@ ii_status ii_net_train(ii_context* ctx, double kappa, const ii_train_params* p,
     dfree(N->pb);
     dfree(N->py);
     N->pb = N->py = nullptr;
+    N->npairs = 0;
     II_CHECK(dev_alloc(ctx, &N->pb, ce * p->npairs));
     II_CHECK(dev_alloc(ctx, &N->py, (size_t)12 * g.stride * p->npairs));
   }
