@@ -91,6 +91,9 @@ struct LoField {
   float* nrm = nullptr;
 };
 
+// strips of W time slices in blocks of bs sites, contiguous (mode 0) where the
+// lattice has no such order
+HopOrder strip_order(const Geom& g, int W, int bs);
 ii_status hop64(ii_context* ctx, const HopSpec& h, const double2* in, double2* out,
                 const double2* x, const double2* dv);
 ii_status hop32(ii_context* ctx, const HopSpec& h, const float2* in, float2* out,

@@ -2924,7 +2924,9 @@ ii_status ii_tune_load(ii_context* ctx, const char* path) {
       }
       ctx->mrhs_nrhs[P] = n;
       ctx->mrhs_rb[P] = rb;
-      ctx->mrhs_ord[P] = o;
+      // an order this lattice does not have is the contiguous one: a kernel would
+      // write its partial sums by it
+      ctx->mrhs_ord[P] = o.mode == 1 ? strip_order(g, o.W, 64) : HopOrder();
       ctx->mrhs_report[P] = "multi-rhs hop shape loaded from a tuning file";
     } else if (std::sscanf(line, "net %d %d %d %d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2],
                            &v[3], &v[4], &v[5], &v[6], &v[7], &v[8], &v[9], &v[10], &v[11],

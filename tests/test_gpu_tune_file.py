@@ -112,3 +112,17 @@ def test_multi_rhs_shapes_timed_where_blocks_are_few(tmp_path):
         for rb in (12, 6, 4, 3, 2):
             assert " %d/contig=" % rb in p
     ctx.close()
+
+
+@pytest.mark.parametrize("line", ["mrhs 0 12 6 1 0 2 256", "mrhs 0 12 6 1 3 2 256",
+                                  "mrhs 0 12 6 1 -1 2 256", "mrhs 0 12 6 7 2 2 256"])
+def test_orders_the_lattice_does_not_have_are_contiguous(tmp_path, line):
+    """An edited file's strip width that does not divide the time slices, or an
+    unknown order, never reaches a kernel."""
+    path = tmp_path / "t.tune"
+    path.write_text("iroiro-hip tuning 1\nlattice 16 16 4 16\n" + line + "\n")
+    ctx = ii.Context((16, 16, 4, 16))
+    ctx.tune_load(path)
+    ctx.tune_save(path)
+    ctx.close()
+    assert "mrhs 0 12 6 0 4 1 256" in path.read_text()
